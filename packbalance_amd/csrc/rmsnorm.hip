@@ -7,13 +7,15 @@
 // 16-byte vectors, so a row of n elements is read as n*sizeof(T)/1024
 // fully-coalesced wave loads.  When a row fits in registers (n <= 64*VEC*NV)
 // it is read from HBM exactly once; the reduction is a wave64 butterfly, so
-// no LDS or block barrier sits on the forward path.  The backward also
+// no LDS or block barrier sits on the forward path.  Wider rows belong to a
+// workgroup instead (rmsnorm_*_wide), up to 1024 lanes of 4 vectors.  The backward also
 // accumulates the per-column dw partial sums of the rows a workgroup owns and
 // writes one fp32 partial row per workgroup; a second small kernel sums the
 // partials (the reference does this with two extra eager passes over x, dy).
 #include <mutex>
 
 #include "common.hpp"
+#include "lds_dma.hpp"
 
 namespace pb {
 namespace {
@@ -125,6 +127,96 @@ __global__ __launch_bounds__(kThreads) void rmsnorm_fwd_reg(
 inline unsigned fwd_reg_grid(int64_t rows) {
   const int64_t want = (rows + kWaves - 1) / kWaves;
   return (unsigned)(want < 1024 ? want : 1024);
+}
+
+// Rows too wide for one wave's registers (bf16 n > 4096, fp32 n > 2048): one
+// workgroup of THREADS lanes holds the row, NV 16-byte vectors per lane, so it
+// is still read once; the row sum crosses the waves through LDS with one
+// barrier per row (two LDS slots, used in turn, so a wave never overwrites a
+// sum another wave is still reading).  The barrier carries no memory fence:
+// the next row's loads, issued before it, stay in flight across the reduction
+// and the stores.  HBM-bound.  Against the two-pass scalar kernel below
+// ([8192, 8192] bf16): forward 118 -> 46 us (5.9 TB/s).
+template <int THREADS>
+__device__ __forceinline__ float row_sum(float v, float (*red)[THREADS / 64], int slot) {
+  constexpr int W = THREADS / 64;
+  v = wave_sum_full(v);
+  if ((threadIdx.x & 63) == 0) red[slot][threadIdx.x >> 6] = v;
+  __builtin_amdgcn_s_waitcnt(0xC07F);  // the LDS write is done (lgkmcnt(0))
+  block_sync_nofence();
+  float s = red[slot][0];
+#pragma unroll
+  for (int k = 1; k < W; ++k) s += red[slot][k];
+  return s;
+}
+
+template <typename TX, typename TW, int NV, int THREADS>
+__global__ __launch_bounds__(THREADS) void rmsnorm_fwd_wide(
+    const TX *__restrict__ x, int64_t xs, const TW *__restrict__ w, TX *__restrict__ y, int64_t ys,
+    float *__restrict__ rstd_out, int64_t rows, int n, float eps) {
+  constexpr int VEC = 16 / sizeof(TX);
+  constexpr int WB = VEC * sizeof(TW);  // bytes of w per vector
+  typedef unsigned wraw_t __attribute__((ext_vector_type(WB / 4)));
+  __shared__ float red[2][THREADS / 64];
+  const int tid = threadIdx.x;
+  int64_t row = blockIdx.x;  // the grid has at most one workgroup per row
+  wraw_t wraw[NV];
+  u32x4 cur[NV];
+  auto load_row = [&](int64_t r, u32x4 (&dst)[NV]) {
+    const TX *xr = x + r * xs;
+#pragma unroll
+    for (int i = 0; i < NV; ++i) {
+      const int c = (i * THREADS + tid) * VEC;
+      if (c < n) dst[i] = __builtin_nontemporal_load(reinterpret_cast<const u32x4 *>(xr + c));
+    }
+  };
+  load_row(row, cur);
+#pragma unroll
+  for (int i = 0; i < NV; ++i) {
+    const int c = (i * THREADS + tid) * VEC;
+    if (c < n) wraw[i] = *reinterpret_cast<const wraw_t *>(w + c);
+  }
+  int slot = 0;
+#pragma unroll 1
+  for (; row < rows; row += gridDim.x, slot ^= 1) {
+    u32x4 nxt[NV];
+    if (row + gridDim.x < rows) load_row(row + gridDim.x, nxt);
+    float ss = 0.f;
+#pragma unroll
+    for (int i = 0; i < NV; ++i) {
+      const int c = (i * THREADS + tid) * VEC;
+      if (c < n) {
+        const TX *e = reinterpret_cast<const TX *>(&cur[i]);
+#pragma unroll
+        for (int k = 0; k < VEC; ++k) ss += to_f32(e[k]) * to_f32(e[k]);
+      }
+    }
+    ss = row_sum<THREADS>(ss, red, slot);
+    const float r = 1.0f / sqrtf(ss / (float)n + eps);
+    if (tid == 0) rstd_out[row] = r;
+    TX *yr = y + row * ys;
+#pragma unroll
+    for (int i = 0; i < NV; ++i) {
+      const int c = (i * THREADS + tid) * VEC;
+      if (c < n) {
+        const TX *e = reinterpret_cast<const TX *>(&cur[i]);
+        const TW *we = reinterpret_cast<const TW *>(&wraw[i]);
+        float o[VEC];
+#pragma unroll
+        for (int k = 0; k < VEC; ++k) o[k] = to_f32(e[k]) * r * to_f32(we[k]);
+        store16_nt<TX>(yr + c, o);
+      }
+    }
+#pragma unroll
+    for (int i = 0; i < NV; ++i) cur[i] = nxt[i];
+  }
+}
+
+// Workgroups of rmsnorm_fwd_wide: four 4-wave workgroups per CU, or two of 16
+// waves (a row each, then rows in a loop).
+inline unsigned wide_grid(int64_t rows, int threads) {
+  const int64_t cap = threads == 256 ? 1024 : 512;
+  return (unsigned)(rows < cap ? rows : cap);
 }
 
 // General row (any n, any alignment): two passes over the row, scalar loads.
@@ -274,6 +366,101 @@ __global__ __launch_bounds__(kThreads) void rmsnorm_bwd_reg(
   }
 }
 
+// Wide rows, backward: one workgroup per row as in rmsnorm_fwd_wide, a lane
+// owning the same columns of every row the workgroup walks (grid-stride), so
+// the dw partial stays in registers and leaves as one fp32 row per workgroup
+// with no cross-wave sum.  The next row's vectors are loaded as this row's dx
+// leaves (as in rmsnorm_bwd_reg).  HBM-bound.  Against the scalar kernel
+// below, which re-reads x and dy and adds dw in memory for every row
+// ([8192, 8192] bf16): 480 -> 69 us (5.9 TB/s).
+template <typename TX, typename TW, int NV, int THREADS>
+__global__ __launch_bounds__(THREADS) void rmsnorm_bwd_wide(
+    const TX *__restrict__ dy, int64_t dys, const TX *__restrict__ x, int64_t xs,
+    const TW *__restrict__ w, const float *__restrict__ rstd, TX *__restrict__ dx, int64_t dxs,
+    float *__restrict__ partial, int64_t rows, int n) {
+  constexpr int VEC = 16 / sizeof(TX);
+  constexpr int WB = VEC * sizeof(TW);
+  typedef unsigned wraw_t __attribute__((ext_vector_type(WB / 4)));
+  __shared__ float red[2][THREADS / 64];
+  const int tid = threadIdx.x;
+  const float inv_n = 1.0f / (float)n;
+  float acc[NV][VEC];
+  wraw_t wraw[NV];
+#pragma unroll
+  for (int i = 0; i < NV; ++i) {
+    const int c = (i * THREADS + tid) * VEC;
+    if (c < n) wraw[i] = *reinterpret_cast<const wraw_t *>(w + c);
+#pragma unroll
+    for (int e = 0; e < VEC; ++e) acc[i][e] = 0.f;
+  }
+  auto wv = [&](int i, int e) { return to_f32(reinterpret_cast<const TW *>(&wraw[i])[e]); };
+  u32x4 cx[NV], cd[NV];
+  auto load_vec = [&](int64_t rr, int i) {
+    const int c = (i * THREADS + tid) * VEC;
+    if (c < n) {
+      cx[i] = __builtin_nontemporal_load(reinterpret_cast<const u32x4 *>(x + rr * xs + c));
+      cd[i] = __builtin_nontemporal_load(reinterpret_cast<const u32x4 *>(dy + rr * dys + c));
+    }
+  };
+  int64_t row = blockIdx.x;  // the grid has at most one workgroup per row
+#pragma unroll
+  for (int i = 0; i < NV; ++i) load_vec(row, i);
+  float r = rstd[row];
+  int slot = 0;
+#pragma unroll 1
+  for (; row < rows; row += gridDim.x, slot ^= 1) {
+    const int64_t nrow = row + gridDim.x;
+    const bool more = nrow < rows;  // uniform over the workgroup
+    const float rn = more ? rstd[nrow] : 0.f;
+    float dot = 0.f;
+#pragma unroll
+    for (int i = 0; i < NV; ++i) {
+      const int c = (i * THREADS + tid) * VEC;
+      if (c < n) {
+        const TX *ex = reinterpret_cast<const TX *>(&cx[i]);
+        const TX *ed = reinterpret_cast<const TX *>(&cd[i]);
+#pragma unroll
+        for (int e = 0; e < VEC; ++e) {
+          const float xh = to_f32(ex[e]) * r, dv = to_f32(ed[e]);
+          dot += dv * wv(i, e) * xh;
+          acc[i][e] += dv * xh;
+        }
+      }
+    }
+    dot = row_sum<THREADS>(dot, red, slot) * inv_n;
+#pragma unroll
+    for (int i = 0; i < NV; ++i) asm volatile("" : "+v"(cx[i]), "+v"(cd[i]));
+#pragma unroll
+    for (int i = 0; i < NV; ++i) {
+      const int c = (i * THREADS + tid) * VEC;
+      if (c < n) {
+        const TX *ex = reinterpret_cast<const TX *>(&cx[i]);
+        const TX *ed = reinterpret_cast<const TX *>(&cd[i]);
+        float o[VEC];
+#pragma unroll
+        for (int e = 0; e < VEC; ++e) {
+          const float xh = to_f32(ex[e]) * r;
+          o[e] = r * (to_f32(ed[e]) * wv(i, e) - xh * dot);
+        }
+        store16_nt<TX>(dx + row * dxs + c, o);
+      }
+      if (more) load_vec(nrow, i);
+    }
+    r = rn;
+  }
+  float *out = partial + (int64_t)blockIdx.x * n;
+#pragma unroll
+  for (int i = 0; i < NV; ++i) {
+    const int c = (i * THREADS + tid) * VEC;
+    if (c < n) {
+#pragma unroll
+      for (int e = 0; e < VEC; e += 4)
+        *reinterpret_cast<f32x4 *>(out + c + e) =
+            f32x4{acc[i][e], acc[i][e + 1], acc[i][e + 2], acc[i][e + 3]};
+    }
+  }
+}
+
 template <typename TX, typename TW>
 __global__ __launch_bounds__(kThreads) void rmsnorm_bwd_loop(
     const TX *__restrict__ dy, int64_t dys, const TX *__restrict__ x, int64_t xs,
@@ -379,8 +566,32 @@ BwdPlan bwd_plan(int64_t rows) {
   return p;
 }
 
+// Workgroups of rmsnorm_bwd_wide.  A workgroup takes one row at a time, so a
+// few thousand rows would leave most of the GPU idle at bwd_plan's eight rows
+// each ([1000, 8192] bf16 would run on 125 CUs): one row per workgroup up to
+// 512, unless the fp32 partial rows of that would pass the static scratch of
+// the allocation-free entry, whose limit on n stays where bwd_plan puts it.
+int wide_nwg(int64_t rows, int64_t n) {
+  int64_t cap = PB_RMSNORM_NOALLOC_SCRATCH_BYTES / (n * (int64_t)sizeof(float));
+  if (cap > 512) cap = 512;
+  const int64_t nwg = rows < cap ? rows : cap;
+  const int64_t base = bwd_plan(rows).nwg;
+  return (int)(nwg > base ? nwg : base);
+}
+
+// Partial rows a caller's workspace must hold, whichever kernel runs: the wide
+// kernels serve no n below 2048 (fp32 rows past 8 vectors of one wave).
+int max_nwg(int64_t rows, int64_t n) {
+  return n > 2048 ? wide_nwg(rows, n) : bwd_plan(rows).nwg;
+}
+
 // Number of 16-byte vectors per lane that a register-resident row needs,
-// rounded up to the instantiated set; 0 when the row must stream.
+// rounded up to the instantiated set; 0 when the row must stream.  Up to 8
+// vectors of one wave's lanes (4096 bf16 / 2048 fp32) the row belongs to one
+// wave; beyond that kWide* name the one-workgroup-per-row kernels: 256 lanes
+// of 4 or 8 vectors (8192 / 16384 bf16), then 1024 lanes of 4 (32768 bf16),
+// past which the backward's registers would spill and the row streams.
+constexpr int kWide4 = 100, kWide8 = 101, kWide1024 = 102;
 template <typename TX>
 int pick_nv(int64_t n, const void *a, int64_t a_stride, const void *b, int64_t b_stride,
             const void *c, int64_t c_stride) {
@@ -396,6 +607,9 @@ int pick_nv(int64_t n, const void *a, int64_t a_stride, const void *b, int64_t b
   if (need <= 2) return 2;
   if (need <= 4) return 4;
   if (need <= 8) return 8;
+  if (need <= 4 * kWaves) return kWide4;
+  if (need <= 8 * kWaves) return kWide8;
+  if (need <= 4 * 16) return kWide1024;
   return 0;
 }
 
@@ -417,6 +631,13 @@ int fwd_typed(const void *x, int64_t xs, const void *w, void *y, int64_t ys, flo
     break;
     PB_FWD(1) PB_FWD(2) PB_FWD(4) PB_FWD(8)
 #undef PB_FWD
+#define PB_FWD(KEY, NV, T)                                                                        \
+  case KEY:                                                                                       \
+    hipLaunchKernelGGL((rmsnorm_fwd_wide<TX, TW, NV, T>), dim3(wide_grid(rows, T)), dim3(T), 0,   \
+                       st, X, xs, W, Y, ys, rstd, rows, (int)n, eps);                             \
+    break;
+    PB_FWD(kWide4, 4, 256) PB_FWD(kWide8, 8, 256) PB_FWD(kWide1024, 4, 1024)
+#undef PB_FWD
     default:
       hipLaunchKernelGGL((rmsnorm_fwd_loop<TX, TW>), grid, dim3(kThreads), 0, st, X, xs, W, Y, ys,
                          rstd, rows, (int)n, eps);
@@ -436,6 +657,10 @@ int bwd_typed(const void *dy, int64_t dys, const void *x, int64_t xs, const void
   int nv = pick_nv<TX>(n, x, xs, dy, dys, dx, dxs);
   if (nv && (reinterpret_cast<uintptr_t>(w) % (16 / sizeof(TX) * sizeof(TW) >= 16 ? 16 : 8)) != 0)
     nv = 0;
+  if (nv >= kWide4) {
+    if (reinterpret_cast<uintptr_t>(ws) % 16) nv = 0;  // 16-byte partial stores
+    else p.nwg = wide_nwg(rows, n);
+  }
   dim3 grid(p.nwg);
   switch (nv) {
 #define PB_BWD(NV)                                                                              \
@@ -444,6 +669,13 @@ int bwd_typed(const void *dy, int64_t dys, const void *x, int64_t xs, const void
                        xs, W, rstd, DX, dxs, ws, rows, (int)n);                                 \
     break;
     PB_BWD(1) PB_BWD(2) PB_BWD(4) PB_BWD(8)
+#undef PB_BWD
+#define PB_BWD(KEY, NV, T)                                                                      \
+  case KEY:                                                                                     \
+    hipLaunchKernelGGL((rmsnorm_bwd_wide<TX, TW, NV, T>), grid, dim3(T), 0, st, DY, dys, X, xs, \
+                       W, rstd, DX, dxs, ws, rows, (int)n);                                     \
+    break;
+    PB_BWD(kWide4, 4, 256) PB_BWD(kWide8, 8, 256) PB_BWD(kWide1024, 4, 1024)
 #undef PB_BWD
     default:
       hipLaunchKernelGGL((rmsnorm_bwd_loop<TX, TW>), grid, dim3(kThreads), 0, st, DY, dys, X, xs,
@@ -512,7 +744,7 @@ extern "C" int pb_rmsnorm_fwd(const void *x, int64_t x_row_stride, int x_dtype, 
 
 extern "C" int64_t pb_rmsnorm_bwd_workspace_bytes(int64_t rows, int64_t n) {
   if (rows <= 0 || n <= 0) return 0;
-  return (int64_t)pb::bwd_plan(rows).nwg * n * (int64_t)sizeof(float);
+  return (int64_t)pb::max_nwg(rows, n) * n * (int64_t)sizeof(float);
 }
 
 extern "C" int pb_rmsnorm_bwd(const void *dy, int64_t dy_row_stride, const void *x,

@@ -78,6 +78,35 @@ def test_rmsnorm_matches_oracle(shape, dtype, wdtype, dev) -> None:
     _close(wr.grad, dw_ref, max(tol, 1e-4), "dw")
 
 
+@pytest.mark.parametrize(
+    "rows,n,dtype,wdtype,pad",
+    [
+        (5, 4104, torch.bfloat16, torch.bfloat16, 0),  # first width past one wave's registers
+        (1, 8192, torch.bfloat16, torch.float32, 0),  # one row, every lane's vectors full
+        (1030, 8192, torch.float16, torch.float16, 8),  # rows walked in a loop, row stride > n
+        (3, 8200, torch.bfloat16, torch.bfloat16, 0),  # first 8-vector width
+        (2, 16392, torch.bfloat16, torch.bfloat16, 0),  # first 1024-lane width
+        (3, 32768, torch.bfloat16, torch.float32, 0),  # the widest register row
+        (2, 32776, torch.bfloat16, torch.bfloat16, 0),  # past it: streaming rows
+        (700, 2052, torch.float32, torch.float32, 0),
+        (515, 5120, torch.float32, torch.float32, 4),
+    ],
+)
+def test_rmsnorm_wide_rows_match_oracle(rows, n, dtype, wdtype, pad, dev) -> None:
+    """One workgroup per row; bf16 dx error is bounded as in the narrow cases, and dw (a
+    sum over at most 1030 rows of values near 1) to the output's own rounding."""
+    x, w, dy = _rms_case((rows, n + pad), dtype, torch.float32, dev, seed=n)
+    x, dy, w = x[:, :n], dy[:, :n], w[:n].to(wdtype)
+    xr, wr = x.detach().requires_grad_(True), w.clone().requires_grad_(True)
+    y = rmsnorm(xr, wr, 1e-5)
+    y.backward(dy)
+    tol = TOL[dtype]
+    dx_ref, dw_ref = OK.rmsnorm_bwd(dy, x, w, 1e-5)
+    _close(y, OK.rmsnorm_fwd(x, w, 1e-5)[0], tol, "y")
+    _close(xr.grad, dx_ref, tol, "dx")
+    _close(wr.grad, dw_ref, max(TOL[wdtype], 1e-4), "dw")
+
+
 def test_rmsnorm_strided_rows(dev) -> None:
     # Rows of a wider buffer (row stride 280, base offset 20 bytes).
     x, w, dy = _rms_case((64, 256), torch.float32, torch.float32, dev, row_view=True)
