@@ -15,7 +15,8 @@
 //
 // Layout: one wave per row, 8 elements per lane and vector (a 16-byte load for
 // 16-bit dtypes, two for fp32), rows of up to 2048 elements held in
-// registers; longer or misaligned rows take a two-pass loop kernel.  The
+// registers; rows of up to 16384 are held by a workgroup (*_wide); longer or
+// misaligned rows take a two-pass loop kernel.  The
 // backward writes per-workgroup dw partials summed by a small kernel.  The
 // forward streams with non-temporal loads and stores, the backward with
 // cached ones (at [4096, 768] rows of the model: backward 15.7 -> 14.9 us
@@ -25,12 +26,14 @@
 #include <utility>
 
 #include "common.hpp"
+#include "lds_dma.hpp"
 
 namespace pb {
 namespace {
 
 constexpr int kWaves = 4;
 constexpr int kThreads = 64 * kWaves;
+constexpr int kWideAbove = 2048;  // widest row that one wave's registers hold
 
 struct AddNormFwd {
   const char *x, *delta, *w;
@@ -114,6 +117,35 @@ __device__ __forceinline__ void st8(char *p, int dt, const float (&v)[8], bool n
   }
 }
 
+// 8 elements as loaded, widened where they are used, so that a row's loads
+// are all issued before the first is waited for (ld8 on a 16-bit dtype waits
+// for its own load).  b holds the second half of fp32 elements.
+struct Raw8 {
+  u32x4 a, b;
+};
+__device__ __forceinline__ void ldraw(Raw8 &r, const char *p, int dt, bool nt) {
+  const u32x4 *q = reinterpret_cast<const u32x4 *>(p);
+  r.a = nt ? __builtin_nontemporal_load(q) : q[0];
+  if (dt == PB_F32) r.b = nt ? __builtin_nontemporal_load(q + 1) : q[1];
+}
+__device__ __forceinline__ void widen(const Raw8 &r, int dt, float (&o)[8]) {
+  if (dt == PB_F32) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      o[i] = __uint_as_float(r.a[i]);
+      o[4 + i] = __uint_as_float(r.b[i]);
+    }
+  } else if (dt == PB_BF16) {
+    const bf16_t *e = reinterpret_cast<const bf16_t *>(&r.a);
+#pragma unroll
+    for (int i = 0; i < 8; ++i) o[i] = to_f32(e[i]);
+  } else {
+    const f16_t *e = reinterpret_cast<const f16_t *>(&r.a);
+#pragma unroll
+    for (int i = 0; i < 8; ++i) o[i] = to_f32(e[i]);
+  }
+}
+
 __device__ __forceinline__ float ld1(const char *p, int dt) {
   if (dt == PB_F32) return *reinterpret_cast<const float *>(p);
   if (dt == PB_BF16) return to_f32(*reinterpret_cast<const bf16_t *>(p));
@@ -163,6 +195,96 @@ __global__ __launch_bounds__(kThreads) void add_rmsnorm_fwd_reg(AddNormFwd a) {
 #pragma unroll
       for (int e = 0; e < 8; ++e) o[e] = h[i][e] * r * wv[i][e];
       st8(a.y + (row * a.ys + c) * yb, a.ydt, o, true);
+    }
+  }
+}
+
+// Rows past one wave's registers: a workgroup of THREADS lanes holds the row
+// (NV vectors of 8 per lane), so every operand is read once; the row sum
+// crosses the waves through LDS, one barrier per row (two slots in turn), and
+// the barrier has no memory fence, so the next row's loads stay in flight
+// across it and the stores.  HBM-bound.  STD fixes the dtypes of the model's
+// flow (fp32 residual and weight, bf16 the rest) at compile time.
+// At [8192, 4096], fp32 residual, bf16 delta and y: 68 us (5.9 TB/s); with the
+// backward 917 us on the scalar two-pass kernels below, 170 us here.
+template <int THREADS>
+__device__ __forceinline__ float row_sum(float v, float (*red)[THREADS / 64], int slot) {
+  v = wave_sum_full(v);
+  if ((threadIdx.x & 63) == 0) red[slot][threadIdx.x >> 6] = v;
+  __builtin_amdgcn_s_waitcnt(0xC07F);  // the LDS write is done (lgkmcnt(0))
+  block_sync_nofence();
+  float s = red[slot][0];
+#pragma unroll
+  for (int k = 1; k < THREADS / 64; ++k) s += red[slot][k];
+  return s;
+}
+
+template <int NV, int THREADS, bool STD>
+__global__ __launch_bounds__(THREADS) void add_rmsnorm_fwd_wide(AddNormFwd a) {
+  __shared__ float red[2][THREADS / 64];
+  const int tid = threadIdx.x;
+  const int xdt = STD ? PB_F32 : a.xdt, wdt = STD ? PB_F32 : a.wdt;
+  const int ddt = STD ? PB_BF16 : a.ddt, ydt = STD ? PB_BF16 : a.ydt;
+  const int xb = esize(xdt), db = esize(ddt), wb = esize(wdt), yb = esize(ydt);
+  const bool add = a.delta != nullptr;
+  Raw8 cx[NV], cd[NV], nx[NV], nd[NV], cw[NV];
+  auto load_row = [&](int64_t r, Raw8 (&x)[NV], Raw8 (&d)[NV]) {
+#pragma unroll
+    for (int i = 0; i < NV; ++i) {
+      const int c = (i * THREADS + tid) * 8;
+      if (c < a.n) {
+        ldraw(x[i], a.x + (r * a.xs + c) * xb, xdt, true);
+        if (add) ldraw(d[i], a.delta + (r * a.ds + c) * db, ddt, true);
+      }
+    }
+  };
+  int64_t row = blockIdx.x;  // the grid has at most one workgroup per row
+  load_row(row, cx, cd);
+#pragma unroll
+  for (int i = 0; i < NV; ++i) {
+    const int c = (i * THREADS + tid) * 8;
+    if (c < a.n) ldraw(cw[i], a.w + (int64_t)c * wb, wdt, false);
+  }
+  int slot = 0;
+#pragma unroll 1
+  for (; row < a.rows; row += gridDim.x, slot ^= 1) {
+    if (row + gridDim.x < a.rows) load_row(row + gridDim.x, nx, nd);
+    float h[NV][8];
+    float ss = 0.f;
+#pragma unroll
+    for (int i = 0; i < NV; ++i) {
+      const int c = (i * THREADS + tid) * 8;
+      if (c < a.n) {
+        widen(cx[i], xdt, h[i]);
+        if (add) {
+          float d[8];
+          widen(cd[i], ddt, d);
+#pragma unroll
+          for (int e = 0; e < 8; ++e) h[i][e] += d[e];
+        }
+#pragma unroll
+        for (int e = 0; e < 8; ++e) ss += h[i][e] * h[i][e];
+      }
+    }
+    ss = row_sum<THREADS>(ss, red, slot);
+    const float r = 1.0f / sqrtf(ss / (float)a.n + a.eps);
+    if (tid == 0) a.rstd[row] = r;
+#pragma unroll
+    for (int i = 0; i < NV; ++i) {
+      const int c = (i * THREADS + tid) * 8;
+      if (c < a.n) {
+        if (a.h) st8(a.h + (row * a.hs + c) * xb, xdt, h[i], true);
+        float o[8], wv[8];
+        widen(cw[i], wdt, wv);
+#pragma unroll
+        for (int e = 0; e < 8; ++e) o[e] = h[i][e] * r * wv[e];
+        st8(a.y + (row * a.ys + c) * yb, ydt, o, true);
+      }
+    }
+#pragma unroll
+    for (int i = 0; i < NV; ++i) {
+      cx[i] = nx[i];
+      cd[i] = nd[i];
     }
   }
 }
@@ -276,6 +398,102 @@ __global__ __launch_bounds__(kThreads) void add_rmsnorm_bwd_reg(AddNormBwd a) {
   }
 }
 
+// Rows past one wave's registers, backward: as add_rmsnorm_fwd_wide; a lane
+// owns the same columns of every row its workgroup walks (grid-stride), so
+// the dw partial stays in registers and needs no cross-wave sum, and each of
+// a row's vectors is replaced by the next row's as soon as its dx is stored.
+// HBM-bound.  [8192, 4096], fp32 residual, bf16 dy and ddelta: 98 us (5.5 TB/s).
+template <int NV, int THREADS, bool STD>
+__global__ __launch_bounds__(THREADS) void add_rmsnorm_bwd_wide(AddNormBwd a) {
+  __shared__ float red[2][THREADS / 64];
+  const int tid = threadIdx.x;
+  const int hdt = STD ? PB_F32 : a.hdt, wdt = STD ? PB_F32 : a.wdt;
+  const int ydt = STD ? PB_BF16 : a.dydt, ddt = STD ? PB_BF16 : a.dddt;
+  const int hb = esize(hdt), yb = esize(ydt), wb = esize(wdt), db = esize(ddt);
+  const float inv_n = 1.0f / (float)a.n;
+  const bool res = a.dres != nullptr;
+  Raw8 ch[NV], cy[NV], cr[NV], cw[NV];
+  float acc[NV][8];
+  auto load_vec = [&](int64_t r, int i) {
+    const int c = (i * THREADS + tid) * 8;
+    if (c < a.n) {
+      ldraw(ch[i], a.h + (r * a.hs + c) * hb, hdt, true);
+      ldraw(cy[i], a.dy + (r * a.dys + c) * yb, ydt, true);
+      if (res) ldraw(cr[i], a.dres + (r * a.drs + c) * hb, hdt, true);
+    }
+  };
+  int64_t row = blockIdx.x;  // the grid has at most one workgroup per row
+#pragma unroll
+  for (int i = 0; i < NV; ++i) {
+    load_vec(row, i);
+    const int c = (i * THREADS + tid) * 8;
+    if (c < a.n) ldraw(cw[i], a.w + (int64_t)c * wb, wdt, false);
+#pragma unroll
+    for (int e = 0; e < 8; ++e) acc[i][e] = 0.f;
+  }
+  float r = a.rstd[row];
+  int slot = 0;
+#pragma unroll 1
+  for (; row < a.rows; row += gridDim.x, slot ^= 1) {
+    const int64_t nrow = row + gridDim.x;
+    const bool more = nrow < a.rows;  // uniform over the workgroup
+    const float rn = more ? a.rstd[nrow] : 0.f;
+    float dot = 0.f;
+#pragma unroll
+    for (int i = 0; i < NV; ++i) {
+      const int c = (i * THREADS + tid) * 8;
+      if (c < a.n) {
+        float hv[8], dy[8], wv[8];
+        widen(ch[i], hdt, hv);
+        widen(cy[i], ydt, dy);
+        widen(cw[i], wdt, wv);
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+          const float hh = hv[e] * r;
+          dot += dy[e] * wv[e] * hh;
+          acc[i][e] += dy[e] * hh;
+        }
+      }
+    }
+    dot = row_sum<THREADS>(dot, red, slot) * inv_n;
+    // The second pass widens again from the raw vectors (the empty asm keeps
+    // the compiler from holding the first pass's values across the barrier).
+#pragma unroll
+    for (int i = 0; i < NV; ++i) asm volatile("" : "+v"(ch[i].a), "+v"(cy[i].a));
+#pragma unroll
+    for (int i = 0; i < NV; ++i) {
+      const int c = (i * THREADS + tid) * 8;
+      if (c < a.n) {
+        float hv[8], dy[8], wv[8], d[8];
+        widen(ch[i], hdt, hv);
+        widen(cy[i], ydt, dy);
+        widen(cw[i], wdt, wv);
+#pragma unroll
+        for (int e = 0; e < 8; ++e) d[e] = r * (dy[e] * wv[e] - hv[e] * r * dot);
+        if (res) {
+          float dr[8];
+          widen(cr[i], hdt, dr);
+#pragma unroll
+          for (int e = 0; e < 8; ++e) d[e] += dr[e];
+        }
+        st8(a.dx + (row * a.dxs + c) * hb, hdt, d, true);
+        if (a.ddelta) st8(a.ddelta + (row * a.dds + c) * db, ddt, d, true);
+      }
+      if (more) load_vec(nrow, i);
+    }
+    r = rn;
+  }
+  float *out = a.partial + (int64_t)blockIdx.x * a.n;
+#pragma unroll
+  for (int i = 0; i < NV; ++i) {
+    const int c = (i * THREADS + tid) * 8;
+    if (c < a.n) {
+      *reinterpret_cast<f32x4 *>(out + c) = f32x4{acc[i][0], acc[i][1], acc[i][2], acc[i][3]};
+      *reinterpret_cast<f32x4 *>(out + c + 4) = f32x4{acc[i][4], acc[i][5], acc[i][6], acc[i][7]};
+    }
+  }
+}
+
 // Any n / alignment: columns strided over the workgroup, rows in sequence,
 // the row dot product reduced through LDS; column c's dw partial is private
 // to its thread.
@@ -380,22 +598,38 @@ __global__ __launch_bounds__(256) void add_rmsnorm_dw_zero(char *dw, int wdt, in
   if (c < n) st1(dw + (int64_t)c * esize(wdt), wdt, 0.f);
 }
 
-int bwd_nwg(int64_t rows, int &rows_per_wg) {
+// Workgroups of the backward = rows of the dw partial table, a function of the
+// sizes alone (the batched reduction is called without knowing which kernel
+// wrote the table): at most 512 (one resident round), of at least one row per
+// wave where a wave takes a row, of at least one row where a workgroup does.
+int bwd_nwg(int64_t rows, int64_t n, int &rows_per_wg) {
   int64_t rpw = (rows + 511) / 512;
-  if (rpw < kWaves) rpw = kWaves;
+  const int64_t least = n > kWideAbove ? 1 : kWaves;
+  if (rpw < least) rpw = least;
   rows_per_wg = (int)rpw;
   const int64_t nwg = (rows + rpw - 1) / rpw;
   return (int)(nwg < 1 ? 1 : nwg);
 }
 
 // Vectors per lane for a register-resident row (0 = loop kernel): n % 8 == 0,
-// every base and row start 16-byte aligned, n <= 2048.
+// every base and row start 16-byte aligned, n <= 2048 for one wave's
+// registers, then kWide*: 256 lanes of 2 or 4 vectors (n <= 4096, 8192), 512
+// of 4 (n <= 16384; more would spill the backward).
+constexpr int kWide2 = 100, kWide4 = 101, kWide512 = 102;
 int pick_nv(int64_t n, std::initializer_list<std::pair<const void *, int64_t>> rows_bytes) {
   if (n % 8) return 0;
   for (const auto &pb : rows_bytes)
     if (pb.first && ((reinterpret_cast<uintptr_t>(pb.first) & 15) || (pb.second & 15))) return 0;
   const int64_t need = (n + 511) / 512;
-  return need <= 1 ? 1 : need <= 2 ? 2 : need <= 4 ? 4 : 0;
+  return need <= 1 ? 1 : need <= 2 ? 2 : need <= 4 ? 4 : need <= 8 ? kWide2
+         : need <= 16 ? kWide4 : need <= 32 ? kWide512 : 0;
+}
+
+// Workgroups of add_rmsnorm_fwd_wide: a row each, then rows in a loop beyond
+// four 4-wave (two 8-wave) workgroups per CU.
+unsigned fwd_wide_grid(int64_t rows, int threads) {
+  const int64_t cap = threads == 256 ? 1024 : 512;
+  return (unsigned)(rows < cap ? rows : cap);
 }
 
 }  // namespace
@@ -439,10 +673,23 @@ extern "C" int pb_add_rmsnorm_fwd(const void *x, int64_t x_row_stride, int x_dty
                              {y, y_row_stride * yb}});
   dim3 grid((unsigned)((rows + kWaves - 1) / kWaves));
   hipStream_t st = as_stream(stream);
+  const bool std_types = a.xdt == PB_F32 && a.wdt == PB_F32 && a.ydt == PB_BF16 &&
+                         (!delta || a.ddt == PB_BF16);
   switch (nv) {
     case 1: hipLaunchKernelGGL((add_rmsnorm_fwd_reg<1>), grid, dim3(kThreads), 0, st, a); break;
     case 2: hipLaunchKernelGGL((add_rmsnorm_fwd_reg<2>), grid, dim3(kThreads), 0, st, a); break;
     case 4: hipLaunchKernelGGL((add_rmsnorm_fwd_reg<4>), grid, dim3(kThreads), 0, st, a); break;
+#define PB_WIDE(KEY, NV, T)                                                                      \
+  case KEY:                                                                                      \
+    if (std_types)                                                                               \
+      hipLaunchKernelGGL((add_rmsnorm_fwd_wide<NV, T, true>), dim3(fwd_wide_grid(rows, T)),      \
+                         dim3(T), 0, st, a);                                                     \
+    else                                                                                         \
+      hipLaunchKernelGGL((add_rmsnorm_fwd_wide<NV, T, false>), dim3(fwd_wide_grid(rows, T)),     \
+                         dim3(T), 0, st, a);                                                     \
+    break;
+    PB_WIDE(kWide2, 2, 256) PB_WIDE(kWide4, 4, 256) PB_WIDE(kWide512, 4, 512)
+#undef PB_WIDE
     default: hipLaunchKernelGGL(add_rmsnorm_fwd_loop, grid, dim3(kThreads), 0, st, a);
   }
   return launch_status("pb_add_rmsnorm_fwd");
@@ -451,7 +698,7 @@ extern "C" int pb_add_rmsnorm_fwd(const void *x, int64_t x_row_stride, int x_dty
 extern "C" int64_t pb_add_rmsnorm_bwd_workspace_bytes(int64_t rows, int64_t n) {
   if (rows <= 0 || n <= 0) return 0;
   int rpw;
-  return (int64_t)pb::bwd_nwg(rows, rpw) * n * (int64_t)sizeof(float);
+  return (int64_t)pb::bwd_nwg(rows, n, rpw) * n * (int64_t)sizeof(float);
 }
 
 namespace pb {
@@ -479,19 +726,31 @@ int add_rmsnorm_bwd_rows(const void *dy, int64_t dy_row_stride, int dy_dtype, co
   a.dydt = dy_dtype; a.hdt = h_dtype; a.wdt = w_dtype; a.dddt = ddelta ? ddelta_dtype : h_dtype;
   a.rows = rows;
   a.n = (int)n;
-  const int nwg = bwd_nwg(rows, a.rows_per_wg);
+  const int nwg = bwd_nwg(rows, n, a.rows_per_wg);
   const int hb = dtype_bytes(h_dtype);
-  const int nv = pick_nv(n, {{dy, dy_row_stride * dtype_bytes(dy_dtype)},
+  int nv = pick_nv(n, {{dy, dy_row_stride * dtype_bytes(dy_dtype)},
                              {h, h_row_stride * hb},
                              {w, 0},
                              {dres, dres_row_stride * hb},
                              {dx, dx_row_stride * hb},
                              {ddelta, ddelta_row_stride * dtype_bytes(a.dddt)}});
+  if (nv >= kWide2 && reinterpret_cast<uintptr_t>(workspace) % 16) nv = 0;  // 16-byte partial stores
+  const bool std_types = a.hdt == PB_F32 && a.wdt == PB_F32 && a.dydt == PB_BF16 &&
+                         (!ddelta || a.dddt == PB_BF16);
   dim3 grid((unsigned)nwg);
   switch (nv) {
     case 1: hipLaunchKernelGGL((add_rmsnorm_bwd_reg<1>), grid, dim3(kThreads), 0, st, a); break;
     case 2: hipLaunchKernelGGL((add_rmsnorm_bwd_reg<2>), grid, dim3(kThreads), 0, st, a); break;
     case 4: hipLaunchKernelGGL((add_rmsnorm_bwd_reg<4>), grid, dim3(kThreads), 0, st, a); break;
+#define PB_WIDE(KEY, NV, T)                                                                      \
+  case KEY:                                                                                      \
+    if (std_types)                                                                               \
+      hipLaunchKernelGGL((add_rmsnorm_bwd_wide<NV, T, true>), grid, dim3(T), 0, st, a);          \
+    else                                                                                         \
+      hipLaunchKernelGGL((add_rmsnorm_bwd_wide<NV, T, false>), grid, dim3(T), 0, st, a);         \
+    break;
+    PB_WIDE(kWide2, 2, 256) PB_WIDE(kWide4, 4, 256) PB_WIDE(kWide512, 4, 512)
+#undef PB_WIDE
     default: hipLaunchKernelGGL(add_rmsnorm_bwd_loop, grid, dim3(kThreads), 0, st, a);
   }
   const int s = launch_status(what);
@@ -584,7 +843,7 @@ extern "C" int pb_rmsnorm_dw_reduce_batched(const float *partials, int64_t probl
                (long long)count, (long long)rows, (long long)n);
   if (count == 0 || rows == 0) return PB_OK;
   int rpw;
-  const int nparts = bwd_nwg(rows, rpw);
+  const int nparts = bwd_nwg(rows, n, rpw);
   PB_CHECK_ARG(partials && dw && problem_stride >= (int64_t)nparts * n,
                "pb_rmsnorm_dw_reduce_batched: null argument or problem stride < partial table");
   hipStream_t st = as_stream(stream);

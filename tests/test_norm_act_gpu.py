@@ -314,6 +314,16 @@ def test_swiglu_rejects_cpu() -> None:
         (64, 512, torch.bfloat16, torch.bfloat16, torch.bfloat16, torch.bfloat16),
         (40, 4096, torch.float32, torch.float32, torch.bfloat16, torch.float32),  # loop kernel
         (37, 100, torch.float32, torch.float16, torch.float32, torch.float32),  # n % 8 != 0
+        # a workgroup per row: the first and last widths of each shape, rows in a loop
+        (5, 2056, torch.float32, torch.bfloat16, torch.bfloat16, torch.float32),
+        (1100, 4096, torch.float32, torch.bfloat16, torch.bfloat16, torch.float32),
+        # (dw is stored in the weight's dtype, so a bf16 weight needs the bf16 dw bound
+        # the check takes from y's dtype: its rounding alone is up to 2^-9 of the value)
+        (3, 4104, torch.float16, torch.bfloat16, torch.bfloat16, torch.bfloat16),
+        (600, 5120, torch.bfloat16, torch.bfloat16, torch.bfloat16, torch.bfloat16),
+        (2, 8200, torch.float32, torch.bfloat16, torch.bfloat16, torch.float32),
+        (1, 16384, torch.float32, torch.float32, torch.float32, torch.float32),
+        (2, 16392, torch.float32, torch.bfloat16, torch.bfloat16, torch.float32),  # loop kernel
     ],
 )
 def test_add_rmsnorm_matches_oracle(rows, n, xdt, ddt, ydt, wdt, dev) -> None:
