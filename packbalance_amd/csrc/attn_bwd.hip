@@ -263,8 +263,8 @@ struct DkdvStep {
   int h, q0, e;
 };
 
-// Pipelined dK/dV (16-byte aligned views and documents, D == DP in {64, 128},
-// sequence a multiple of 64).  Wave w owns 32 KV rows with K and V fragments
+// Pipelined dK/dV (16-byte aligned views; without GEN also aligned documents
+// and lse, D == DP in {64, 128} and a sequence that is a multiple of 64).  Wave w owns 32 KV rows with K and V fragments
 // in registers and dK/dV accumulators.  The workgroup walks steps t = (query
 // sub-tile of 32 rows, query head of the group), sub-tile outer: per step
 // S = Q K^T and dP = dO V^T (lane <-> KV row), P = exp2(S*scale*log2e -
@@ -282,7 +282,12 @@ constexpr int kAheadDkdv = DP == 64 ? 2 : DP / 16;
 
 // Head dim 64 fits two waves per SIMD (with the row fragments streamed);
 // head dim 128 needs ~400 registers and runs one.
-template <int DP, int WAVES, bool SPLIT>
+// GEN: any sequence length and any head dim that is a multiple of 8 (see
+// attn_fwd_pipe).  Query rows past the end arrive as zero Q, dO, lse and delta,
+// so their P is at most 1, their dS 0, and both products add nothing.  Against
+// the register-staged kernels ([4, 1999], 12 / 4 heads, D 64): dK/dV 390 ->
+// 153 us, dQ 130 -> 47 us and a 7 us sum.
+template <int DP, int WAVES, bool SPLIT, bool GEN>
 __global__ __launch_bounds__(64 * WAVES) __attribute__((amdgpu_waves_per_eu(DP == 64 ? 2 : 1, DP == 64 ? 2 : 1)))
 void attn_bwd_dkdv_pipe(BwdArgs a) {
   constexpr int NT = 64 * WAVES, BN = 32 * WAVES;
@@ -349,6 +354,10 @@ void attn_bwd_dkdv_pipe(BwdArgs a) {
     const bf16_t *krow = a.k.row(b, hk, kvr), *vrow = a.v.row(b, hk, kvr);
 #pragma unroll
     for (int dk = 0; dk < NDK; ++dk) {
+      if (GEN && 16 * dk + 8 * hh >= a.D) {
+        kf[dk] = vf[dk] = bf16x8_t{};
+        continue;
+      }
       kf[dk] = *reinterpret_cast<const bf16x8_t *>(krow + 16 * dk + 8 * hh);
       vf[dk] = *reinterpret_cast<const bf16x8_t *>(vrow + 16 * dk + 8 * hh);
     }
@@ -361,8 +370,14 @@ void attn_bwd_dkdv_pipe(BwdArgs a) {
   }
 
   uint32_t qoff[NDMA], goff[NDMA];
-  Dma::offsets(a.q.ss, wave, lane, qoff);
-  Dma::offsets(a.dout.ss, wave, lane, goff);
+  int drow = 0;  // GEN: this thread's row of a tile's first DMA instruction
+  if constexpr (GEN) {
+    drow = Dma::offsets_gen(a.q.ss, wave, lane, a.D, qoff);
+    Dma::offsets_gen(a.dout.ss, wave, lane, a.D, goff);
+  } else {
+    Dma::offsets(a.q.ss, wave, lane, qoff);
+    Dma::offsets(a.dout.ss, wave, lane, goff);
+  }
   // Per-lane fragment offsets within a sub-tile (see attn_fwd_pipe).
   int roffs[NDK], coffs[NDB][2];
   {
@@ -435,7 +450,24 @@ void attn_bwd_dkdv_pipe(BwdArgs a) {
   const auto grs = buf_rsrc(a.dout.row(b, h0, 0), 0x7fffffff);
   const uint32_t qsh2 = (uint32_t)(a.q.sh * 2), qss2 = (uint32_t)(a.q.ss * 2);
   const uint32_t gsh2 = (uint32_t)(a.dout.sh * 2), gss2 = (uint32_t)(a.dout.ss * 2);
-  auto dma_step = [&](const DkdvStep &s, auto Rc) {
+  // GEN: lse and delta rows are 4-byte aligned only, so they move 4 bytes per
+  // lane, as the documents do (dma_docs_gen).
+  const auto lrs = buf_rsrc(a.lse + ((int64_t)b * a.Hq + h0) * S, 0x7fffffff);
+  const auto trs = buf_rsrc(a.delta + ((int64_t)b * a.Hq + h0) * S, 0x7fffffff);
+  const auto drs = buf_rsrc(docb, 0x7fffffff);
+  auto dma_step_gen = [&](const DkdvStep &s, auto Rc) {
+    const uint32_t dh = (uint32_t)(s.h - h0), q0 = (uint32_t)s.q0;
+    const int left = S - s.q0;
+    const uint32_t ro = (dh * (uint32_t)S + q0) * 4u;
+    const uint32_t rv = l32 < left ? 4u * l32 : kDmaZero;
+    // (lane i writes LDS floats i: lanes 32-63 fill delta's half)
+    if (wave == 0 && lane < 32) dma4_rs(lrs, ro, rv, lslot(Rc));
+    if (wave == 0 && lane >= 32) dma4_rs(trs, ro, rv, lslot(Rc));
+    if (wave == (WAVES > 1 ? 1 : 0)) dma_docs_gen(drs, s.q0, S, lane, dslot(Rc));
+    Dma::copy_gen(qrs, dh * qsh2 + q0 * qss2, qoff, drow, left, qslot(Rc), wave);
+    Dma::copy_gen(grs, dh * gsh2 + q0 * gss2, goff, drow, left, gslot(Rc), wave);
+  };
+  auto dma_step_in = [&](const DkdvStep &s, auto Rc) {
     const int64_t ro = ((int64_t)b * a.Hq + s.h) * S + s.q0;
     // lse to LDS floats [0, 32) (lanes 0-7), delta to [32, 64) (lanes 8-15):
     // two DMAs, since a buffer resource is wave-uniform.
@@ -446,6 +478,10 @@ void attn_bwd_dkdv_pipe(BwdArgs a) {
     const uint32_t dh = (uint32_t)(s.h - h0), q0 = (uint32_t)s.q0;
     Dma::copy_rs(qrs, dh * qsh2 + q0 * qss2, qoff, qslot(Rc), wave);
     Dma::copy_rs(grs, dh * gsh2 + q0 * gss2, goff, gslot(Rc), wave);
+  };
+  auto dma_step = [&](const DkdvStep &s, auto Rc) {
+    if constexpr (GEN) dma_step_gen(s, Rc);
+    else dma_step_in(s, Rc);
   };
 
   // Element mask of a PARTIAL step: same document, kv <= q (q < S always).
@@ -619,6 +655,7 @@ void attn_bwd_dkdv_pipe(BwdArgs a) {
 #pragma unroll
   for (int db = 0; db < NDB; ++db) {
     const int d = 32 * db + l32;
+    if (GEN && d >= a.D) continue;
 #pragma unroll
     for (int j = 0; j < 16; ++j) {
       const int kvw = kt * BN + wave * 32 + 8 * (j >> 2) + 4 * hh + (j & 3);
@@ -661,12 +698,13 @@ void attn_bwd_dkdv_pipe(BwdArgs a) {
 // on one XCD (consecutive KV tiles of one pack and KV head) then read the same
 // Q / dO tiles at about the same time, from that XCD's L2 (cfg3 backward
 // 4.94 -> 4.82 ms against walking up from each KV tile's diagonal).
-// Every step's 32 query rows lie inside the sequence: no buffer bound.  At
-// most kPairsMaxSteps steps per KV tile (G * S / 32); longer problems take the
+// At most kPairsMaxSteps steps per KV tile (G * S / 32); longer problems take the
 // 2-wave kernel above.
 constexpr int kPairsMaxSteps = 1024;
 
-template <int DP, bool DS>
+// GEN: any sequence length and any head dim 72 .. 128 that is a multiple of 8
+// (zero rows and columns as in attn_bwd_dkdv_pipe).
+template <int DP, bool DS, bool GEN>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2)))
 void attn_bwd_dkdv_pairs(BwdArgs a) {
   constexpr int NT = 256, NB = 2, BN = 32 * NB;
@@ -727,8 +765,10 @@ void attn_bwd_dkdv_pairs(BwdArgs a) {
   {
     const bf16_t *row = pwave ? a.k.row(b, hk, kvr) : a.v.row(b, hk, kvr);
 #pragma unroll
-    for (int dk = 0; dk < NDK; ++dk)
-      kvf[dk] = *reinterpret_cast<const bf16x8_t *>(row + 16 * dk + 8 * hh);
+    for (int dk = 0; dk < NDK; ++dk) {
+      if (GEN && 16 * dk + 8 * hh >= a.D) kvf[dk] = bf16x8_t{};
+      else kvf[dk] = *reinterpret_cast<const bf16x8_t *>(row + 16 * dk + 8 * hh);
+    }
   }
   f32x16_t acc[NDB];  // dV (P-wave) or dK (dP-wave)
 #pragma unroll
@@ -739,13 +779,17 @@ void attn_bwd_dkdv_pairs(BwdArgs a) {
   // chunk i * 128 + tid, rows 8 i + tid / 16, and the swizzle repeats every
   // 16 rows, so chunks i and i + 2 share a lane offset): the dP-waves, whose
   // dS stores share the in-order vmcnt, then never wait on a DMA.
+  // GEN: rows past the sequence end and columns past the head dim are zeros
+  // (kDmaZero); instruction i's row is drow + i * (rows per instruction).
   uint32_t qoff[NCH], goff[NCH];
+  const int drow = (DS ? tid & 127 : tid) / (DP / 8);
 #pragma unroll
   for (int i = 0; i < NCH; ++i) {
     int r, c;
     SwzTile<DP>::at(DS ? i * 128 + (tid & 127) : i * NT + tid, r, c);
-    qoff[i] = (uint32_t)((r * a.q.ss + c * 8) * 2);
-    goff[i] = (uint32_t)((r * a.dout.ss + c * 8) * 2);
+    const bool in = !GEN || c * 8 < a.D;
+    qoff[i] = in ? (uint32_t)((r * a.q.ss + c * 8) * 2) : kDmaZero;
+    goff[i] = in ? (uint32_t)((r * a.dout.ss + c * 8) * 2) : kDmaZero;
   }
   int roffs[NDK], coffs[NDB][2];
   {
@@ -801,10 +845,22 @@ void attn_bwd_dkdv_pairs(BwdArgs a) {
   auto dma_step = [&](int si, auto Rc) {
     const uint32_t q0 = si & 0xfffff, g = (si >> 20) & 0xff;
     const uint32_t ro = (g * (uint32_t)S + q0) * 4u;
-    if (wave == 0 && lane < 8) dma16_rs(lrs, ro, 16 * lane, lslot(Rc));
-    if (wave == 0 && lane >= 8 && lane < 16) dma16_rs(trs, ro, 16 * (lane - 8), lslot(Rc));
-    if (wave == 1 && lane < 16) dma16_rs(drs, q0 * 8u, 16 * lane, dslot(Rc));
+    const int left = S - (int)q0;
+    if constexpr (GEN) {  // 4 bytes per lane (see attn_bwd_dkdv_pipe)
+      const uint32_t rv = l32 < left ? 4u * l32 : kDmaZero;
+      if (wave == 0 && lane < 32) dma4_rs(lrs, ro, rv, lslot(Rc));
+      if (wave == 0 && lane >= 32) dma4_rs(trs, ro, rv, lslot(Rc));
+      if (wave == 1) dma_docs_gen(drs, (int)q0, S, lane, dslot(Rc));
+    } else {
+      if (wave == 0 && lane < 8) dma16_rs(lrs, ro, 16 * lane, lslot(Rc));
+      if (wave == 0 && lane >= 8 && lane < 16) dma16_rs(trs, ro, 16 * (lane - 8), lslot(Rc));
+      if (wave == 1 && lane < 16) dma16_rs(drs, q0 * 8u, 16 * lane, dslot(Rc));
+    }
     const uint32_t qo = g * qsh2 + q0 * qss2, go = g * gsh2 + q0 * gss2;
+    // Rows of one instruction: 128 or 256 lanes of 16 bytes.
+    auto in_row = [&](int i, uint32_t off) {
+      return !GEN || drow < left - i * ((DS ? 128 : NT) / (DP / 8)) ? off : kDmaZero;
+    };
     if constexpr (DS) {
       if (pwave) {
         // The LDS destinations are formed here, not hoisted out of the loop
@@ -813,16 +869,18 @@ void attn_bwd_dkdv_pairs(BwdArgs a) {
         asm volatile("" : "+s"(wb));
 #pragma unroll
         for (int i = 0; i < 2 * NCH; ++i)
-          dma16_rs(qrs, qo + (i >> 1) * 16 * qss2, qoff[i & 1], qslot(Rc) + i * 2048 + wb);
+          dma16_rs(qrs, qo + (i >> 1) * 16 * qss2, in_row(i, qoff[i & 1]), qslot(Rc) + i * 2048 + wb);
 #pragma unroll
         for (int i = 0; i < 2 * NCH; ++i)
-          dma16_rs(grs, go + (i >> 1) * 16 * gss2, goff[i & 1], gslot(Rc) + i * 2048 + wb);
+          dma16_rs(grs, go + (i >> 1) * 16 * gss2, in_row(i, goff[i & 1]), gslot(Rc) + i * 2048 + wb);
       }
     } else {
 #pragma unroll
-      for (int i = 0; i < NCH; ++i) dma16_rs(qrs, qo, qoff[i], qslot(Rc) + (i * 4 + wave) * 1024);
+      for (int i = 0; i < NCH; ++i)
+        dma16_rs(qrs, qo, in_row(i, qoff[i]), qslot(Rc) + (i * 4 + wave) * 1024);
 #pragma unroll
-      for (int i = 0; i < NCH; ++i) dma16_rs(grs, go, goff[i], gslot(Rc) + (i * 4 + wave) * 1024);
+      for (int i = 0; i < NCH; ++i)
+        dma16_rs(grs, go, in_row(i, goff[i]), gslot(Rc) + (i * 4 + wave) * 1024);
     }
   };
   const int kvmax = kt * BN + blk * 32 + 31;
@@ -936,6 +994,7 @@ void attn_bwd_dkdv_pairs(BwdArgs a) {
 #pragma unroll
     for (int db = 0; db < NDB; ++db) {
       const int d = 32 * db + l32;
+      if (GEN && d >= a.D) continue;
 #pragma unroll
       for (int j = 0; j < 16; ++j) {
         const int kvw = kt * BN + blk * 32 + 8 * (j >> 2) + 4 * hh + (j & 3);
@@ -1035,6 +1094,7 @@ void attn_bwd_dkdv_pairs(BwdArgs a) {
 #pragma unroll
     for (int db = 0; db < NDB; ++db) {
       const int d = 32 * db + l32;
+      if (GEN && d >= a.D) continue;
 #pragma unroll
       for (int j = 0; j < 16; ++j) {
         const int kvw = kt * BN + blk * 32 + 8 * (j >> 2) + 4 * hh + (j & 3);
@@ -1255,7 +1315,9 @@ constexpr int kAheadDq = 1;  // K / V fragment reads in flight ahead of their MF
 
 // Two waves per SIMD where the registers allow it (D = 64, and D = 128 with
 // 4-wave workgroups); the 2-wave D = 128 variant needs more and runs one.
-template <int DP, int WAVES>
+// GEN: any sequence length and any head dim that is a multiple of 8 (see
+// attn_fwd_pipe).
+template <int DP, int WAVES, bool GEN>
 __global__ __launch_bounds__(64 * WAVES)
 __attribute__((amdgpu_waves_per_eu(DP == 64 || WAVES == 4 ? 2 : 1, DP == 64 || WAVES == 4 ? 2 : 1)))
 void attn_bwd_dq_pipe(BwdArgs a) {
@@ -1333,6 +1395,10 @@ void attn_bwd_dq_pipe(BwdArgs a) {
     const bf16_t *orow = a.o.row(b, h, qr);
 #pragma unroll
     for (int dk = 0; dk < NDK; ++dk) {
+      if (GEN && 16 * dk + 8 * hh >= a.D) {
+        qf[dk] = gf[dk] = bf16x8_t{};
+        continue;
+      }
       qf[dk] = *reinterpret_cast<const bf16x8_t *>(qrow + 16 * dk + 8 * hh);
       gf[dk] = *reinterpret_cast<const bf16x8_t *>(grow + 16 * dk + 8 * hh);
       const bf16x8_t of = *reinterpret_cast<const bf16x8_t *>(orow + 16 * dk + 8 * hh);
@@ -1347,8 +1413,14 @@ void attn_bwd_dq_pipe(BwdArgs a) {
   for (int i = 0; i < NDB; ++i) dq_acc[i] = zero16();
 
   uint32_t koff[NDMA], voff[NDMA];
-  Dma::offsets(a.k.ss, wave, lane, koff);
-  Dma::offsets(a.v.ss, wave, lane, voff);
+  int drow = 0;  // GEN: this thread's row of a tile's first DMA instruction
+  if constexpr (GEN) {
+    drow = Dma::offsets_gen(a.k.ss, wave, lane, a.D, koff);
+    Dma::offsets_gen(a.v.ss, wave, lane, a.D, voff);
+  } else {
+    Dma::offsets(a.k.ss, wave, lane, koff);
+    Dma::offsets(a.v.ss, wave, lane, voff);
+  }
   int roffs[NDK], coffs[NDB][2];
   {
     const int j = lane & 15, g = lane >> 4;
@@ -1386,9 +1458,15 @@ void attn_bwd_dq_pipe(BwdArgs a) {
   // (The row is passed in, not computed here: calling another lambda inside
   // this generic lambda's DMA address makes clang drop the kernel's stub.)
   auto dma_sub = [&](int kv0, auto Rc) {
-    if (wave == 0 && lane < 16) dma16_rs(drs, (uint32_t)kv0 * 8u, 16 * lane, dslot(Rc));
-    Dma::copy_rs(krs, (uint32_t)kv0 * kss2, koff, kslot(Rc), wave);
-    Dma::copy_rs(vrs, (uint32_t)kv0 * vss2, voff, vslot(Rc), wave);
+    if constexpr (GEN) {
+      if (wave == 0) dma_docs_gen(drs, kv0, S, lane, dslot(Rc));
+      Dma::copy_gen(krs, (uint32_t)kv0 * kss2, koff, drow, S - kv0, kslot(Rc), wave);
+      Dma::copy_gen(vrs, (uint32_t)kv0 * vss2, voff, drow, S - kv0, vslot(Rc), wave);
+    } else {
+      if (wave == 0 && lane < 16) dma16_rs(drs, (uint32_t)kv0 * 8u, 16 * lane, dslot(Rc));
+      Dma::copy_rs(krs, (uint32_t)kv0 * kss2, koff, kslot(Rc), wave);
+      Dma::copy_rs(vrs, (uint32_t)kv0 * vss2, voff, vslot(Rc), wave);
+    }
   };
   // Element mask of a PARTIAL sub-tile: same document and kv <= q.
   // Tests and shortcuts as in attn_fwd_pipe (query rows past the sequence end
@@ -1533,11 +1611,12 @@ void attn_bwd_dq_pipe(BwdArgs a) {
   if (part) {
     // This chunk's unscaled dQ rows, fp32 (summed and scaled by attn_bwd_dq_reduce).
     const int64_t prow = (((int64_t)split * a.B + b) * a.Hq + h) * S + qi;
-    float *pq = a.dq_part + prow * DP;
+    float *pq = a.dq_part + prow * (GEN ? a.D : DP);
 #pragma unroll
     for (int db = 0; db < NDB; ++db)
 #pragma unroll
       for (int jq = 0; jq < 4; ++jq) {
+        if (GEN && 32 * db + 8 * jq >= a.D) continue;
         typedef float f32x4_t __attribute__((ext_vector_type(4)));
         f32x4_t o4;
 #pragma unroll
@@ -1551,6 +1630,7 @@ void attn_bwd_dq_pipe(BwdArgs a) {
   for (int db = 0; db < NDB; ++db)
 #pragma unroll
     for (int jq = 0; jq < 4; ++jq) {
+      if (GEN && 32 * db + 8 * jq >= a.D) continue;
       typedef __bf16 bf16x4_t __attribute__((ext_vector_type(4)));
       bf16x4_t o4;
 #pragma unroll
@@ -1559,13 +1639,15 @@ void attn_bwd_dq_pipe(BwdArgs a) {
     }
 }
 
-// dQ of split query tiles = scale * sum of the chunk partials (bf16): DP/4
+// dQ of split query tiles = scale * sum of the chunk partials (bf16): D/4
 // threads per (pack, head, query row), four elements each; rows of unsplit
-// tiles were written by attn_bwd_dq_pipe and are skipped.
+// tiles were written by attn_bwd_dq_pipe and are skipped.  DP = 0 takes the
+// head dim (a multiple of 8) from the arguments.
 template <int DP>
 __device__ __forceinline__ void dq_reduce_body(const BwdArgs &a, int bm, int block) {
-  constexpr int TPR = DP / 4, RPB = 256 / TPR;
+  const int D = DP ? DP : a.D, TPR = D / 4, RPB = 256 / TPR;
   typedef float f32x4_t __attribute__((ext_vector_type(4)));
+  if ((int)threadIdx.x >= RPB * TPR) return;
   const int64_t row = (int64_t)block * RPB + threadIdx.x / TPR;
   const int d0 = (threadIdx.x % TPR) * 4;
   const int64_t rows = (int64_t)a.B * a.Hq * a.S;
@@ -1576,10 +1658,10 @@ __device__ __forceinline__ void dq_reduce_body(const BwdArgs &a, int bm, int blo
   const int cnt = a.qcnt[b * a.nqt_dq + q / bm];
   const int nch = (cnt + a.dq_chunk - 1) / a.dq_chunk;
   if (nch <= 1) return;
-  const float *pq = a.dq_part + row * DP + d0;
+  const float *pq = a.dq_part + row * D + d0;
   f32x4_t acc = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll 4
-  for (int c = 0; c < nch; ++c) acc += *reinterpret_cast<const f32x4_t *>(pq + c * rows * DP);
+  for (int c = 0; c < nch; ++c) acc += *reinterpret_cast<const f32x4_t *>(pq + c * rows * D);
   typedef __bf16 bf16x4_t __attribute__((ext_vector_type(4)));
   bf16x4_t o4;
 #pragma unroll
@@ -1619,7 +1701,8 @@ __global__ __launch_bounds__(64 * WAVES) void attn_bwd_dq_wide(BwdArgs a) {
 // non-temporal (dO and O are streamed once; at cfg3 185 -> 179 us with four
 // rows instead of eight, 221 -> 185 us non-temporal instead of cached).
 constexpr int kDeltaRowsPerGroup = 4;
-template <int DP>
+// Lanes past the head dim (GEN) add zeros.
+template <int DP, bool GEN>
 __global__ __launch_bounds__(256) void attn_bwd_delta(BwdArgs a) {
   constexpr int TPR = DP / 8, RPP = 256 / TPR, NP = kDeltaRowsPerGroup;
   const int64_t rows = (int64_t)a.B * a.Hq * a.S;
@@ -1629,7 +1712,8 @@ __global__ __launch_bounds__(256) void attn_bwd_delta(BwdArgs a) {
 #pragma unroll
   for (int p = 0; p < NP; ++p) {
     r[p] = ((int64_t)blockIdx.x * NP + p) * RPP + threadIdx.x / TPR;
-    if (r[p] < rows) {
+    gv[p] = ov[p] = u32x4{0u, 0u, 0u, 0u};
+    if (r[p] < rows && (!GEN || 8 * sub < a.D)) {
       const int s = (int)(r[p] % a.S);
       const int64_t bh = r[p] / a.S;
       const int h = (int)(bh % a.Hq), b = (int)(bh / a.Hq);
@@ -1666,7 +1750,8 @@ __global__ __launch_bounds__(256) void attn_bwd_delta(BwdArgs a) {
 // (2 bytes per pair and head) from HBM.
 constexpr int kDsMaxTiles = kPairsMaxSteps / 8;  // 64-row KV tiles per list (G >= 4)
 
-template <int DP>
+// GEN: any sequence length and any head dim 72 .. 128 that is a multiple of 8.
+template <int DP, bool GEN>
 __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4, 4)))
 void attn_bwd_dq_ds(BwdArgs a) {
   static_assert(DP == 128, "head dim 128");
@@ -1727,7 +1812,9 @@ void attn_bwd_dq_ds(BwdArgs a) {
   const uint32_t tri = (uint32_t)(qt * (qt + 1) / 2);
   const uint32_t blkb = (uint32_t)(G * 8192), halfb = (uint32_t)(G * 4096), quadb = (uint32_t)(g0 * 4096);
   uint32_t koff[1];
-  Dma::offsets(a.k.ss, wave, lane, koff);
+  int drow = 0;  // GEN: this thread's row of a K half
+  if constexpr (GEN) drow = Dma::offsets_gen(a.k.ss, wave, lane, a.D, koff);
+  else Dma::offsets(a.k.ss, wave, lane, koff);
   const uint32_t soff0 = (uint32_t)((wave * 64 + lane) * 16), soff1 = soff0 + 8 * 1024;
   // ds_read_b64_tr_b16 addresses (see lds_col_frag): K^T of head-dim block
   // db (swizzled K half), dS^T of this wave's sub-block (64-byte pitch).
@@ -1758,7 +1845,9 @@ void attn_bwd_dq_ds(BwdArgs a) {
     const int uu = u < U ? u : U - 1;
     const int e = __builtin_amdgcn_readfirstlane(ents[uu >> 1]);
     const uint32_t kt = (uint32_t)plan_tile(e), half = (uint32_t)(uu & 1);
-    Dma::copy_rs(krs, (kt * 64 + half * 32) * kss2, koff, kslot(Rc), wave);
+    const uint32_t kv0 = kt * 64 + half * 32;
+    if constexpr (GEN) Dma::copy_gen(krs, kv0 * kss2, koff, drow, a.S - (int)kv0, kslot(Rc), wave);
+    else Dma::copy_rs(krs, kv0 * kss2, koff, kslot(Rc), wave);
     const uint32_t so = (tri + kt) * blkb + half * halfb + quadb;
     dma16_rs_nt(drs, so, soff0, sslot(Rc) + wave * 1024);
     dma16_rs_nt(drs, so, soff1, sslot(Rc) + (8 + wave) * 1024);
@@ -1804,11 +1893,13 @@ void attn_bwd_dq_ds(BwdArgs a) {
   // query half), register j <-> head-dim row 8 (j / 4) + 4 hh + j % 4.
   const int sl = lane & 31;
   const int q = qt * 64 + qs * 32 + 8 * ((sl & 15) >> 2) + 4 * (sl >> 4) + (sl & 3);
+  if (GEN && q >= a.S) return;
   bf16_t *qrow = a.dq.row(b, h, q);
 #pragma unroll
   for (int db = 0; db < NDB; ++db)
 #pragma unroll
     for (int jq = 0; jq < 4; ++jq) {
+      if (GEN && 32 * db + 8 * jq >= a.D) continue;
       typedef __bf16 bf16x4_t __attribute__((ext_vector_type(4)));
       bf16x4_t o4;
 #pragma unroll
@@ -1913,16 +2004,18 @@ extern "C" int pb_attn_bwd(const pb_bhsd *q, const pb_bhsd *k, const pb_bhsd *v,
 #define PB_BY_D(M, ...) \
   do { if (d <= 32) M(32, __VA_ARGS__); else if (d <= 64) M(64, __VA_ARGS__); else M(128, __VA_ARGS__); } while (0)
   // DMA-pipelined kernels where views, documents and the sequence length allow.
-  const bool pipe = a.vec && (d == 64 || d == 128) && s % 64 == 0 &&
-                    (reinterpret_cast<uintptr_t>(doc_ids) & 15) == 0 && doc_stride % 2 == 0 &&
-                    (reinterpret_cast<uintptr_t>(lse) & 15) == 0 &&
-                    (reinterpret_cast<uintptr_t>(workspace) & 15) == 0 &&
+  const bool pipe = a.vec && (reinterpret_cast<uintptr_t>(workspace) & 15) == 0 &&
                     32 * std::max({q->stride_s, dout->stride_s, k->stride_s, v->stride_s}) <
                         (1LL << 30) &&
                     s * std::max(k->stride_s, v->stride_s) * 2 < (1LL << 31) &&
                     ((hq / hkv - 1) * std::max(q->stride_h, dout->stride_h) +
                      s * std::max(q->stride_s, dout->stride_s)) * 2 < (1LL << 31) &&
                     (hq / hkv) * s * 4 < (1LL << 31) && s * 8 < (1LL << 31);
+  // The forms without bounds; every other length, head dim and alignment of
+  // the documents and lse takes the GEN forms.
+  const bool gen = !((d == 64 || d == 128) && s % 64 == 0 &&
+                     (reinterpret_cast<uintptr_t>(doc_ids) & 15) == 0 && doc_stride % 2 == 0 &&
+                     (reinterpret_cast<uintptr_t>(lse) & 15) == 0);
   // The paired kernel addresses one (pack, GQA group)'s Q / dO rows, and its
   // lse / delta rows, with 32-bit byte offsets.
   const int64_t G = hq / hkv;
@@ -1930,22 +2023,24 @@ extern "C" int pb_attn_bwd(const pb_bhsd *q, const pb_bhsd *k, const pb_bhsd *v,
       ((G - 1) * std::max(q->stride_h, dout->stride_h) + s * std::max(q->stride_s, dout->stride_s)) *
               2 < (1LL << 31) &&
       G * s * 4 < (1LL << 31);
-  const bool pairs = pipe && cfg.pairs && G * s / 32 <= kPairsMaxSteps && pairs_fit;
+  const bool pairs = pipe && cfg.pairs && 2 * G * ((s + 63) / 64) <= kPairsMaxSteps && pairs_fit;
   if (pairs && cfg.ds) {
     // Kept dS: D, then dK/dV storing dS, then dQ = scale * dS K.
     a.ds = ws + delta_bytes;
     a.ds_pair = ds_pair_bytes(G, s);
     const int64_t rows = b * hq * s;
     const int64_t drows = (int64_t)kDeltaRowsPerGroup * (256 / (128 / 8));  // rows per workgroup
-    hipLaunchKernelGGL(attn_bwd_delta<128>, dim3((unsigned)((rows + drows - 1) / drows)), dim3(256),
-                       0, st, a);
+    const dim3 g_d((unsigned)((rows + drows - 1) / drows)), g_ds((unsigned)(b * (hq / 4) * a.nqt_dq));
+    if (gen) hipLaunchKernelGGL((attn_bwd_delta<128, true>), g_d, dim3(256), 0, st, a);
+    else hipLaunchKernelGGL((attn_bwd_delta<128, false>), g_d, dim3(256), 0, st, a);
     rc = launch_status("pb_attn_bwd(delta)");
     if (rc) return rc;
-    hipLaunchKernelGGL((attn_bwd_dkdv_pairs<128, true>), g_kv, dim3(256), 0, st, a);
+    if (gen) hipLaunchKernelGGL((attn_bwd_dkdv_pairs<128, true, true>), g_kv, dim3(256), 0, st, a);
+    else hipLaunchKernelGGL((attn_bwd_dkdv_pairs<128, true, false>), g_kv, dim3(256), 0, st, a);
     rc = launch_status("pb_attn_bwd(dkdv)");
     if (rc) return rc;
-    hipLaunchKernelGGL(attn_bwd_dq_ds<128>, dim3((unsigned)(b * (hq / 4) * a.nqt_dq)), dim3(512), 0,
-                       st, a);
+    if (gen) hipLaunchKernelGGL((attn_bwd_dq_ds<128, true>), g_ds, dim3(512), 0, st, a);
+    else hipLaunchKernelGGL((attn_bwd_dq_ds<128, false>), g_ds, dim3(512), 0, st, a);
     return launch_status("pb_attn_bwd(dq)");
   }
   if (pipe && cfg.dq_chunk > 0) {
@@ -1953,27 +2048,38 @@ extern "C" int pb_attn_bwd(const pb_bhsd *q, const pb_bhsd *k, const pb_bhsd *v,
     g_q.x *= (unsigned)cfg.dq_splits;
   }
   if (pipe) {
-#define PB_DQP(DP, W) hipLaunchKernelGGL((attn_bwd_dq_pipe<DP, W>), g_q, dim3(64 * W), 0, st, a)
-    if (cfg.dq_waves == 4) { if (d == 128) PB_DQP(128, 4); else PB_DQP(64, 4); }
-    else { if (d == 128) PB_DQP(128, 2); else PB_DQP(64, 2); }
+#define PB_DQP(DP, W)                                                                            \
+  do {                                                                                           \
+    if (gen) hipLaunchKernelGGL((attn_bwd_dq_pipe<DP, W, true>), g_q, dim3(64 * W), 0, st, a);   \
+    else hipLaunchKernelGGL((attn_bwd_dq_pipe<DP, W, false>), g_q, dim3(64 * W), 0, st, a);      \
+  } while (0)
+    if (cfg.dq_waves == 4) { if (d > 64) PB_DQP(128, 4); else PB_DQP(64, 4); }
+    else { if (d > 64) PB_DQP(128, 2); else PB_DQP(64, 2); }
 #undef PB_DQP
   } else if (cfg.dq_waves == 4) PB_BY_D(PB_DQ, 4);
   else PB_BY_D(PB_DQ, 2);
   rc = launch_status("pb_attn_bwd(dq)");
   if (rc) return rc;
   if (pipe) {
-#define PB_KVP(DP, W, SP) \
-  hipLaunchKernelGGL((attn_bwd_dkdv_pipe<DP, W, SP>), g_kv, dim3(64 * W), 0, st, a)
-    if (pairs)
-      hipLaunchKernelGGL((attn_bwd_dkdv_pairs<128, false>), g_kv, dim3(256), 0, st, a);
-    else if (cfg.kv_waves == 4) { if (d == 128) PB_KVP(128, 4, false); else PB_KVP(64, 4, false); }
+#define PB_KVP(DP, W, SP)                                                                        \
+  do {                                                                                           \
+    if (gen)                                                                                     \
+      hipLaunchKernelGGL((attn_bwd_dkdv_pipe<DP, W, SP, true>), g_kv, dim3(64 * W), 0, st, a);   \
+    else                                                                                         \
+      hipLaunchKernelGGL((attn_bwd_dkdv_pipe<DP, W, SP, false>), g_kv, dim3(64 * W), 0, st, a);  \
+  } while (0)
+    if (pairs && gen)
+      hipLaunchKernelGGL((attn_bwd_dkdv_pairs<128, false, true>), g_kv, dim3(256), 0, st, a);
+    else if (pairs)
+      hipLaunchKernelGGL((attn_bwd_dkdv_pairs<128, false, false>), g_kv, dim3(256), 0, st, a);
+    else if (cfg.kv_waves == 4) PB_KVP(64, 4, false);  // (wider head dims take 64-row KV tiles)
     else if (cfg.split) {
       // Lists of >= kKvChunkSteps steps are walked as two halves by two workgroups.
       a.kv_chunk = kKvChunkSteps;
       g_kv.x *= 2;
-      if (d == 128) PB_KVP(128, 2, true); else PB_KVP(64, 2, true);
+      if (d > 64) PB_KVP(128, 2, true); else PB_KVP(64, 2, true);
     }
-    else { if (d == 128) PB_KVP(128, 2, false); else PB_KVP(64, 2, false); }
+    else { if (d > 64) PB_KVP(128, 2, false); else PB_KVP(64, 2, false); }
 #undef PB_KVP
   } else if (cfg.kv_waves == 4) PB_BY_D(PB_KV, 4, false);
   else if (cfg.split) PB_BY_D(PB_KV, 2, true);
@@ -1994,8 +2100,11 @@ extern "C" int pb_attn_bwd(const pb_bhsd *q, const pb_bhsd *k, const pb_bhsd *v,
     if (d == 128)
       hipLaunchKernelGGL(attn_bwd_reduce_both<128>, grid, dim3(256), 0, st, a, cfg.dq_q_tile(),
                          (int)kv_blocks);
-    else
+    else if (d == 64)
       hipLaunchKernelGGL(attn_bwd_reduce_both<64>, grid, dim3(256), 0, st, a, cfg.dq_q_tile(),
+                         (int)kv_blocks);
+    else
+      hipLaunchKernelGGL(attn_bwd_reduce_both<0>, grid, dim3(256), 0, st, a, cfg.dq_q_tile(),
                          (int)kv_blocks);
     return launch_status("pb_attn_bwd");
   }
@@ -2009,7 +2118,8 @@ extern "C" int pb_attn_bwd(const pb_bhsd *q, const pb_bhsd *k, const pb_bhsd *v,
   if (q_blocks > 0) {
     const dim3 rgrid((unsigned)q_blocks);
     if (d == 128) hipLaunchKernelGGL(attn_bwd_dq_reduce<128>, rgrid, dim3(256), 0, st, a, cfg.dq_q_tile());
-    else hipLaunchKernelGGL(attn_bwd_dq_reduce<64>, rgrid, dim3(256), 0, st, a, cfg.dq_q_tile());
+    else if (d == 64) hipLaunchKernelGGL(attn_bwd_dq_reduce<64>, rgrid, dim3(256), 0, st, a, cfg.dq_q_tile());
+    else hipLaunchKernelGGL(attn_bwd_dq_reduce<0>, rgrid, dim3(256), 0, st, a, cfg.dq_q_tile());
   }
   return launch_status("pb_attn_bwd");
 }

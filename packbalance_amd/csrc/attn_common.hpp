@@ -169,7 +169,41 @@ struct TileDma {
 #pragma unroll
     for (int i = 0; i < NDMA; ++i) dma16_rs(rs, soff, off[i], dst + (i * W + wave) * 1024);
   }
+  // Any sequence length and any head dim d <= DP that is a multiple of 8: the
+  // chunks of columns past d, and of rows past the sequence end, become zeros
+  // (kDmaZero).  Chunk i's row is row0 + i * kRowStep in every lane, so a
+  // tile needs one compare and one select per instruction, `left` = rows of
+  // the sequence from the tile's first row on (may exceed the tile, or be <= 0).
+  static constexpr int kRowStep = NT / (DP / 8);
+  __device__ static __forceinline__ int offsets_gen(int64_t ss, int wave, int lane, int d,
+                                                    uint32_t *off) {
+    int r0 = 0;
+#pragma unroll
+    for (int i = 0; i < NDMA; ++i) {
+      int r, c;
+      SwzTile<DP>::at((i * (NT / 64) + wave) * 64 + lane, r, c);
+      off[i] = c * 8 < d ? (uint32_t)((r * ss + c * 8) * 2) : kDmaZero;
+      if (i == 0) r0 = r;
+    }
+    return r0;
+  }
+  __device__ static __forceinline__ void copy_gen(__amdgpu_buffer_rsrc_t rs, uint32_t soff,
+                                                  const uint32_t *off, int row0, int left,
+                                                  char *dst, int wave) {
+    constexpr int W = NT / 64;
+#pragma unroll
+    for (int i = 0; i < NDMA; ++i)
+      dma16_rs(rs, soff, row0 < left - i * kRowStep ? off[i] : kDmaZero, dst + (i * W + wave) * 1024);
+  }
 };
+
+// Document ids of rows r0 .. r0 + 31 of one pack into LDS by all 64 lanes of
+// a wave, two lanes per id (rows past the end become zeros): document rows
+// are 8-byte aligned only.
+__device__ __forceinline__ void dma_docs_gen(__amdgpu_buffer_rsrc_t rs, int r0, int S, int lane,
+                                             int64_t *dst) {
+  dma4_rs(rs, (uint32_t)r0 * 8u, (lane >> 1) < S - r0 ? 4u * lane : kDmaZero, dst);
+}
 
 // Exchange with lane ^ 32 without LDS (v_permlane32_swap): returns
 // f(x, x of the partner lane) for a commutative f.
@@ -270,7 +304,10 @@ inline bool views_vectorizable(int64_t d, std::initializer_list<const pb_bhsd *>
 // sub-block holds query row 8 ((s % 16) / 4) + 4 (s / 16) + s % 4 (the row
 // order of the dK/dV kernel's dS accumulators).
 constexpr int64_t kDsMaxBytes = 32LL << 30;
-inline int64_t ds_tri(int64_t s) { return (s / 64) * (s / 64 + 1) / 2; }
+inline int64_t ds_tri(int64_t s) {
+  const int64_t t = (s + 63) / 64;
+  return t * (t + 1) / 2;
+}
 inline int64_t ds_pair_bytes(int64_t g, int64_t s) { return ds_tri(s) * g * 8192; }
 inline int64_t ds_bytes(int64_t b, int64_t hq, int64_t hkv, int64_t s) {
   return b * hkv * ds_pair_bytes(hq / hkv, s);
@@ -278,7 +315,7 @@ inline int64_t ds_bytes(int64_t b, int64_t hq, int64_t hkv, int64_t s) {
 
 struct AttnConfig {
   int fwd_waves, dq_waves, kv_waves, split;
-  int pairs;  // head dim 128 on a full grid: dK/dV by attn_bwd_dkdv_pairs on 64-row KV tiles
+  int pairs;  // head dim 72 .. 128 on a full grid: dK/dV by attn_bwd_dkdv_pairs on 64-row KV tiles
   // dS kept: the paired dK/dV kernel stores its bf16 dS tiles and dQ = scale * dS K
   // is a streaming pass over them (attn_bwd_dq_ds) instead of a kernel that
   // recomputes S and dP; D = rowsum(dO * O) then comes from attn_bwd_delta.
@@ -299,9 +336,9 @@ inline AttnConfig attn_config(int64_t b, int64_t hq, int64_t hkv, int64_t s, int
   c.dq_waves = big_q ? 4 : 2;
   c.kv_waves = b * hkv * tiles(128) >= kFill ? 4 : 2;
   c.split = (c.kv_waves == 2 && b * hkv * tiles(64) < kFill && hq > hkv) ? 1 : 0;
-  // Head dim 128 on a full grid: two (P, dP) wave pairs per 64-row KV tile,
-  // two workgroups per CU (the KV tile of the 2-wave kernels).
-  c.pairs = (d == 128 && c.kv_waves == 4) ? 1 : 0;
+  // Head dims padded to 128 on a full grid: two (P, dP) wave pairs per 64-row
+  // KV tile, two workgroups per CU (the KV tile of the 2-wave kernels).
+  c.pairs = (d > 64 && d % 8 == 0 && c.kv_waves == 4) ? 1 : 0;
   if (c.pairs) c.kv_waves = 2;
   c.ds = (c.pairs && (hq / hkv) % 4 == 0 && ds_pair_bytes(hq / hkv, s) < (1LL << 31) &&
           ds_bytes(b, hq, hkv, s) <= kDsMaxBytes) ? 1 : 0;

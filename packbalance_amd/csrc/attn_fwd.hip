@@ -23,9 +23,9 @@
 // permutation), so P never touches LDS; V^T fragments come from the
 // transposing LDS load ds_read_b64_tr_b16.
 //
-// Two kernels share this scheme: attn_fwd_pipe (16-byte aligned views, head
-// dim 64 or 128, sequence a multiple of 64: DMA-fed swizzled LDS rings and a
-// software-pipelined body, described below) and attn_fwd_generic (everything
+// Two kernels share this scheme: attn_fwd_pipe (16-byte aligned views with a
+// head dim that is a multiple of 8, any length: DMA-fed swizzled LDS rings and
+// a software-pipelined body, described below) and attn_fwd_generic (everything
 // else: K/V staged through registers into padded LDS tiles, element-wise
 // loads where 16-byte access is not allowed).
 #include <algorithm>
@@ -229,8 +229,8 @@ __global__ __launch_bounds__(64 * WAVES) __attribute__((amdgpu_waves_per_eu(2, 2
   }
 }
 
-// Pipelined path (16-byte aligned views and documents, D == DP in {64, 128},
-// sequence length a multiple of 64).
+// Pipelined path (16-byte aligned views; without GEN also 16-byte aligned
+// documents, D == DP in {64, 128} and a sequence length that is a multiple of 64).
 //
 // A wave owns MQ query rows (NQB = MQ/32 column blocks of S^T; each K / V
 // fragment read from LDS feeds NQB MFMAs).  The launch uses MQ = 32, two
@@ -255,7 +255,16 @@ __global__ __launch_bounds__(64 * WAVES) __attribute__((amdgpu_waves_per_eu(2, 2
 // slow path: the max, the O rescale (after PV(u-1), which was relative to the
 // old max) and the exponentials again.  The body waits only for the DMA it
 // issued.
-template <int DP, int MQ, int WAVES>
+//
+// GEN takes any sequence length, any head dim that is a multiple of 8 (padded
+// to DP) and document rows of any alignment: the DMA zero-fills what lies
+// past the sequence or the head dim (TileDma::copy_gen), documents move 4
+// bytes per lane, and the causal test masks the zero rows (a tile that reaches
+// past the end is always a diagonal one).  It costs a compare and a select per
+// DMA instruction, 169 -> 172 registers at D 64.  Against the register-staged
+// kernel above: [4, 1999], 12 / 4 heads, D 64: 84 -> 40 us and an 8 us merge;
+// [1, 6001], 32 / 8 heads, D 128: 404 -> 324 us with the merge.
+template <int DP, int MQ, int WAVES, bool GEN>
 __global__ __launch_bounds__(64 * WAVES)
 __attribute__((amdgpu_waves_per_eu(MQ == 64 ? 1 : 2, MQ == 64 ? 1 : 2)))
 void attn_fwd_pipe(FwdArgs a) {
@@ -325,14 +334,28 @@ void attn_fwd_pipe(FwdArgs a) {
   // One buffer resource per operand for the whole loop; a sub-tile's DMA
   // passes its first row's byte offset as the scalar offset (the host keeps
   // S * row stride * 2 below 2 GiB on this path).
-  const auto krs = buf_rsrc(Kb, (int64_t)S * a.k_ss * 2);
-  const auto vrs = buf_rsrc(Vb, (int64_t)S * a.v_ss * 2);
-  const auto drs = buf_rsrc(docb, (int64_t)S * 8);
+  const auto krs = buf_rsrc(Kb, GEN ? 0x7fffffff : (int64_t)S * a.k_ss * 2);
+  const auto vrs = buf_rsrc(Vb, GEN ? 0x7fffffff : (int64_t)S * a.v_ss * 2);
+  const auto drs = buf_rsrc(docb, GEN ? 0x7fffffff : (int64_t)S * 8);
   const uint32_t kss2 = (uint32_t)(a.k_ss * 2), vss2 = (uint32_t)(a.v_ss * 2);
 
   uint32_t koff[NDMA], voff[NDMA];
-  Dma::offsets(a.k_ss, wave, lane, koff);
-  Dma::offsets(a.v_ss, wave, lane, voff);
+  int drow = 0;  // GEN: this thread's row of a tile's first DMA instruction
+  if constexpr (GEN) {
+    drow = Dma::offsets_gen(a.k_ss, wave, lane, a.D, koff);
+    Dma::offsets_gen(a.v_ss, wave, lane, a.D, voff);
+  } else {
+    Dma::offsets(a.k_ss, wave, lane, koff);
+    Dma::offsets(a.v_ss, wave, lane, voff);
+  }
+  auto copy_k = [&](int r0, char *dst) {
+    if constexpr (GEN) Dma::copy_gen(krs, (uint32_t)r0 * kss2, koff, drow, S - r0, dst, wave);
+    else Dma::copy_rs(krs, (uint32_t)r0 * kss2, koff, dst, wave);
+  };
+  auto copy_v = [&](int r0, char *dst) {
+    if constexpr (GEN) Dma::copy_gen(vrs, (uint32_t)r0 * vss2, voff, drow, S - r0, dst, wave);
+    else Dma::copy_rs(vrs, (uint32_t)r0 * vss2, voff, dst, wave);
+  };
   // Per-lane byte offsets of the fragments within a sub-tile: K row
   // fragments (row l32, columns 16dk + 8hh) and the two transposing reads of
   // a V column fragment (rows 4hh + j/4 and +8, column 32db + ...); rows
@@ -381,8 +404,10 @@ void attn_fwd_pipe(FwdArgs a) {
     qdoc[qb] = docb[qr];
     const bf16_t *qrow = a.q + b * a.q_sb + h * a.q_sh + (int64_t)qr * a.q_ss;
 #pragma unroll
-    for (int dk = 0; dk < NDK; ++dk)
-      qf[qb][dk] = *reinterpret_cast<const bf16x8_t *>(qrow + 16 * dk + 8 * hh);
+    for (int dk = 0; dk < NDK; ++dk) {
+      if (GEN && 16 * dk + 8 * hh >= a.D) qf[qb][dk] = bf16x8_t{};
+      else qf[qb][dk] = *reinterpret_cast<const bf16x8_t *>(qrow + 16 * dk + 8 * hh);
+    }
   }
 
   f32x16_t oacc[NQB][NDB];
@@ -536,7 +561,11 @@ void attn_fwd_pipe(FwdArgs a) {
   // kdoc of sub-tile rows kv0..kv0+31 into a ring slot: one DMA instruction
   // by 16 lanes of wave 0 (issued for every sub-tile, read for PARTIAL ones).
   auto load_kdoc = [&](int kv0, int64_t *dst) {
-    if (wave == 0 && lane < 16) dma16_rs(drs, (uint32_t)kv0 * 8u, 16 * lane, dst);
+    if constexpr (GEN) {
+      if (wave == 0) dma_docs_gen(drs, kv0, S, lane, dst);
+    } else {
+      if (wave == 0 && lane < 16) dma16_rs(drs, (uint32_t)kv0 * 8u, 16 * lane, dst);
+    }
   };
 
   f32x16_t sc[NQB];
@@ -546,10 +575,10 @@ void attn_fwd_pipe(FwdArgs a) {
 #pragma unroll
     for (int i = 0; i < 4; ++i) ew[i] = entry(i + 1);
     auto prefetch = [&](auto Rc, int u) {
-      const int e = entry(u);
-      load_kdoc(row0(e, u), dslot(Rc));
-      Dma::copy_rs(krs, (uint32_t)row0(e, u) * kss2, koff, kslot(Rc), wave);
-      if (decltype(Rc)::value == 0) Dma::copy_rs(vrs, (uint32_t)row0(e, u) * vss2, voff, vslot(Rc), wave);
+      const int r0 = row0(entry(u), u);
+      load_kdoc(r0, dslot(Rc));
+      copy_k(r0, kslot(Rc));
+      if (decltype(Rc)::value == 0) copy_v(r0, vslot(Rc));
     };
     prefetch(I0(), 0);
     prefetch(I1(), 1);
@@ -605,9 +634,10 @@ void attn_fwd_pipe(FwdArgs a) {
       using IR = std::integral_constant<int, R>;
       using IR1 = std::integral_constant<int, R1>;
       using IR2 = std::integral_constant<int, R2>;
-      load_kdoc(row0(e3, u + 3), dslot(IR()));
-      Dma::copy_rs(krs, (uint32_t)row0(e3, u + 3) * kss2, koff, kslot(IR()), wave);
-      Dma::copy_rs(vrs, (uint32_t)row0(e1, u + 1) * vss2, voff, vslot(IR1()), wave);
+      const int rk = row0(e3, u + 3), rv = row0(e1, u + 1);
+      load_kdoc(rk, dslot(IR()));
+      copy_k(rk, kslot(IR()));
+      copy_v(rv, vslot(IR1()));
       // Fragments in the order the steps consume them: steps 0 .. kAhead-1
       // before the first MFMA, step k + kAhead during step k, so at most 12
       // LDS reads are outstanding and each MFMA waits only for its own
@@ -715,11 +745,12 @@ void attn_fwd_pipe(FwdArgs a) {
     if (part) {
       // One chunk's normalised output and log-sum-exp, fp32.
       const int64_t prow = (((int64_t)split * a.B + b) * a.Hq + h) * S + qi[qb];
-      float *po = a.part_o + prow * DP;
+      float *po = a.part_o + prow * (GEN ? a.D : DP);
 #pragma unroll
       for (int db = 0; db < NDB; ++db)
 #pragma unroll
         for (int jq = 0; jq < 4; ++jq) {
+          if (GEN && 32 * db + 8 * jq >= a.D) continue;
           typedef float f32x4_t __attribute__((ext_vector_type(4)));
           f32x4_t o4;
 #pragma unroll
@@ -734,6 +765,7 @@ void attn_fwd_pipe(FwdArgs a) {
     for (int db = 0; db < NDB; ++db)
 #pragma unroll
       for (int jq = 0; jq < 4; ++jq) {
+        if (GEN && 32 * db + 8 * jq >= a.D) continue;
         typedef __bf16 bf16x4_t __attribute__((ext_vector_type(4)));
         bf16x4_t o4;
 #pragma unroll
@@ -746,15 +778,17 @@ void attn_fwd_pipe(FwdArgs a) {
   }
 }
 
-// Merge of the per-chunk outputs of split query tiles: DP/4 threads per
+// Merge of the per-chunk outputs of split query tiles: D/4 threads per
 // (pack, head, query row), four output elements each; rows of unsplit tiles
 // were written by the attention kernel and are skipped.  Pass 1 takes the
 // largest chunk log-sum-exp, pass 2 accumulates the 2^(lse_c - max)-weighted
 // chunk outputs with independent (unrolled) 16-byte loads.
+// DP = 0 takes the head dim (a multiple of 8) from the arguments.
 template <int DP>
 __global__ __launch_bounds__(256) void attn_fwd_combine(FwdArgs a) {
-  constexpr int TPR = DP / 4, RPB = 256 / TPR;
+  const int D = DP ? DP : a.D, TPR = D / 4, RPB = 256 / TPR;
   typedef float f32x4_t __attribute__((ext_vector_type(4)));
+  if ((int)threadIdx.x >= RPB * TPR) return;
   const int64_t row = (int64_t)blockIdx.x * RPB + threadIdx.x / TPR;
   const int d0 = (threadIdx.x % TPR) * 4;
   const int64_t rows = (int64_t)a.B * a.Hq * a.S;
@@ -766,7 +800,7 @@ __global__ __launch_bounds__(256) void attn_fwd_combine(FwdArgs a) {
   const int nch = (cnt + a.chunk - 1) / a.chunk;
   if (nch <= 1) return;
   const float *pl = a.part_lse + row;
-  const float *po = a.part_o + row * DP + d0;
+  const float *po = a.part_o + row * D + d0;
   float mx = -INFINITY;
 #pragma unroll 4
   for (int c = 0; c < nch; ++c) mx = fmaxf(mx, pl[c * rows]);
@@ -776,7 +810,7 @@ __global__ __launch_bounds__(256) void attn_fwd_combine(FwdArgs a) {
 #pragma unroll 4
     for (int c = 0; c < nch; ++c) {
       const float w = fast_exp2(pl[c * rows] - mx);
-      const f32x4_t o = *reinterpret_cast<const f32x4_t *>(po + c * rows * DP);
+      const f32x4_t o = *reinterpret_cast<const f32x4_t *>(po + c * rows * D);
       den += w;
       acc += w * o;
     }
@@ -836,10 +870,10 @@ extern "C" int pb_attn_fwd(const pb_bhsd *q, const pb_bhsd *k, const pb_bhsd *v,
   hipStream_t st = as_stream(stream);
   // DMA offsets are 32-bit: one (pack, KV head) view of K / V (S rows) and
   // the pack's document ids must span < 2 GiB.
-  const bool pipe = a.vec && (d == 64 || d == 128) && s % 64 == 0 &&
-                    (reinterpret_cast<uintptr_t>(doc_ids) & 15) == 0 && doc_stride % 2 == 0 &&
-                    s * std::max(k->stride_s, v->stride_s) * 2 < (1LL << 31) &&
+  const bool pipe = a.vec && s * std::max(k->stride_s, v->stride_s) * 2 < (1LL << 31) &&
                     s * 8 < (1LL << 31);
+  const bool gen = !((d == 64 || d == 128) && s % 64 == 0 &&
+                     (reinterpret_cast<uintptr_t>(doc_ids) & 15) == 0 && doc_stride % 2 == 0);
   if (pipe && cfg.fwd_chunk > 0) {
     PB_CHECK_ARG(workspace != nullptr, "pb_attn_fwd: workspace is required for this shape");
     a.chunk = cfg.fwd_chunk;
@@ -850,11 +884,15 @@ extern "C" int pb_attn_fwd(const pb_bhsd *q, const pb_bhsd *k, const pb_bhsd *v,
     grid.x *= (unsigned)cfg.fwd_splits;
   }
   if (pipe) {
-#define PB_PIPE(DP, W) hipLaunchKernelGGL((attn_fwd_pipe<DP, 32, W>), grid, dim3(64 * W), 0, st, a)
+#define PB_PIPE(DP, W)                                                                           \
+  do {                                                                                           \
+    if (gen) hipLaunchKernelGGL((attn_fwd_pipe<DP, 32, W, true>), grid, dim3(64 * W), 0, st, a); \
+    else hipLaunchKernelGGL((attn_fwd_pipe<DP, 32, W, false>), grid, dim3(64 * W), 0, st, a);    \
+  } while (0)
     if (cfg.fwd_waves == 4) {
-      if (d == 128) PB_PIPE(128, 4); else PB_PIPE(64, 4);
+      if (d > 64) PB_PIPE(128, 4); else PB_PIPE(64, 4);
     } else {
-      if (d == 128) PB_PIPE(128, 2); else PB_PIPE(64, 2);
+      if (d > 64) PB_PIPE(128, 2); else PB_PIPE(64, 2);
     }
 #undef PB_PIPE
     if (a.chunk > 0) {
@@ -863,7 +901,8 @@ extern "C" int pb_attn_fwd(const pb_bhsd *q, const pb_bhsd *k, const pb_bhsd *v,
       const int64_t rows = b * hq * s, rpb = 256 / (d / 4);
       const dim3 cgrid((unsigned)((rows + rpb - 1) / rpb));
       if (d == 128) hipLaunchKernelGGL(attn_fwd_combine<128>, cgrid, dim3(256), 0, st, a);
-      else hipLaunchKernelGGL(attn_fwd_combine<64>, cgrid, dim3(256), 0, st, a);
+      else if (d == 64) hipLaunchKernelGGL(attn_fwd_combine<64>, cgrid, dim3(256), 0, st, a);
+      else hipLaunchKernelGGL(attn_fwd_combine<0>, cgrid, dim3(256), 0, st, a);
     }
   } else {
     // Generic kernel: 32 query rows per wave, same query tile as the plan.

@@ -73,6 +73,18 @@ __device__ __forceinline__ void dma16_rs(__amdgpu_buffer_rsrc_t rs, uint32_t sof
                                            voff, soff, 0, 0);
 }
 
+// A lane offset past every resource's bound: the lane reads nothing and its
+// LDS bytes become zeros, whatever the scalar offset (bounds are < 2 GiB).
+constexpr uint32_t kDmaZero = 0x80000000u;
+
+// LDS DMA of 4 bytes per active lane: lane i writes LDS bytes [4i, 4i + 4) of
+// `dst`.  For rows whose starts are only 4- or 8-byte aligned.
+__device__ __forceinline__ void dma4_rs(__amdgpu_buffer_rsrc_t rs, uint32_t soff, uint32_t voff,
+                                        void *dst) {
+  __builtin_amdgcn_raw_ptr_buffer_load_lds(rs, (__attribute__((address_space(3))) void *)dst, 4,
+                                           voff, soff, 0, 0);
+}
+
 // dma16_rs for data read exactly once: the non-temporal cache policy (nt)
 // marks the lines for early eviction, so a stream does not push re-used
 // tiles out of L2.

@@ -103,6 +103,13 @@ def test_reference_flex_test_case(dev) -> None:
         # 16-step list (two halves), every other tile 14 steps or fewer (whole)
         (1, 8, 2, 1024, 64, [512, 448, -64]),
         (1, 8, 2, 1024, 128, [512, 448, -64]),
+        # lengths that end in every part of a 64-row tile, head dims padded to 64 and 128
+        (1, 4, 2, 1, 64, [1]),
+        (2, 4, 2, 65, 64, [40, 25]),
+        (2, 3, 1, 95, 128, [90, -5]),
+        (1, 4, 4, 97, 96, [33, 64]),
+        (2, 6, 2, 191, 40, [100, 91]),
+        (1, 12, 4, 1999, 64, [1200, 300, 499]),  # split lists of a ragged length
     ],
 )
 def test_attention_matches_oracle(B, Hq, Hkv, S, D, docs, dev) -> None:
@@ -182,6 +189,53 @@ def test_attention_deterministic(dev) -> None:
     b = _run(q, k, v, do, doc)
     for x, y in zip(a, b):
         assert torch.equal(x, y)
+
+
+@pytest.mark.parametrize(
+    "B,Hq,Hkv,S,D",
+    [
+        (9, 32, 8, 1025, 128),  # paired dK/dV with kept dS, one row into a tile
+        (9, 32, 8, 1087, 96),  # the same, head dim padded, one row short of a tile
+        (10, 16, 8, 1056, 128),  # paired dK/dV without kept dS, a sub-tile wholly past the end
+        (9, 12, 12, 639, 72),
+        (12, 24, 8, 1000, 64),  # four-wave kernels at head dim 64
+        (3, 12, 4, 2047, 56),  # the smaller grids: lists in chunks
+        (1, 9, 3, 1350, 64),  # dK/dV split by head, long lists in two halves
+        (1, 4, 1, 801, 120),
+    ],
+)
+def test_ragged_matches_padded(B, Hq, Hkv, S, D, dev) -> None:
+    """The kernels with bounds (any length, head dims that are multiples of 8) against
+    the unbounded ones on the same values: the length padded to a multiple of 64 with
+    another document, the head dim padded with zeros.  Both sides round fp32 sums that
+    differ in order only, so the relative 2-norm stays within one bf16 rounding on
+    either side (2 x 2^-9)."""
+    Sp, Dp = -(-S // 64) * 64, 64 if D <= 64 else 128
+    g = torch.Generator(device=dev).manual_seed(S * D)
+
+    def heads(h):  # [B, S, H, D] memory; columns past D are zero
+        t = torch.randn(B, Sp, h, Dp, device=dev, generator=g).to(torch.bfloat16)
+        t[..., D:] = 0
+        return t.transpose(1, 2)
+
+    q, k, v, do = heads(Hq), heads(Hkv), heads(Hkv), heads(Hq)
+    packs = [W.fill_sequential(np.random.default_rng(S + b), S, np.log(300), 1.0, 1, S)
+             for b in range(B)]
+    doc = W.doc_ids_from_lengths(packs, S).to(dev)
+    doc_p = torch.full((B, Sp), 1 << 40, dtype=torch.int64, device=dev)
+    doc_p[:, :S] = doc
+    do_p = do.clone()
+    do_p[:, :, S:] = 0
+    want = _run(q, k, v, do_p, doc_p, scale=D ** -0.5)
+    cut = [t.transpose(1, 2)[:, :S, :, :D].contiguous().transpose(1, 2) for t in (q, k, v, do)]
+    for layout in ("dense", "view"):
+        if layout == "view":  # rows of the padded memory
+            cut = [t[:, :, :S, :D] for t in (q, k, v, do)]
+        got = _run(*cut, doc, scale=D ** -0.5)
+        for name, a, b in zip(("out", "dq", "dk", "dv"), got, want):
+            b = b[:, :, :S, :D].double()
+            err = (a.double() - b).norm() / b.norm()
+            assert err <= 2 ** -8, f"{layout} {name}: {err:.2e}"
 
 
 @pytest.mark.parametrize("pack", [1, 0])
