@@ -1,0 +1,75 @@
+// Kernel arguments of the bf16 attention kernels, shared by the workgroup
+// kernels (attn_fwd.hip, attn_bwd.hip) and the wave kernels (attn_wave.hip).
+#pragma once
+
+#include "attn_common.hpp"
+
+namespace pb {
+namespace attn {
+
+struct FwdArgs {
+  const bf16_t *q;
+  int64_t q_sb, q_sh, q_ss;
+  const bf16_t *k;
+  int64_t k_sb, k_sh, k_ss;
+  const bf16_t *v;
+  int64_t v_sb, v_sh, v_ss;
+  bf16_t *o;
+  int64_t o_sb, o_sh, o_ss;
+  float *lse;  // [B][Hq][S], log2 domain of the scaled scores
+  const int64_t *doc;
+  int64_t doc_sb;
+  const int32_t *cnt;   // [B][nqt]
+  const int32_t *list;  // [B][nqt][nkt]
+  int B, Hq, Hkv, S, D, nqt, nkt;
+  float sl2;  // softmax scale * log2(e)
+  int vec;    // 16-byte global access allowed
+  // KV split (pipelined kernel): chunk = KV tiles per workgroup (0: whole
+  // list); bm = query rows per tile; partial outputs [split][B][Hq][S][D]
+  // and log-sum-exps [split][B][Hq][S], fp32.
+  int chunk, bm;
+  float *part_o, *part_lse;
+};
+
+struct View {
+  bf16_t *p;
+  int64_t sb, sh, ss;
+  __device__ __forceinline__ bf16_t *row(int b, int h, int64_t s) const {
+    return p + b * sb + h * sh + s * ss;
+  }
+};
+
+struct BwdArgs {
+  View q, k, v, o, dout, dq, dk, dv;
+  const float *lse;
+  float *delta;
+  const int64_t *doc;
+  int64_t doc_sb;
+  const int32_t *qcnt, *qlist;  // dQ plan (by query tile)
+  const int32_t *kcnt, *klist;  // dK/dV plan (by KV tile)
+  float *dk_part, *dv_part;     // split: fp32 [B][Hq][S][D] partials
+  // split, pipelined kernel: a KV tile whose list has at least kv_chunk steps
+  // is walked by two workgroups (first and second half of its steps); the
+  // second writes its partials here.  0: whole lists, these are unused.
+  float *dk_part2, *dv_part2;
+  int kv_chunk, kv_tile;
+  // dQ KV split: KV tiles per workgroup (0: whole list), unscaled fp32 dQ
+  // partials [split][B][Hq][S][D] of query tiles with more than one chunk.
+  int dq_chunk;
+  float *dq_part;
+  // Kept dS blocks (AttnConfig::ds): the region of pack b, KV head hk starts
+  // at ds + (b * Hkv + hk) * ds_pair bytes.
+  char *ds;
+  int64_t ds_pair;
+  int B, Hq, Hkv, S, D;
+  int nqt_dq, nkt_dq, nqt_kv, nkt_kv;
+  float sl2, scale;
+  int vec;
+};
+
+// The wave kernels (AttnConfig::wave): forward, and dQ then dK/dV.
+int launch_fwd_wave(const FwdArgs &a, hipStream_t st);
+int launch_bwd_wave(const BwdArgs &a, hipStream_t st);
+
+}  // namespace attn
+}  // namespace pb

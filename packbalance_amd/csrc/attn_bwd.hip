@@ -32,47 +32,11 @@
 #include <algorithm>
 #include <type_traits>
 
-#include "attn_common.hpp"
+#include "attn_args.hpp"
 
 namespace pb {
 namespace attn {
 
-
-struct View {
-  bf16_t *p;
-  int64_t sb, sh, ss;
-  __device__ __forceinline__ bf16_t *row(int b, int h, int64_t s) const {
-    return p + b * sb + h * sh + s * ss;
-  }
-};
-
-struct BwdArgs {
-  View q, k, v, o, dout, dq, dk, dv;
-  const float *lse;
-  float *delta;
-  const int64_t *doc;
-  int64_t doc_sb;
-  const int32_t *qcnt, *qlist;  // dQ plan (by query tile)
-  const int32_t *kcnt, *klist;  // dK/dV plan (by KV tile)
-  float *dk_part, *dv_part;     // split: fp32 [B][Hq][S][D] partials
-  // split, pipelined kernel: a KV tile whose list has at least kv_chunk steps
-  // is walked by two workgroups (first and second half of its steps); the
-  // second writes its partials here.  0: whole lists, these are unused.
-  float *dk_part2, *dv_part2;
-  int kv_chunk, kv_tile;
-  // dQ KV split: KV tiles per workgroup (0: whole list), unscaled fp32 dQ
-  // partials [split][B][Hq][S][D] of query tiles with more than one chunk.
-  int dq_chunk;
-  float *dq_part;
-  // Kept dS blocks (AttnConfig::ds): the region of pack b, KV head hk starts
-  // at ds + (b * Hkv + hk) * ds_pair bytes.
-  char *ds;
-  int64_t ds_pair;
-  int B, Hq, Hkv, S, D;
-  int nqt_dq, nkt_dq, nqt_kv, nkt_kv;
-  float sl2, scale;
-  int vec;
-};
 
 // Split dK/dV on the pipelined kernel: KV tiles whose step list is at least
 // this long are walked by two workgroups (a 2048-token document's first KV
@@ -81,10 +45,11 @@ struct BwdArgs {
 constexpr int kKvChunkSteps = 16;
 
 // ---------------------------------------------------------------- dK, dV
-template <int DP, int WAVES, bool SPLIT>
+// BM = query rows per plan tile.
+template <int DP, int WAVES, bool SPLIT, int BM>
 __global__ __launch_bounds__(64 * WAVES) void attn_bwd_dkdv(BwdArgs a) {
   constexpr int NT = 64 * WAVES;
-  constexpr int BN = 32 * WAVES, BM = kQStep;
+  constexpr int BN = 32 * WAVES;
   constexpr int QP = DP + 8;  // row-major pitch (elements)
   constexpr int NDK = DP / 16, NDB = DP / 32, CH = DP / 8;
   constexpr int NCH = BM * CH;             // 16-byte chunks of one [BM x DP] tile
@@ -187,10 +152,10 @@ __global__ __launch_bounds__(64 * WAVES) void attn_bwd_dkdv(BwdArgs a) {
     __syncthreads();
     if (step + 1 < steps) fetch(step + 1);
 
-    // S = Q K^T, dP = dO V^T: two 32-query blocks x this wave's 32 KV rows.
-    bf16x8_t pf[4], dsf[4];
+    // S = Q K^T, dP = dO V^T: 32-query blocks x this wave's 32 KV rows.
+    bf16x8_t pf[BM / 16], dsf[BM / 16];
 #pragma unroll
-    for (int qb = 0; qb < 2; ++qb) {
+    for (int qb = 0; qb < BM / 32; ++qb) {
       f32x16_t sacc = zero16(), pacc = zero16();
 #pragma unroll
       for (int dk = 0; dk < NDK; ++dk) {
@@ -212,7 +177,7 @@ __global__ __launch_bounds__(64 * WAVES) void attn_bwd_dkdv(BwdArgs a) {
 #pragma unroll
     for (int db = 0; db < NDB; ++db)
 #pragma unroll
-      for (int qk = 0; qk < 4; ++qk) {
+      for (int qk = 0; qk < BM / 16; ++qk) {
         dv_acc[db] = mfma32(pf[qk], lds_col_frag(Gs, QP, 16 * qk, 32 * db, lane), dv_acc[db]);
         dk_acc[db] = mfma32(dsf[qk], lds_col_frag(Qs, QP, 16 * qk, 32 * db, lane), dk_acc[db]);
       }
@@ -1181,10 +1146,11 @@ __global__ __launch_bounds__(256) void attn_bwd_reduce(BwdArgs a) {
 }
 
 // ---------------------------------------------------------------- dQ
-template <int DP, int WAVES>
+// BN = KV rows per plan tile.
+template <int DP, int WAVES, int BN>
 __device__ __forceinline__ void dq_body(const BwdArgs &a) {
   constexpr int NT = 64 * WAVES;
-  constexpr int BM = 32 * WAVES, BN = kKvStep;
+  constexpr int BM = 32 * WAVES;
   constexpr int KP = DP + 8;
   constexpr int NDK = DP / 16, NDB = DP / 32, CH = DP / 8;
   constexpr int NLD = BN * CH / NT;
@@ -1262,9 +1228,9 @@ __device__ __forceinline__ void dq_body(const BwdArgs &a) {
 
     const int kv0 = plan_tile(e) * BN;
     const bool full = plan_full(e);
-    bf16x8_t dsf[4];
+    bf16x8_t dsf[BN / 16];
 #pragma unroll
-    for (int blk = 0; blk < 2; ++blk) {
+    for (int blk = 0; blk < BN / 32; ++blk) {
       f32x16_t sacc = zero16(), pacc = zero16();
 #pragma unroll
       for (int dk = 0; dk < NDK; ++dk) {
@@ -1285,7 +1251,7 @@ __device__ __forceinline__ void dq_body(const BwdArgs &a) {
 #pragma unroll
     for (int db = 0; db < NDB; ++db)
 #pragma unroll
-      for (int kk = 0; kk < 4; ++kk)
+      for (int kk = 0; kk < BN / 16; ++kk)
         dq_acc[db] = mfma32(lds_col_frag(Ks, KP, 16 * kk, 32 * db, lane), dsf[kk], dq_acc[db]);
   }
   if (!qvalid) return;
@@ -1683,15 +1649,15 @@ __global__ __launch_bounds__(256) void attn_bwd_reduce_both(BwdArgs a, int bm, i
 
 // Two entry points over one body: two waves per SIMD (so one wave's softmax
 // overlaps the other's MFMAs) wherever the registers fit without spilling.
-template <int DP, int WAVES>
+template <int DP, int WAVES, int BN>
 __global__ __launch_bounds__(64 * WAVES) __attribute__((amdgpu_waves_per_eu(2, 2))) void
 attn_bwd_dq(BwdArgs a) {
-  dq_body<DP, WAVES>(a);
+  dq_body<DP, WAVES, BN>(a);
 }
 
 template <int DP, int WAVES>
 __global__ __launch_bounds__(64 * WAVES) void attn_bwd_dq_wide(BwdArgs a) {
-  dq_body<DP, WAVES>(a);
+  dq_body<DP, WAVES, kKvStep>(a);
 }
 
 // ---------------------------------------------------------------- kept-dS dQ
@@ -1930,13 +1896,13 @@ extern "C" int pb_attn_config(int64_t b, int64_t hq, int64_t hkv, int64_t s, int
   }
   const AttnConfig c = attn_config(b, hq, hkv, s, d);
   out[0] = c.fwd_q_tile();
-  out[1] = kKvStep;
-  out[2] = kQStep;
+  out[1] = c.fwd_kv_step();
+  out[2] = c.kv_q_step();
   out[3] = c.kv_tile();
   out[4] = c.dq_q_tile();
-  out[5] = kKvStep;
+  out[5] = c.dq_kv_step();
   out[6] = attn_bwd_workspace(b, hq, hkv, s, d);
-  out[7] = c.split;
+  out[7] = c.split || c.wave_bwd;
   out[8] = attn_fwd_workspace(b, hq, hkv, s, d);
   out[9] = c.fwd_chunk;
   return PB_OK;
@@ -1983,8 +1949,8 @@ extern "C" int pb_attn_bwd(const pb_bhsd *q, const pb_bhsd *k, const pb_bhsd *v,
   a.kcnt = kv_plan_counts; a.klist = kv_plan_lists;
   a.B = (int)b; a.Hq = (int)hq; a.Hkv = (int)hkv; a.S = (int)s; a.D = (int)d;
   a.nqt_dq = (int)((s + cfg.dq_q_tile() - 1) / cfg.dq_q_tile());
-  a.nkt_dq = (int)((s + kKvStep - 1) / kKvStep);
-  a.nqt_kv = (int)((s + kQStep - 1) / kQStep);
+  a.nkt_dq = (int)((s + cfg.dq_kv_step() - 1) / cfg.dq_kv_step());
+  a.nqt_kv = (int)((s + cfg.kv_q_step() - 1) / cfg.kv_q_step());
   a.nkt_kv = (int)((s + cfg.kv_tile() - 1) / cfg.kv_tile());
   a.sl2 = scale * kLog2e;
   a.scale = scale;
@@ -1998,9 +1964,12 @@ extern "C" int pb_attn_bwd(const pb_bhsd *q, const pb_bhsd *k, const pb_bhsd *v,
     if (DP == 128 && W == 2)                                                        \
       hipLaunchKernelGGL((attn_bwd_dq_wide<DP, W>), g_q, dim3(64 * W), 0, st, a);   \
     else                                                                            \
-      hipLaunchKernelGGL((attn_bwd_dq<DP, W>), g_q, dim3(64 * W), 0, st, a);        \
+      hipLaunchKernelGGL((attn_bwd_dq<DP, W, W == 1 ? 32 : kKvStep>), g_q, dim3(64 * W), 0, st, a);     \
   } while (0)
-#define PB_KV(DP, W, SP) hipLaunchKernelGGL((attn_bwd_dkdv<DP, W, SP>), g_kv, dim3(64 * W), 0, st, a)
+#define PB_KV(DP, W, SP)                                                                    \
+  hipLaunchKernelGGL((attn_bwd_dkdv<DP, W, SP, W == 1 ? 32 : kQStep>), g_kv, dim3(64 * W), 0, st, a)
+#define PB_BY_D64(M, ...) \
+  do { if (d <= 32) M(32, __VA_ARGS__); else M(64, __VA_ARGS__); } while (0)
 #define PB_BY_D(M, ...) \
   do { if (d <= 32) M(32, __VA_ARGS__); else if (d <= 64) M(64, __VA_ARGS__); else M(128, __VA_ARGS__); } while (0)
   // DMA-pipelined kernels where views, documents and the sequence length allow.
@@ -2011,6 +1980,7 @@ extern "C" int pb_attn_bwd(const pb_bhsd *q, const pb_bhsd *k, const pb_bhsd *v,
                     ((hq / hkv - 1) * std::max(q->stride_h, dout->stride_h) +
                      s * std::max(q->stride_s, dout->stride_s)) * 2 < (1LL << 31) &&
                     (hq / hkv) * s * 4 < (1LL << 31) && s * 8 < (1LL << 31);
+  if (pipe && cfg.wave_bwd) return launch_bwd_wave(a, st);
   // The forms without bounds; every other length, head dim and alignment of
   // the documents and lse takes the GEN forms.
   const bool gen = !((d == 64 || d == 128) && s % 64 == 0 &&
@@ -2057,6 +2027,7 @@ extern "C" int pb_attn_bwd(const pb_bhsd *q, const pb_bhsd *k, const pb_bhsd *v,
     else { if (d > 64) PB_DQP(128, 2); else PB_DQP(64, 2); }
 #undef PB_DQP
   } else if (cfg.dq_waves == 4) PB_BY_D(PB_DQ, 4);
+  else if (cfg.dq_waves == 1) PB_BY_D64(PB_DQ, 1);  // the tiles of the wave kernels
   else PB_BY_D(PB_DQ, 2);
   rc = launch_status("pb_attn_bwd(dq)");
   if (rc) return rc;
@@ -2082,9 +2053,11 @@ extern "C" int pb_attn_bwd(const pb_bhsd *q, const pb_bhsd *k, const pb_bhsd *v,
     else { if (d > 64) PB_KVP(128, 2, false); else PB_KVP(64, 2, false); }
 #undef PB_KVP
   } else if (cfg.kv_waves == 4) PB_BY_D(PB_KV, 4, false);
+  else if (cfg.kv_waves == 1) PB_BY_D64(PB_KV, 1, false);
   else if (cfg.split) PB_BY_D(PB_KV, 2, true);
   else PB_BY_D(PB_KV, 2, false);
 #undef PB_BY_D
+#undef PB_BY_D64
 #undef PB_KV
 #undef PB_DQ
   rc = launch_status("pb_attn_bwd(dkdv)");

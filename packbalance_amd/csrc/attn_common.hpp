@@ -322,10 +322,38 @@ struct AttnConfig {
   int ds;
   int fwd_chunk, fwd_splits;  // 0 / 1: no forward KV split
   int dq_chunk, dq_splits;    // the same for the (q-major) dQ kernel
+  // Head dims to 64 on small grids: the wave kernels (attn_wave.hip) on 32 x 32
+  // tiles.  Views they cannot take run the register-staged kernels on the same tiles.
+  int wave_fwd, wave_bwd;
+  int fwd_kv_step() const { return wave_fwd ? 32 : kKvStep; }
+  int dq_kv_step() const { return wave_bwd ? 32 : kKvStep; }
+  int kv_q_step() const { return wave_bwd ? 32 : kQStep; }
   int fwd_q_tile() const { return 32 * fwd_waves; }
   int dq_q_tile() const { return 32 * dq_waves; }
   int kv_tile() const { return 32 * kv_waves; }
 };
+
+// When the wave kernels serve a shape (see attn_wave.hip): head dims to 64 and
+// a small grid, counted in 128-row query tiles over all heads; kWaveMaxS bounds
+// the list entries a wave can hold.  The lines lie where the wave kernels win
+// for short and for whole-sequence documents alike, with the head counts of
+// [B, S], 12 / 4 heads, D 64 in us, workgroup -> wave kernels:
+//   forward   [4, 2048] 42 -> 27 (one document: 68 -> 60), [8, 2048] 72 -> 52,
+//             but [16, 2048] 107 -> 94 (one document: 179 -> 204)
+//   backward  [4, 2048] 112 -> 66 (249 -> 149), [16, 2048] 299 -> 241 (535 ->
+//             491), but [16, 4096] 752 -> 765 (1648 -> 1804)
+constexpr int kWaveLeast = 6;  // least steps of a list worth another wave
+constexpr int64_t kWaveMaxS = 4096;
+inline int64_t wave_tiles(int64_t b, int64_t hq, int64_t s, int64_t d) {
+  if (d > 64 || d % 8 || s > kWaveMaxS) return INT64_MAX;
+  return b * hq * ((s + 127) / 128);
+}
+inline bool wave_fwd_grid(int64_t b, int64_t hq, int64_t s, int64_t d) {
+  return wave_tiles(b, hq, s, d) <= (s <= 2048 ? 1536 : 1024);
+}
+inline bool wave_bwd_grid(int64_t b, int64_t hq, int64_t s, int64_t d) {
+  return wave_tiles(b, hq, s, d) <= 3072;
+}
 
 inline AttnConfig attn_config(int64_t b, int64_t hq, int64_t hkv, int64_t s, int64_t d) {
   const int64_t kFill = 512;  // two workgroups per CU on 256 CUs
@@ -343,6 +371,13 @@ inline AttnConfig attn_config(int64_t b, int64_t hq, int64_t hkv, int64_t s, int
   c.ds = (c.pairs && (hq / hkv) % 4 == 0 && ds_pair_bytes(hq / hkv, s) < (1LL << 31) &&
           ds_bytes(b, hq, hkv, s) <= kDsMaxBytes) ? 1 : 0;
   if (c.ds) c.dq_waves = 2;  // dQ on the 64-row query tiles of the dS blocks
+  c.wave_fwd = wave_fwd_grid(b, hq, s, d) ? 1 : 0;
+  c.wave_bwd = wave_bwd_grid(b, hq, s, d) ? 1 : 0;
+  if (c.wave_fwd) c.fwd_waves = 1;
+  if (c.wave_bwd) {
+    c.dq_waves = c.kv_waves = 1;
+    c.split = c.pairs = c.ds = 0;
+  }
   // Aim for ~2048 chunk workgroups over all lists, but at least 4 KV tiles
   // each (a chunk also pays the prologue and the merge).  Measured on the
   // cfg2 step (two [2, 2048] micro-batches on two streams; attention kernel
@@ -359,8 +394,12 @@ inline AttnConfig attn_config(int64_t b, int64_t hq, int64_t hkv, int64_t s, int
       splits_out = (int)((nkt + chunk - 1) / chunk);
     }
   };
-  kv_split(c.fwd_q_tile(), c.fwd_chunk, c.fwd_splits);
-  kv_split(c.dq_q_tile(), c.dq_chunk, c.dq_splits);
+  c.fwd_chunk = kWaveLeast;  // (KV tiles of a list before a second wave shares it)
+  c.fwd_splits = 1;
+  c.dq_chunk = 0;
+  c.dq_splits = 1;
+  if (!c.wave_fwd) kv_split(c.fwd_q_tile(), c.fwd_chunk, c.fwd_splits);
+  if (!c.wave_bwd) kv_split(c.dq_q_tile(), c.dq_chunk, c.dq_splits);
   return c;
 }
 
@@ -368,7 +407,7 @@ inline AttnConfig attn_config(int64_t b, int64_t hq, int64_t hkv, int64_t s, int
 // [splits, b, hq, s, d] and log-sum-exps [splits, b, hq, s], fp32.
 inline int64_t attn_fwd_workspace(int64_t b, int64_t hq, int64_t hkv, int64_t s, int64_t d) {
   const AttnConfig c = attn_config(b, hq, hkv, s, d);
-  if (c.fwd_chunk == 0) return 0;
+  if (c.fwd_chunk == 0 || c.wave_fwd) return 0;
   const int64_t rows = (int64_t)c.fwd_splits * b * hq * s;
   return (rows * d * 4 + 255) / 256 * 256 + (rows * 4 + 255) / 256 * 256;
 }

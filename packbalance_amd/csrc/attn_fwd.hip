@@ -31,41 +31,18 @@
 #include <algorithm>
 #include <type_traits>
 
-#include "attn_common.hpp"
+#include "attn_args.hpp"
 
 namespace pb {
 namespace attn {
 
-struct FwdArgs {
-  const bf16_t *q;
-  int64_t q_sb, q_sh, q_ss;
-  const bf16_t *k;
-  int64_t k_sb, k_sh, k_ss;
-  const bf16_t *v;
-  int64_t v_sb, v_sh, v_ss;
-  bf16_t *o;
-  int64_t o_sb, o_sh, o_ss;
-  float *lse;  // [B][Hq][S], log2 domain of the scaled scores
-  const int64_t *doc;
-  int64_t doc_sb;
-  const int32_t *cnt;   // [B][nqt]
-  const int32_t *list;  // [B][nqt][nkt]
-  int B, Hq, Hkv, S, D, nqt, nkt;
-  float sl2;  // softmax scale * log2(e)
-  int vec;    // 16-byte global access allowed
-  // KV split (pipelined kernel): chunk = KV tiles per workgroup (0: whole
-  // list); bm = query rows per tile; partial outputs [split][B][Hq][S][D]
-  // and log-sum-exps [split][B][Hq][S], fp32.
-  int chunk, bm;
-  float *part_o, *part_lse;
-};
-
 // Generic path: any head dim <= 128, any strides / alignment (element-wise
 // loads where 16-byte access is not allowed), K/V staged through registers.
-template <int DP, int WAVES>
+// BN = KV rows per plan tile.
+template <int DP, int WAVES, int BN>
 __global__ __launch_bounds__(64 * WAVES) __attribute__((amdgpu_waves_per_eu(2, 2))) void attn_fwd_generic(FwdArgs a) {
   constexpr int NT = 64 * WAVES;
-  constexpr int BM = 32 * WAVES, BN = kKvStep;
+  constexpr int BM = 32 * WAVES, NBLK = BN / 32;
   constexpr int KP = DP + 8;  // K / V row pitch in LDS (elements)
   constexpr int NDK = DP / 16;
   constexpr int NDB = DP / 32;
@@ -140,10 +117,10 @@ __global__ __launch_bounds__(64 * WAVES) __attribute__((amdgpu_waves_per_eu(2, 2
     __syncthreads();
     if (it + 1 < cnt) fetch(lst[it + 1]);
 
-    // S^T = K Q^T for the two 32-row halves of the tile.
-    f32x16_t sacc[2];
+    // S^T = K Q^T for the 32-row blocks of the tile.
+    f32x16_t sacc[NBLK];
 #pragma unroll
-    for (int blk = 0; blk < 2; ++blk) {
+    for (int blk = 0; blk < NBLK; ++blk) {
       sacc[blk] = zero16();
 #pragma unroll
       for (int dk = 0; dk < NDK; ++dk) {
@@ -159,7 +136,7 @@ __global__ __launch_bounds__(64 * WAVES) __attribute__((amdgpu_waves_per_eu(2, 2
     float mloc = -INFINITY;
     if (!full) {
 #pragma unroll
-      for (int blk = 0; blk < 2; ++blk)
+      for (int blk = 0; blk < NBLK; ++blk)
 #pragma unroll
         for (int j = 0; j < 16; ++j) {
           const int kr_ = 32 * blk + 8 * (j >> 2) + 4 * hh + (j & 3);
@@ -169,7 +146,7 @@ __global__ __launch_bounds__(64 * WAVES) __attribute__((amdgpu_waves_per_eu(2, 2
         }
     }
 #pragma unroll
-    for (int blk = 0; blk < 2; ++blk)
+    for (int blk = 0; blk < NBLK; ++blk)
 #pragma unroll
       for (int j = 0; j < 16; ++j) mloc = fmaxf(mloc, sacc[blk][j]);
     mloc = fmaxf(mloc, __shfl_xor(mloc, 32)) * a.sl2;
@@ -183,9 +160,9 @@ __global__ __launch_bounds__(64 * WAVES) __attribute__((amdgpu_waves_per_eu(2, 2
 #pragma unroll
       for (int j = 0; j < 16; ++j) oacc[db][j] *= alpha;
 
-    bf16x8_t pf[4];
+    bf16x8_t pf[2 * NBLK];
 #pragma unroll
-    for (int blk = 0; blk < 2; ++blk)
+    for (int blk = 0; blk < NBLK; ++blk)
 #pragma unroll
       for (int j = 0; j < 16; ++j) {
         const float p = fast_exp2(fmaf(sacc[blk][j], a.sl2, -m_use));
@@ -198,7 +175,7 @@ __global__ __launch_bounds__(64 * WAVES) __attribute__((amdgpu_waves_per_eu(2, 2
 #pragma unroll
     for (int db = 0; db < NDB; ++db)
 #pragma unroll
-      for (int kk = 0; kk < 4; ++kk)
+      for (int kk = 0; kk < 2 * NBLK; ++kk)
         oacc[db] = mfma32(lds_col_frag(Vs, KP, 16 * kk, 32 * db, lane), pf[kk], oacc[db]);
   }
 
@@ -859,7 +836,7 @@ extern "C" int pb_attn_fwd(const pb_bhsd *q, const pb_bhsd *k, const pb_bhsd *v,
   a.B = (int)b; a.Hq = (int)hq; a.Hkv = (int)hkv; a.S = (int)s; a.D = (int)d;
   const AttnConfig cfg = attn_config(b, hq, hkv, s, d);
   a.nqt = (int)((s + cfg.fwd_q_tile() - 1) / cfg.fwd_q_tile());
-  a.nkt = (int)((s + kKvStep - 1) / kKvStep);
+  a.nkt = (int)((s + cfg.fwd_kv_step() - 1) / cfg.fwd_kv_step());
   a.sl2 = scale * kLog2e;
   a.vec = views_vectorizable(d, {q, k, v, out});
   a.chunk = 0;
@@ -872,6 +849,7 @@ extern "C" int pb_attn_fwd(const pb_bhsd *q, const pb_bhsd *k, const pb_bhsd *v,
   // the pack's document ids must span < 2 GiB.
   const bool pipe = a.vec && s * std::max(k->stride_s, v->stride_s) * 2 < (1LL << 31) &&
                     s * 8 < (1LL << 31);
+  if (pipe && cfg.wave_fwd) return launch_fwd_wave(a, st);
   const bool gen = !((d == 64 || d == 128) && s % 64 == 0 &&
                      (reinterpret_cast<uintptr_t>(doc_ids) & 15) == 0 && doc_stride % 2 == 0);
   if (pipe && cfg.fwd_chunk > 0) {
@@ -905,10 +883,13 @@ extern "C" int pb_attn_fwd(const pb_bhsd *q, const pb_bhsd *k, const pb_bhsd *v,
       else hipLaunchKernelGGL(attn_fwd_combine<0>, cgrid, dim3(256), 0, st, a);
     }
   } else {
-    // Generic kernel: 32 query rows per wave, same query tile as the plan.
+    // Generic kernel: 32 query rows per wave, same tiles as the plan.
     const int w = cfg.fwd_q_tile() / 32;
-#define PB_FWD(DP, W) hipLaunchKernelGGL((attn_fwd_generic<DP, W>), grid, dim3(64 * W), 0, st, a)
-    if (w == 4) {
+#define PB_FWD(DP, W)                                                                          \
+  hipLaunchKernelGGL((attn_fwd_generic<DP, W, W == 1 ? 32 : kKvStep>), grid, dim3(64 * W), 0, st, a)
+    if (w == 1) {  // the tiles of attn_fwd_wave (d <= 64)
+      if (d <= 32) PB_FWD(32, 1); else PB_FWD(64, 1);
+    } else if (w == 4) {
       if (d <= 32) PB_FWD(32, 4); else if (d <= 64) PB_FWD(64, 4); else PB_FWD(128, 4);
     } else {
       if (d <= 32) PB_FWD(32, 2); else if (d <= 64) PB_FWD(64, 2); else PB_FWD(128, 2);

@@ -197,7 +197,10 @@ def _plans(doc: torch.Tensor, hq: int, hkv: int, head_dim: int, block_mask) -> d
         return cache[key]
     b, s = doc.shape
     cfg = attn_config(b, hq, hkv, s, head_dim)
-    plans = {k: _Plan(doc, k, *cfg["tiles"][k]) for k in (FWD, BWD_KV, BWD_Q)}
+    plans = {k: _Plan(doc, k, *cfg["tiles"][k]) for k in (FWD, BWD_KV)}
+    # dQ walks KV tiles as the forward does: the same plan where the tiles are the same
+    same = cfg["tiles"][BWD_Q] == cfg["tiles"][FWD]
+    plans[BWD_Q] = plans[FWD] if same else _Plan(doc, BWD_Q, *cfg["tiles"][BWD_Q])
     plans["workspace"] = cfg["workspace"]
     plans["fwd_workspace"] = cfg["fwd_workspace"]
     if cache is not None:

@@ -238,6 +238,54 @@ def test_ragged_matches_padded(B, Hq, Hkv, S, D, dev) -> None:
             assert err <= 2 ** -8, f"{layout} {name}: {err:.2e}"
 
 
+@pytest.mark.parametrize(
+    "B,Hq,Hkv,S,D,mu,misaligned",
+    [
+        (1, 4, 2, 4096, 64, 1e9, False),  # one document: the longest lists, 64 steps a wave
+        (1, 2, 1, 4096, 64, 40, False),  # short lists: single waves
+        (2, 12, 4, 2048, 64, 200, False),  # dK/dV lists shared by four waves
+        (4, 16, 16, 2017, 64, 500, False),  # by two
+        (9, 16, 16, 2048, 48, 150, False),  # by none
+        (5, 8, 1, 777, 64, 90, False),  # G = 8
+        (8, 12, 4, 2048, 64, 300, False),  # the largest forward grid of these kernels
+        (9, 12, 4, 2048, 64, 300, False),  # past it: another forward, the same backward
+        (2, 4, 2, 333, 64, 60, True),  # rows without 16-byte alignment: register-staged
+        (2, 4, 2, 333, 32, 60, True),
+    ],
+)
+def test_small_grid_matches_padded_head_dim(B, Hq, Hkv, S, D, mu, misaligned, dev) -> None:
+    """The 32 x 32 tile kernels of small grids (head dims to 64) against the workgroup
+    kernels on the same values with the head dim padded to 128 by zeros.  Either side
+    rounds P or dS and then the output to bf16, each at most 2^-9 of the value and
+    2^-9 / sqrt(3) in the mean square, so the relative 2-norm of the difference stays
+    below 2 x 2^-9."""
+    g = torch.Generator(device=dev).manual_seed(S * D + B)
+
+    def heads(h):
+        t = torch.randn(B, S, h, 128, device=dev, generator=g).to(torch.bfloat16)
+        t[..., D:] = 0
+        return t.transpose(1, 2)
+
+    wide = [heads(Hq), heads(Hkv), heads(Hkv), heads(Hq)]
+    packs = [W.fill_sequential(np.random.default_rng(S + b), S, np.log(mu), 1.0, 1, S)
+             for b in range(B)]
+    doc = W.doc_ids_from_lengths(packs, S).to(dev)
+    want = _run(*wide, doc, scale=D ** -0.5)
+
+    def cut(t):
+        if not misaligned:
+            return t[..., :D].transpose(1, 2).contiguous().transpose(1, 2)
+        mem = torch.zeros(B, S, t.shape[1], D + 1, dtype=t.dtype, device=dev)
+        mem[..., :D] = t[..., :D].transpose(1, 2)
+        return mem[..., :D].transpose(1, 2)
+
+    got = _run(*(cut(t) for t in wide), doc, scale=D ** -0.5)
+    for name, a, b in zip(("out", "dq", "dk", "dv"), got, want):
+        b = b[..., :D].double()
+        err = (a.double() - b).norm() / b.norm()
+        assert err <= 2 ** -8, f"{name}: {err:.2e}"
+
+
 @pytest.mark.parametrize("pack", [1, 0])
 def test_attention_cfg3_pack(pack, dev) -> None:
     """cfg3 shape (S=8192, Hq=32, Hkv=8, D=128): all 8 packs run, one pack x one
