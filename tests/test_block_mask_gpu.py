@@ -128,3 +128,41 @@ def test_attention_plans_match_oracle(q_tile, kv_tile, by_kv, dev) -> None:
             assert counts[i, r] == len(want), (i, r)
             assert lists[i, r, : len(want)].tolist() == want, (i, r)
     assert kinds == {0, 1, 2}
+
+
+@pytest.mark.parametrize("q_tile,kv_tile", [(32, 32), (128, 64), (64, 128), (1024, 32), (7, 5)])
+@pytest.mark.parametrize("s,kind", [(1, "sorted"), (97, "sorted"), (1025, "sorted"), (700, "mixed"),
+                                    (1999, "padded")])
+def test_plan_rows_match_dense(q_tile, kv_tile, s, kind, dev) -> None:
+    """Both orientations of a plan against the dense mask: ids that recur in any order,
+    one id per token, tiles longer than a wave, and tiles cut by the sequence end."""
+    from packbalance_amd import _native as N
+
+    rng = np.random.default_rng(s + q_tile)
+    d = np.sort(rng.integers(0, max(1, s // 60), s)).astype(np.int64)
+    if kind == "mixed":
+        d = rng.permutation(d)
+    if kind == "padded":
+        d[-40:] = -1
+    doc = torch.from_numpy(d)[None].to(dev)
+    nq, nk = -(-s // q_tile), -(-s // kv_tile)
+    pos = np.arange(s)
+    causal, same = pos[:, None] >= pos[None], d[:, None] == d[None]
+    want = np.zeros((nq, nk), dtype=np.int64) - 1  # -1: empty
+    for i in range(nq):
+        for j in range(nk):
+            qs, ks = slice(i * q_tile, (i + 1) * q_tile), slice(j * kv_tile, (j + 1) * kv_tile)
+            c, e = causal[qs, ks], same[qs, ks]
+            if (c & e).any():
+                full = c.shape == (q_tile, kv_tile) and (c & e).all()
+                want[i, j] = 1 if full else 2 if e[c].all() else 0
+    for by_kv in (0, 1):
+        w = want.T if by_kv else want
+        counts = torch.empty((1, w.shape[0]), dtype=torch.int32, device=dev)
+        lists = torch.full((1,) + w.shape, -7, dtype=torch.int32, device=dev)
+        ws = torch.empty(nq * nk, dtype=torch.uint8, device=dev)
+        N.call("pb_attn_plan", doc.data_ptr(), doc.stride(0), 1, s, q_tile, kv_tile, by_kv,
+               counts.data_ptr(), lists.data_ptr(), ws.data_ptr(), N.stream_ptr(doc))
+        for r in range(w.shape[0]):
+            row = [(c << 2) | int(k) for c, k in enumerate(w[r]) if k >= 0]
+            assert lists[0, r, :int(counts[0, r])].tolist() == row, (by_kv, r)
