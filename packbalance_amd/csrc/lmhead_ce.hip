@@ -8,11 +8,11 @@
 // dx = dlogits W, dW = dlogits^T x, both scaled by grad_output.
 //
 // Everything runs on one bf16 MFMA GEMM, C[m][n] = sum_k A[m][k] B[n][k]
-// (both operands K-contiguous, "NT"), with four epilogues.  gemm_nt_dma takes
-// K in whole 64-element slices: LDS-DMA rings of swizzled slices, 256 x 128
-// tiles on 8 waves for the backward products and 256 x 256 tiles for the
-// forward; gemm_nt (128 x 128 x 64, four waves of 64 x 64, register-staged)
-// handles any other K.  Epilogues:
+// (both operands K-contiguous, "NT"), with four epilogues.  gemm_nt_dma reads
+// LDS-DMA rings of swizzled K slices in one of three tile shapes; gemm_nt
+// (128 x 128 x 64, four waves of 64 x 64, register-staged) takes the dx / dW
+// products whose K is not whole 64-element slices, and rows too far apart for
+// a tile's 2 GiB of DMA offsets.  Epilogues:
 //   kLse      A = W, B = x: C = logits^T, lane <-> token.  Per token, a
 //             (max, sum exp) partial over the tile's vocab rows and the
 //             target logit; the [tokens x vocab] tile is discarded, or also
@@ -29,6 +29,8 @@
 // single workgroup sums the rows in a fixed order (deterministic scalar).
 #include <math.h>
 
+#include <type_traits>
+
 #include "common.hpp"
 #include "lds_dma.hpp"
 
@@ -36,7 +38,11 @@ namespace pb {
 namespace ce {
 
 typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
+typedef __bf16 bf16x4_t __attribute__((ext_vector_type(4)));
 typedef float f32x16_t __attribute__((ext_vector_type(16)));
+typedef short i16x4_t __attribute__((ext_vector_type(4)));
+typedef short i16x8_t __attribute__((ext_vector_type(8)));
+typedef __attribute__((address_space(3))) i16x4_t lds_i16x4_t;
 
 constexpr int BM = 128, BN = 128, BK = 64;
 constexpr int AP = BK + 8;  // LDS row pitch (elements): 144 bytes, 16-byte aligned rows
@@ -107,16 +113,16 @@ __device__ __forceinline__ void store_out(void *out, int dtype, int64_t idx, flo
 }
 
 // ---------------------------------------------------------------- DMA GEMM
-// gemm_nt_dma: the product for K-slices that are whole multiples of 64, on
-// tiles of WM x WN waves, each wave 32*IM x 32*JN (IM x JN MFMA blocks).  The
+// gemm_nt_dma: the product on tiles of WM x WN waves, each wave 32*IM x 32*JN (IM x JN MFMA blocks).  The
 // A and B K-slices arrive by LDS DMA (16-byte buffer loads, rows past M / N
 // read as zero) in the swizzled 128-byte-row layout of SwzTile<64>
 // (conflict-free ds_read_b128 fragments, no padding), through a ring of
-// STAGES slices: the slices STAGES-1 steps ahead are in flight while one is
+// STAGES slices: the slices up to STAGES steps ahead are in flight while one is
 // computed, with a single barrier per slice.  Workgroup i runs on XCD i % 8;
 // each XCD takes a contiguous range of tiles in groups of kGroupM tile rows,
 // so the workgroups resident on one XCD share A and B panels in its L2.
-// gemm_nt (below) is the register-staged kernel for every other shape.
+// K need not be whole slices with TAIL (K % 8 == 0: whole 16-byte chunks).
+// gemm_nt (below) is the register-staged kernel for every other K.
 constexpr int kGroupM = 8;
 
 __device__ __forceinline__ void tile_of(int id, int ntm, int ntn, int &tm, int &tn) {
@@ -129,12 +135,28 @@ __device__ __forceinline__ void tile_of(int id, int ntm, int ntn, int &tm, int &
   tn = local / rows;
 }
 
+// Row of token n's target relative to vocab row v0 + m when it is one of the
+// `rows` rows from there (below M) and the token counts, else -1.
+__device__ __forceinline__ int target_row(const GemmArgs &g, int n, int m, int rows) {
+  const int64_t t = n < g.N ? g.targets[n] : g.ignore_index;
+  const int64_t rel = t - g.v0 - m;
+  return t != g.ignore_index && rel >= 0 && rel < rows && m + rel < g.M ? (int)rel : -1;
+}
+
+// Keeps this wave's LDS accesses (in order in the hardware) in program order.
+__device__ __forceinline__ void lds_order() {
+  asm volatile("" ::: "memory");
+  __builtin_amdgcn_wave_barrier();
+}
+
+constexpr int kDlPitch = 64 + 8;                      // elements per staging row of kDlogits
+constexpr int kDlStage = 64 * kDlPitch * 2;           // bytes a wave stages
+
 // Epilogue of a finished tile (both kernels), WM x WN waves of 64*WM*WN
 // threads: acc[i][j] of wave (wm, wn) = (wave / WN, wave % WN) holds rows
 // m0 + 32*IM*wm + 32i + 8(r/4) + 4hh + r%4 and column n0 + 32*JN*wn + 32j + l32.
-// kDlogits stages its bf16 rows (vocab-major, pitch BN + 8) in `stage`, one
-// wave row (32*IM rows) at a time, so both dlogits layouts leave as 16-byte
-// stores; the caller has finished every read of `stage` as an operand buffer.
+// `stage`: LDS of the workgroup (kLse) or of this wave (kDlogits, kDlStage
+// bytes) whose reads as an operand buffer are finished.
 template <int MODE, int WM, int WN, int IM, int JN>
 __device__ __forceinline__ void gemm_epilogue(const GemmArgs &g, f32x16_t (&acc)[IM][JN], int tm,
                                               int m0, int n0, bf16_t *stage,
@@ -202,41 +224,53 @@ __device__ __forceinline__ void gemm_epilogue(const GemmArgs &g, f32x16_t (&acc)
           }
       }
     }
+    auto partial = [&](auto Full) {
+      constexpr bool full = decltype(Full)::value;  // every row of the tile is < M
 #pragma unroll
-    for (int j = 0; j < JN; ++j) {
-      const int nl = WC * wn + 32 * j + l32;
-      const int n = n0 + nl;
-      const bool nvalid = n < g.N;
-      const int64_t t = nvalid ? g.targets[n] : g.ignore_index;
-      const bool valid = nvalid && t != g.ignore_index;
-      float mx = -INFINITY;
+      for (int j = 0; j < JN; ++j) {
+        const int nl = WC * wn + 32 * j + l32;
+        const int n = n0 + nl;
+        const int rel = target_row(g, n, m0 + WR * wm + 4 * hh, WR);
+        float mx = -INFINITY;
 #pragma unroll
-      for (int i = 0; i < IM; ++i)
+        for (int i = 0; i < IM; ++i)
 #pragma unroll
-        for (int r = 0; r < 16; ++r) {
-          const int m = m0 + WR * wm + 32 * i + 8 * (r >> 2) + 4 * hh + (r & 3);
-          if (m < g.M) {
-            mx = fmaxf(mx, acc[i][j][r]);
-            if (valid && (int64_t)(g.v0 + m) == t) g.tgt[n] = acc[i][j][r];
+          for (int r = 0; r < 16; ++r) {
+            const int mo = 32 * i + 8 * (r >> 2) + (r & 3);
+            if (full || m0 + WR * wm + 4 * hh + mo < g.M) mx = fmaxf(mx, acc[i][j][r]);
           }
-        }
-      mx *= kLog2e;
-      float sm = 0.f;
+        if (__any(rel >= 0)) {  // few waves hold the target of one of their tokens
+          float tv = 0.f;
 #pragma unroll
-      for (int i = 0; i < IM; ++i)
+          for (int i = 0; i < IM; ++i)
 #pragma unroll
-        for (int r = 0; r < 16; ++r) {
-          const int m = m0 + WR * wm + 32 * i + 8 * (r >> 2) + 4 * hh + (r & 3);
-          if (m < g.M) sm += fast_exp2(acc[i][j][r] * kLog2e - mx);
+            for (int r = 0; r < 16; ++r)
+              tv = rel == 32 * i + 8 * (r >> 2) + (r & 3) ? acc[i][j][r] : tv;
+          if (rel >= 0 && (rel & 4) == 0) g.tgt[n] = tv;
         }
-      const float mo = __shfl_xor(mx, 32), so = __shfl_xor(sm, 32);
-      const float mn = fmaxf(mx, mo);
-      if (mn != -INFINITY) sm = sm * fast_exp2(mx - mn) + so * fast_exp2(mo - mn);
-      if (hh == 0) {
-        red_m[wm][nl] = mn;
-        red_s[wm][nl] = sm;
+        mx *= kLog2e;
+        float sm = 0.f;
+#pragma unroll
+        for (int i = 0; i < IM; ++i)
+#pragma unroll
+          for (int r = 0; r < 16; ++r) {
+            const int mo = 32 * i + 8 * (r >> 2) + (r & 3);
+            if (full || m0 + WR * wm + 4 * hh + mo < g.M)
+              sm += fast_exp2(acc[i][j][r] * kLog2e - mx);
+          }
+        const float mo = __shfl_xor(mx, 32), so = __shfl_xor(sm, 32);
+        const float mn = fmaxf(mx, mo);
+        if (mn != -INFINITY) sm = sm * fast_exp2(mx - mn) + so * fast_exp2(mo - mn);
+        if (hh == 0) {
+          red_m[wm][nl] = mn;
+          red_s[wm][nl] = sm;
+        }
       }
-    }
+    };
+    if (m0 + WM * WR <= g.M)
+      partial(std::true_type());
+    else
+      partial(std::false_type());
     __syncthreads();
     if (tid < BNT) {
       const int n = n0 + tid;
@@ -254,65 +288,96 @@ __device__ __forceinline__ void gemm_epilogue(const GemmArgs &g, f32x16_t (&acc)
       }
     }
   } else if constexpr (MODE == kDlogits) {
-    static_assert(BNT == 128, "dlogits staging assumes 128 tokens per tile");
-    static_assert((WR * 16) % NT == 0, "staging rows split evenly over the threads");
-    constexpr int TPS = BNT + 8;  // staging row pitch (elements)
-    constexpr int TG = NT / BNT;  // token-row groups per store sweep
+    // Each wave writes its own block, 64 vocab rows at a time, through its own
+    // 64 x 64 staging tile [token][vocab]: a lane's accumulator registers
+    // 4q .. 4q+3 are four vocab rows of one token, one 8-byte LDS write.  dL
+    // leaves as 16-byte row reads (128 bytes a token), dL^T as transposing
+    // reads (16 vocab rows x 32 tokens an instruction).  No barrier, so the
+    // waves and the other workgroup of the CU keep the matrix cores busy.
+    // (One wave row at a time through shared tiles, two barriers each and dL as
+    // single 16-byte pieces of a row per lane: dlogits of n 2999, d 576, V 49152
+    // 394 -> 290 us with PairShape, n 4096, d 2048, V 50304 976 -> 836 with WideShape;
+    // bound by the stores of both layouts, which the K loop hides in part.)
+    static_assert(JN % 2 == 0 && IM % 2 == 0, "dlogits staging takes 64 x 64 blocks");
     float lse2[JN], scale[JN], one[JN];
-    int64_t tj[JN];
+    int rel[JN];
 #pragma unroll
     for (int j = 0; j < JN; ++j) {
       const int n = n0 + WC * wn + 32 * j + l32;
       const bool nvalid = n < g.N;
-      tj[j] = nvalid ? g.targets[n] : g.ignore_index;
-      const bool valid = nvalid && tj[j] != g.ignore_index;
+      const bool valid = nvalid && g.targets[n] != g.ignore_index;
       const float lse = nvalid ? g.lse[n] : 0.f;
       lse2[j] = lse * kLog2e;
       scale[j] = valid ? (*g.grad_out) * (1.0f + 2.0f * g.z * lse) : 0.f;
       one[j] = valid ? (*g.grad_out) : 0.f;
+      rel[j] = target_row(g, n, m0 + WR * wm + 4 * hh, WR);
     }
-    for (int pass = 0; pass < WM; ++pass) {
-      __syncthreads();  // the staging rows are free
-      if (wm == pass) {
+    auto block = [&](int h, int hj, auto Full) {
+      constexpr bool full = decltype(Full)::value;  // the whole tile lies within M x N
+      const int mb = m0 + WR * wm + 64 * h, nb = n0 + WC * wn + 64 * hj;
+      lds_order();  // the reads of the block before stay before these writes
 #pragma unroll
-        for (int j = 0; j < JN; ++j) {
-          const int nl = WC * wn + 32 * j + l32;
-          const bool nvalid = n0 + nl < g.N;
+      for (int j = 0; j < 2; ++j)
 #pragma unroll
-          for (int i = 0; i < IM; ++i)
+        for (int i = 0; i < 2; ++i)
 #pragma unroll
-            for (int r = 0; r < 16; ++r) {
-              const int ml = 32 * i + 8 * (r >> 2) + 4 * hh + (r & 3);
-              const int m = m0 + WR * pass + ml;
-              float gv = fast_exp2(acc[i][j][r] * kLog2e - lse2[j]) * scale[j];
-              if ((int64_t)(g.v0 + m) == tj[j]) gv -= one[j];
-              stage[ml * TPS + nl] = (bf16_t)(m < g.M && nvalid ? gv : 0.f);
+          for (int q = 0; q < 4; ++q) {
+            const int jj = 2 * hj + j;
+            bf16x4_t v;
+#pragma unroll
+            for (int x = 0; x < 4; ++x) {
+              const int mo = 32 * i + 8 * q + x;
+              float gv = fast_exp2(acc[2 * h + i][jj][4 * q + x] * kLog2e - lse2[jj]) * scale[jj];
+              if (!full) gv = mb + 4 * hh + mo < g.M && nb + 32 * j + l32 < g.N ? gv : 0.f;
+              v[x] = (bf16_t)gv;
             }
+            *reinterpret_cast<bf16x4_t *>(&stage[(32 * j + l32) * kDlPitch + 32 * i + 8 * q + 4 * hh]) = v;
+          }
+#pragma unroll
+      for (int j = 0; j < 2; ++j) {
+        const int jj = 2 * hj + j, rl = rel[jj] - 64 * h;
+        const bool here = rl >= 0 && rl < 64 && (rl & 4) == 0;
+        if (__any(here)) {  // few blocks hold the target of one of their tokens
+          float tv = 0.f;
+#pragma unroll
+          for (int i = 0; i < 2; ++i)
+#pragma unroll
+            for (int r = 0; r < 16; ++r)
+              tv = rl == 32 * i + 8 * (r >> 2) + (r & 3) ? acc[2 * h + i][jj][r] : tv;
+          if (here)
+            stage[(32 * j + l32) * kDlPitch + 4 * hh + rl] =
+                (bf16_t)(fast_exp2(tv * kLog2e - lse2[jj]) * scale[jj] - one[jj]);
         }
       }
-      __syncthreads();
-      const int mb = m0 + WR * pass;
-      // dL^T [vocab][tokens]: 16 threads per 256-byte staging row.
+      lds_order();
+      const int tok = lane >> 3, c8 = (lane & 7) * 8;
 #pragma unroll
-      for (int k = 0; k < WR * 16 / NT; ++k) {
-        const int c = tid + NT * k;
-        const int ml = c >> 4, n8 = (c & 15) * 8;
-        if (mb + ml < g.M && n0 + n8 < g.N)
-          *reinterpret_cast<u32x4 *>(g.dlt + (int64_t)(mb + ml) * g.ldlt + n0 + n8) =
-              *reinterpret_cast<const u32x4 *>(&stage[ml * TPS + n8]);
+      for (int k = 0; k < 8; ++k)
+        if (full || (nb + tok + 8 * k < g.N && mb + c8 < g.M))
+          *reinterpret_cast<u32x4 *>(g.dl + (int64_t)(nb + tok + 8 * k) * g.ldl + mb + c8) =
+              *reinterpret_cast<const u32x4 *>(&stage[(tok + 8 * k) * kDlPitch + c8]);
+      const int li = lane & 15, tg = 8 * (lane >> 4);
+#pragma unroll
+      for (int k = 0; k < 8; ++k) {
+        const int t0 = 32 * (k & 1) + tg, mr = 16 * (k >> 1);
+        const bf16_t *src = &stage[(t0 + (li >> 2)) * kDlPitch + mr + 4 * (li & 3)];
+        const i16x4_t lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_i16x4_t *)(src));
+        const i16x4_t hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_i16x4_t *)(src + 4 * kDlPitch));
+        const i16x8_t v = {lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
+        if (full || (mb + mr + li < g.M && nb + t0 < g.N))
+          *reinterpret_cast<i16x8_t *>(g.dlt + (int64_t)(mb + mr + li) * g.ldlt + nb + t0) = v;
       }
-      // dL [tokens][vocab]: lane <-> token, eight vocab rows per 16-byte store.
+    };
+    const bool full = m0 + WM * WR <= g.M && n0 + BNT <= g.N;
 #pragma unroll
-      for (int k = 0; k < WR * 16 / NT; ++k) {
-        const int nl = tid & (BNT - 1), m8 = 8 * ((tid / BNT) + TG * k);
-        if (n0 + nl < g.N && mb + m8 < g.M) {
-          bf16x8_t v;
+    for (int h = 0; h < IM / 2; ++h)
 #pragma unroll
-          for (int x = 0; x < 8; ++x) v[x] = stage[(m8 + x) * TPS + nl];
-          *reinterpret_cast<bf16x8_t *>(g.dl + (int64_t)(n0 + nl) * g.ldl + mb + m8) = v;
-        }
+      for (int hj = 0; hj < JN / 2; ++hj) {
+        if (full)
+          block(h, hj, std::true_type());
+        else
+          block(h, hj, std::false_type());
       }
-    }
   } else {
 #pragma unroll
     for (int i = 0; i < IM; ++i)
@@ -351,14 +416,15 @@ __device__ __forceinline__ void gemm_epilogue(const GemmArgs &g, f32x16_t (&acc)
 // Tile shape of one DMA-kernel instantiation: WM x WN waves of 32*IM x 32*JN
 // outputs, K slices of KW elements (64 or 32: 128- or 64-byte LDS rows in
 // the SwzTile<KW> swizzle), a ring of STAGES slices.
-template <int WM_, int WN_, int IM_, int JN_, int STAGES_, int KW_ = 64>
+template <int WM_, int WN_, int IM_, int JN_, int STAGES_, int KW_ = 64, int WPS_ = 1>
 struct DmaShape {
   static constexpr int WM = WM_, WN = WN_, IM = IM_, JN = JN_, STAGES = STAGES_, KW = KW_;
+  static constexpr int WPS = WPS_;  // waves per SIMD that the registers must allow
   static constexpr int NT = 64 * WM * WN, BMT = 32 * IM * WM, BNT = 32 * JN * WN;
 };
 
-template <int MODE, class SH>
-__global__ __launch_bounds__(SH::NT) void gemm_nt_dma(GemmArgs g) {
+template <int MODE, class SH, bool TAIL = false>
+__global__ __launch_bounds__(SH::NT, SH::WPS) void gemm_nt_dma(GemmArgs g) {
   constexpr int WM = SH::WM, WN = SH::WN, IM = SH::IM, JN = SH::JN, STAGES = SH::STAGES;
   constexpr int KW = SH::KW, KB = 2 * KW, KS = KW / 16;  // slice width, row bytes, K steps
   constexpr int NT = SH::NT, BMT = SH::BMT, BNT = SH::BNT, W = NT / 64;
@@ -369,7 +435,7 @@ __global__ __launch_bounds__(SH::NT) void gemm_nt_dma(GemmArgs g) {
   static_assert(KW == 64 || KW == 32, "slice width");
   static_assert(NA * 16 * NT == AB && NB * 16 * NT == BNT * KB, "stage / thread mismatch");
   static_assert(STAGES >= 2 && STAGES <= 4, "ring of 2 to 4 slices");
-  static_assert(MODE != kDlogits || WR * (BNT + 8) * 2 <= SB, "dlogits staging must fit a stage");
+  static_assert(MODE != kDlogits || W <= STAGES * (SB / kDlStage), "dlogits staging must fit the stages");
   static_assert(MODE != kLse || 32 * (BNT + 8) * 2 <= SB, "logits staging must fit a stage");
   // Stages are separate LDS objects, so the compiler does not wait for the
   // DMA into one before reading another.
@@ -391,7 +457,7 @@ __global__ __launch_bounds__(SH::NT) void gemm_nt_dma(GemmArgs g) {
   const int m0 = tm * BMT, n0 = tn * BNT;
   const int kb = MODE == kAccum && g.part ? blockIdx.y * g.k_per_split : 0;
   const int ke = MODE == kAccum && g.part ? min(g.K, kb + g.k_per_split) : g.K;
-  const int nk = (ke - kb) / KW;  // >= 1, checked by the host
+  const int nk = TAIL ? (ke - kb + KW - 1) / KW : (ke - kb) / KW;  // >= 1, checked by the host
 
   // DMA: chunk p of a stage <- row r, 16-byte chunk c of the K-slice.
   uint32_t aoff[NA], boff[NB];
@@ -414,13 +480,27 @@ __global__ __launch_bounds__(SH::NT) void gemm_nt_dma(GemmArgs g) {
   const int64_t blim = ((int64_t)(g.N - 1 - n0) * g.ldb + (ke - kb)) * 2;
   // Slices past the last reload the last one into a slot nobody reads again,
   // so every step waits for the same DMA count.
-  auto dma = [&](int t, char *dst) {
+  // TAIL: the last slice's chunks from column K on are read as zeros.  A lane's
+  // chunk column is the same in all its DMAs (they lie whole swizzle periods apart).
+  bool past = false;
+  if constexpr (TAIL) {
+    static_assert(W % 4 == 0, "a lane's chunk column does not depend on the DMA");
+    int r, c;
+    SwzTile<KW>::at(wave * 64 + lane, r, c);
+    past = (nk - 1) * KW + c * 8 >= ke - kb;
+  }
+  auto dma1 = [&](int t, char *dst, int x) {
     const int64_t ko = (int64_t)(t < nk ? t : nk - 1) * KB;
+    const bool zero = TAIL && t >= nk - 1 && past;
+    if (x < NA)
+      dma16(abase + ko, alim - ko, zero ? kDmaZero : aoff[x], dst + (x * W + wave) * 1024);
+    else
+      dma16(bbase + ko, blim - ko, zero ? kDmaZero : boff[x - NA],
+            dst + AB + ((x - NA) * W + wave) * 1024);
+  };
+  auto dma = [&](int t, char *dst) {
 #pragma unroll
-    for (int i = 0; i < NA; ++i) dma16(abase + ko, alim - ko, aoff[i], dst + (i * W + wave) * 1024);
-#pragma unroll
-    for (int i = 0; i < NB; ++i)
-      dma16(bbase + ko, blim - ko, boff[i], dst + AB + (i * W + wave) * 1024);
+    for (int x = 0; x < NA + NB; ++x) dma1(t, dst, x);
   };
   // Fragment offsets: rows WR*wm + 32i + l32 of A, WC*wn + 32j + l32 of B,
   // 16-byte chunk 2ks + hh.  The swizzle depends on the row only through
@@ -457,54 +537,75 @@ __global__ __launch_bounds__(SH::NT) void gemm_nt_dma(GemmArgs g) {
       }
   };
 
-  // Fragments are double-buffered across the slice's K steps: step ks+1's
-  // LDS reads are in flight while step ks's MFMAs issue.
-  auto compute = [&](const char *sb) {
-    bf16x8_t a[2][IM], b[2][JN];
-    auto load = [&](int ks, int buf) {
-#pragma unroll
-      for (int i = 0; i < IM; ++i)
-        a[buf][i] = *reinterpret_cast<const bf16x8_t *>(sb + aof[ks] + RB32 * i);
-#pragma unroll
-      for (int j = 0; j < JN; ++j)
-        b[buf][j] = *reinterpret_cast<const bf16x8_t *>(sb + bof[ks] + RB32 * j);
-    };
-    load(0, 0);
-#pragma unroll
-    for (int ks = 0; ks < KS; ++ks) {
-      // sched_barrier keeps the scheduler from sinking the reads back
-      // behind the MFMAs (it would reuse one fragment buffer otherwise).
-      __builtin_amdgcn_sched_barrier(0);
-      if (ks + 1 < KS) load(ks + 1, (ks + 1) & 1);
-      __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-      for (int i = 0; i < IM; ++i)
-#pragma unroll
-        for (int j = 0; j < JN; ++j)
-          acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[ks & 1][i], b[ks & 1][j],
-                                                               acc[i][j], 0, 0, 0);
-    }
-    __builtin_amdgcn_sched_barrier(0);
+  // Fragments are double-buffered across the K steps, also from one slice to
+  // the next: a K step's reads are issued one by one between the MFMAs of the
+  // step before it.  The slice's one barrier therefore stands before its LAST
+  // K step, whose fragments have arrived by then (lgkmcnt(0)): behind it the
+  // next slice is visible, this one's slot is free for the slice STAGES ahead,
+  // and the waves go on with MFMAs whose operands they hold while the reads of
+  // the next slice and the DMA of the one STAGES ahead go out between them.
+  // (With the barrier between slices and a K step's reads in one burst, the
+  // matrix cores waited for both waves' first reads: lse at n 16384, d 4096,
+  // V 128256 15.2 -> 13.8 ms, 1250 TFLOP/s, the rate of a large bf16 product.)
+  bf16x8_t a[2][IM], b[2][JN];
+  // Fragment x of a K step, in the order the MFMAs need them: a0, b0 .. , a1 ..
+  auto load1 = [&](const char *sb, int ks, int buf, int x) {
+    const int i = x == 0 ? 0 : x <= JN ? -1 : x - JN;
+    if (i >= 0)
+      a[buf][i] = *reinterpret_cast<const bf16x8_t *>(sb + aof[ks] + RB32 * i);
+    else
+      b[buf][x - 1] = *reinterpret_cast<const bf16x8_t *>(sb + bof[ks] + RB32 * (x - 1));
   };
-  // One step: slice kt (in slot kt % STAGES) has landed for this thread, the
-  // barrier makes it visible and frees slot (kt - 1) % STAGES, which takes
-  // slice kt + STAGES - 1.
+  static_assert(KS % 2 == 0, "K step 0 of every slice is in fragment buffer 0");
   auto step = [&](int kt, auto Ic) {
     constexpr int I = decltype(Ic)::value;
-    wait_vmcnt<(STAGES - 2) * (NA + NB)>();
-    block_sync_nofence();
-    dma(kt + STAGES - 1, slot(std::integral_constant<int, I + STAGES - 1>()));
-    compute(slot(Ic));
+    using INext = std::integral_constant<int, I + 1>;
+    constexpr int NM = IM * JN, NR = IM + JN;
+#pragma unroll
+    for (int ks = 0; ks < KS; ++ks) {
+      const bool last = ks + 1 == KS;
+      const int na = last ? NR + NA + NB : NR;  // accesses issued with this K step's MFMAs
+      if (last) {
+        __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0): this slice is read
+        wait_vmcnt<(STAGES - 2) * (NA + NB)>();
+        block_sync_nofence();
+      }
+#pragma unroll
+      for (int t = 0; t < NM; ++t) {
+        // sched_barrier keeps the scheduler from sinking the reads back
+        // behind the MFMAs (it would reuse one fragment buffer otherwise).
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int x = t * na / NM; x < (t + 1) * na / NM; ++x) {
+          if (x >= NR)
+            dma1(kt + STAGES, slot(Ic), x - NR);
+          else if (last)
+            load1(slot(INext()), 0, 0, x);
+          else
+            load1(slot(Ic), ks + 1, (ks + 1) & 1, x);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+        const int i = t / JN, j = t % JN;
+        acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[ks & 1][i], b[ks & 1][j], acc[i][j],
+                                                             0, 0, 0);
+      }
+    }
+    __builtin_amdgcn_sched_barrier(0);
   };
   using I0 = std::integral_constant<int, 0>;
   using I1 = std::integral_constant<int, 1>;
   using I2 = std::integral_constant<int, 2>;
   using I3 = std::integral_constant<int, 3>;
   dma(0, st0);
-  if constexpr (STAGES > 2) dma(1, st1);
-  if constexpr (STAGES > 3) dma(2, st2);
+  dma(1, st1);
+  if constexpr (STAGES > 2) dma(2, st2);
+  if constexpr (STAGES > 3) dma(3, st3);
   if constexpr (MODE == kAccum)
     if (preload) preload_acc();
+  wait_vmcnt<(STAGES - 1) * (NA + NB)>();
+  block_sync_nofence();
+#pragma unroll
+  for (int x = 0; x < IM + JN; ++x) load1(st0, 0, 0, x);
   int kt = 0;
   for (; kt + STAGES <= nk; kt += STAGES) {
     step(kt, I0());
@@ -519,7 +620,13 @@ __global__ __launch_bounds__(SH::NT) void gemm_nt_dma(GemmArgs g) {
     if (kt + 2 < nk) step(kt + 2, I2());
   wait_vmcnt<0>();
   __syncthreads();  // every wave is done with the stages (kDlogits / kLse stage in st0)
-  gemm_epilogue<MODE, WM, WN, IM, JN>(g, acc, tm, m0, n0, reinterpret_cast<bf16_t *>(st0), red_m,
+  char *stage = st0;
+  if constexpr (MODE == kDlogits) {
+    constexpr int WPT = SB / kDlStage;  // waves staged per slot
+    const int sl = wave / WPT;
+    stage = (sl == 0 ? st0 : sl == 1 ? st1 : STAGES > 2 && sl == 2 ? st2 : st3) + wave % WPT * kDlStage;
+  }
+  gemm_epilogue<MODE, WM, WN, IM, JN>(g, acc, tm, m0, n0, reinterpret_cast<bf16_t *>(stage), red_m,
                                       red_s, preload);
 }
 
@@ -595,7 +702,10 @@ __global__ __launch_bounds__(256) void gemm_nt(GemmArgs g) {
     }
   }
 
-  gemm_epilogue<MODE, 2, 2, 2, 2>(g, acc, tm, m0, n0, smem, red_m, red_s);
+  if (MODE == kDlogits) __syncthreads();  // every wave is done with the tiles
+  static_assert(sizeof(smem) >= 4 * kDlStage, "dlogits staging");
+  gemm_epilogue<MODE, 2, 2, 2, 2>(
+      g, acc, tm, m0, n0, MODE == kDlogits ? smem + wave * (kDlStage / 2) : smem, red_m, red_s);
 }
 
 // out (+)= sum of the split-K partials (the kAccum epilogue, applied after a
@@ -835,26 +945,47 @@ __global__ __launch_bounds__(256) void pack_bf16(const T *__restrict__ src, int6
 
 unsigned tiles(int m, int n) { return (unsigned)(((m + BM - 1) / BM) * ((n + BN - 1) / BN)); }
 
-// Tile shape of the DMA kernel: 256 x 128 on 8 waves (two per SIMD), a
-// three-slice ring of 48 KiB slices.  Smaller tiles need more bytes per flop
-// and a 2-slice ring does not cover the operand latency (measured slower).
+// Tile shapes of the DMA kernel.  A K step's LDS reads and DMA writes take, per
+// MFMA cycle of a SIMD, RowShape 1.4, PairShape 1.1, WideShape 1.0 cycles of
+// the CU's LDS: the larger the wave's block, the fewer.
+// RowShape: 256 x 128 tiles on 8 waves of 64 x 64 (two per SIMD), a three-slice
+// ring of 48 KiB slices.  The dx / dW products, and the lse product while one
+// workgroup per CU covers the grid (n 256, d 768, V 32000: 26.1 us, PairShape
+// 27.6).
 using RowShape = DmaShape<4, 2, 2, 2, 3>;
-// 256 x 256 tiles on 8 waves of 128 x 64 (6 fragment reads per 8 MFMAs
-// instead of 4 per 4, half the operand bytes per flop), 32-wide K slices in
-// a four-slice ring of 32 KiB.  Used for the forward (lse) product when the
-// grid still has >= 1024 tiles (four per CU): cfg4 16.1 -> 15.6 ms.  The
-// backward products measured slower on it (dx and dW 51.8 -> 52.8 ms for
-// the chunk loop), and dlogits' staging takes 128 tokens, so they keep
-// RowShape.
+// WideShape: 256 x 256 tiles on 8 waves of 128 x 64 (half the operand bytes per
+// flop), 32-wide K slices in a four-slice ring of 32 KiB.
 using WideShape = DmaShape<2, 4, 4, 2, 4, 32>;
+// PairShape: 256 x 128 tiles on 4 waves of 128 x 64 with 72 KiB of slices, two
+// workgroups per CU: one's epilogue runs beside the other's K loop, and the
+// grid has twice WideShape's tiles.
+using PairShape = DmaShape<2, 2, 4, 2, 3, 32, 2>;
 template <class SH> unsigned dma_tiles(int m, int n) {
   return (unsigned)(((m + SH::BMT - 1) / SH::BMT) * ((n + SH::BNT - 1) / SH::BNT));
 }
-// The DMA kernel takes K-slices of whole 64-element blocks (operands are
-// already 16-byte aligned with row strides % 8 == 0).
-bool dma_ok(int64_t k) { return k > 0 && k % 64 == 0; }
-bool wide_ok(int64_t m, int64_t n, int64_t k) {
-  return dma_ok(k) && dma_tiles<WideShape>((int)m, (int)n) >= 1024;
+// A tile's rows lie within the 2 GiB of a DMA's byte offset.
+bool dma_rows(const GemmArgs &g) { return g.lda <= (1 << 22) && g.ldb <= (1 << 22); }
+// RowShape takes K in whole 64-element slices.
+bool dma_ok(const GemmArgs &g) { return g.K % 64 == 0 && dma_rows(g); }
+// WideShape for the logits products from K = `least` on, when its tiles give
+// every CU one: below, the epilogue weighs as much as the K loop.  Measured with
+// V 50304, WideShape / PairShape: lse at n 8192, d 128 220 / 195 us; n 2999,
+// d 576, V 49152 185 / 191; n 8192, d 768 604 / 658; n 4096, d 2048 723 / 810.
+// dlogits, whose stores add to the epilogue: n 8192, d 768 1006 / 948 us; n 4096,
+// d 1024 512 / 534; d 2048 839 / 940.
+constexpr int kWideLse = 512, kWideDlogits = 1024;
+bool wide_ok(const GemmArgs &g, int least) {
+  return g.K >= least && dma_tiles<WideShape>(g.M, g.N) > 256;
+}
+template <int MODE, class SH> void launch_dma(const GemmArgs &g, int splits, hipStream_t st) {
+  const dim3 grid(dma_tiles<SH>(g.M, g.N), (unsigned)splits), block(SH::NT);
+  if constexpr (SH::KW == 32) {
+    if (g.K % 32 != 0) {
+      hipLaunchKernelGGL((gemm_nt_dma<MODE, SH, true>), grid, block, 0, st, g);
+      return;
+    }
+  }
+  hipLaunchKernelGGL((gemm_nt_dma<MODE, SH>), grid, block, 0, st, g);
 }
 
 }  // namespace ce
@@ -928,15 +1059,15 @@ int lmhead_fwd(const void *x, int64_t ldx, const void *w, int64_t ldw, int64_t n
     hipLaunchKernelGGL(sum_rows, dim3(1), dim3(1024), 0, st, (const float *)nullptr, 0, loss_sum);
     return launch_status("pb_lmhead_ce_fwd(empty)");
   }
-  const bool dma = dma_ok(d), wide = wide_ok(v, n, d);
-  const int bm = wide ? WideShape::BMT : dma ? RowShape::BMT : BM;  // lse partials per token
-  const int nmt = (int)((v + bm - 1) / bm);
-  float *ws = static_cast<float *>(workspace);
+  static_assert(RowShape::BMT == WideShape::BMT && PairShape::BMT == WideShape::BMT, "lse partials");
   GemmArgs g = {};
-  g.A = static_cast<const bf16_t *>(w);
   g.lda = ldw;
-  g.B = static_cast<const bf16_t *>(x);
   g.ldb = ldx;
+  const int bm = dma_rows(g) ? WideShape::BMT : BM;
+  const int nmt = (int)((v + bm - 1) / bm);  // lse partials per token
+  float *ws = static_cast<float *>(workspace);
+  g.A = static_cast<const bf16_t *>(w);
+  g.B = static_cast<const bf16_t *>(x);
   g.M = (int)v; g.N = (int)n; g.K = (int)d;
   g.v0 = 0; g.V = (int)v;
   g.targets = targets;
@@ -948,14 +1079,14 @@ int lmhead_fwd(const void *x, int64_t ldx, const void *w, int64_t ldw, int64_t n
   g.lgt = logits;
   g.ldlg = ldlg;
   g.round_bf16 = round_bf16;
-  if (wide)
-    hipLaunchKernelGGL((gemm_nt_dma<kLse, WideShape>), dim3(dma_tiles<WideShape>(g.M, g.N)),
-                       dim3(WideShape::NT), 0, st, g);
-  else if (dma)
-    hipLaunchKernelGGL((gemm_nt_dma<kLse, RowShape>), dim3(dma_tiles<RowShape>(g.M, g.N)),
-                       dim3(RowShape::NT), 0, st, g);
-  else
+  if (!dma_rows(g))
     hipLaunchKernelGGL(gemm_nt<kLse>, dim3(tiles(g.M, g.N)), dim3(256), 0, st, g);
+  else if (wide_ok(g, kWideLse))
+    launch_dma<kLse, WideShape>(g, 1, st);
+  else if (dma_ok(g) && dma_tiles<RowShape>(g.M, g.N) <= 256)
+    launch_dma<kLse, RowShape>(g, 1, st);
+  else
+    launch_dma<kLse, PairShape>(g, 1, st);
   int rc = launch_status("pb_lmhead_ce_fwd(gemm)");
   if (rc) return rc;
   hipLaunchKernelGGL(lse_combine, dim3((unsigned)((n + 63) / 64)), dim3(1024), 0, st, g.part_m,
@@ -1089,11 +1220,12 @@ int dlogits_chunk(const void *x, int64_t ldx, const void *w, int64_t ldw, int64_
   g.ldl = ldl;
   g.ldlt = ldlt;
   g.round_bf16 = round_bf16;
-  if (dma_ok(d))
-    hipLaunchKernelGGL((gemm_nt_dma<kDlogits, RowShape>), dim3(dma_tiles<RowShape>(g.M, g.N)),
-                       dim3(RowShape::NT), 0, st, g);
-  else
+  if (!dma_rows(g))
     hipLaunchKernelGGL(gemm_nt<kDlogits>, dim3(tiles(g.M, g.N)), dim3(256), 0, st, g);
+  else if (wide_ok(g, kWideDlogits))
+    launch_dma<kDlogits, WideShape>(g, 1, st);
+  else
+    launch_dma<kDlogits, PairShape>(g, 1, st);
   return launch_status("pb_lmhead_ce(dlogits)");
 }
 
@@ -1152,9 +1284,8 @@ int lmhead_bwd(const void *x, int64_t ldx, const void *w, int64_t ldw, const voi
     gx.part = part;
     gx.k_per_split = L.k_per_split;
     const int splits = part ? (vc + L.k_per_split - 1) / L.k_per_split : 1;
-    if (dma_ok(vc))
-      hipLaunchKernelGGL((gemm_nt_dma<kAccum, RowShape>), dim3(dma_tiles<RowShape>(gx.M, gx.N), splits),
-                         dim3(RowShape::NT), 0, st, gx);
+    if (dma_ok(gx))
+      launch_dma<kAccum, RowShape>(gx, splits, st);
     else
       hipLaunchKernelGGL(gemm_nt<kAccum>, dim3(tiles(gx.M, gx.N), splits), dim3(256), 0, st, gx);
     if (part) {
@@ -1173,9 +1304,8 @@ int lmhead_bwd(const void *x, int64_t ldx, const void *w, int64_t ldw, const voi
     gw.ldo = lddw;
     gw.out_dtype = dw_dtype;
     gw.accum_out = dw_accumulate != 0;
-    if (dma_ok(n))
-      hipLaunchKernelGGL((gemm_nt_dma<kStore, RowShape>), dim3(dma_tiles<RowShape>(gw.M, gw.N)),
-                         dim3(RowShape::NT), 0, st, gw);
+    if (dma_ok(gw))
+      launch_dma<kStore, RowShape>(gw, 1, st);
     else
       hipLaunchKernelGGL(gemm_nt<kStore>, dim3(tiles(gw.M, gw.N)), dim3(256), 0, st, gw);
     rc = launch_status("pb_lmhead_ce_bwd(dx/dw)");

@@ -102,6 +102,26 @@ _CE_PARAMS = [pytest.param(*c, stored, id=f"{i}-{'stored' if stored else 'recomp
               if not (stored and c[3] == torch.float32 and c[4] == torch.float32)]
 
 
+# (n, v, d, row stride of x and W): the logits products' tile shapes (256 x 256 tiles from
+# d 512 / 1024 on and > 256 of them, else 256 x 128), d of whole 32-wide K slices or not, and
+# rows too far apart for the DMA offsets.  Each output is the same product and softmax as
+# test_fused_ce_matches_oracle's, at its tolerances.
+@pytest.mark.parametrize("n,v,d,ld", [
+    (1030, 16500, 520, 544), (1030, 16500, 1024, 1024), (1030, 16500, 1032, 1056),
+    (300, 517, 40, 64), (129, 1000, 8, 32), (260, 1032, 1000, 1000), (300, 12000, 512, 512),
+    (5, 300, 64, (1 << 22) + 8)])
+def test_logits_tile_shapes_match_oracle(n, v, d, ld, dev) -> None:
+    g = torch.Generator().manual_seed(v + d)
+    xb = torch.full((n, ld), float("nan"), dtype=torch.bfloat16, device=dev)
+    wb = torch.full((v, min(ld, d + 32)), float("nan"), dtype=torch.bfloat16, device=dev)
+    xb[:, :d] = torch.randn(n, d, generator=g).to(dev)
+    wb[:, :d] = (torch.randn(v, d, generator=g) * (0.05 if d >= 256 else 1.0)).to(dev)
+    t = torch.randint(0, v, (n,), generator=g)
+    t[::7] = -100
+    t[1], t[-1] = 0, v - 1
+    _check(xb[:, :d], wb[:, :d], t.to(dev), 0.01, f"n {n} v {v} d {d}")
+
+
 @pytest.mark.parametrize("shape,v,d,xdt,wdt,z,stored", _CE_PARAMS)
 def test_fused_ce_matches_oracle(shape, v, d, xdt, wdt, z, stored, dev) -> None:
     x, w, t = _case(shape, v, d, xdt, wdt, dev, seed=v + d, wstd=0.05 if d >= 256 else 1.0,
