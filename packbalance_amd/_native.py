@@ -43,9 +43,10 @@ class BHSD(C.Structure):
 
     @classmethod
     def of(cls, t: torch.Tensor) -> "BHSD":
-        if t.dim() != 4 or t.stride(-1) != 1:
+        st = t.stride()
+        if len(st) != 4 or st[3] != 1:
             raise ValueError("expected a [B, H, S, D] tensor with unit stride on D")
-        return cls(t.data_ptr(), t.stride(0), t.stride(1), t.stride(2))
+        return cls(t.data_ptr(), st[0], st[1], st[2])
 
 
 _pv = C.POINTER(BHSD)
@@ -213,7 +214,9 @@ def check(status: int, what: str) -> None:
 
 
 def call(name: str, *args) -> None:
-    check(getattr(lib(), name)(*args), name)
+    status = getattr(_lib or lib(), name)(*args)
+    if status != PB_OK:
+        check(status, name)
 
 
 def dtype_code(t: torch.Tensor) -> int:
@@ -235,7 +238,9 @@ def require_device(*tensors: torch.Tensor, op: str) -> None:
 
 
 def stream_ptr(t: torch.Tensor) -> int:
-    return torch.cuda.current_stream(t.device).cuda_stream
+    """The current stream of t's device (its handle, without a Stream object: that costs
+    4 us of a call's host time)."""
+    return torch._C._cuda_getCurrentRawStream(t.device.index)
 
 
 def ptr(t: torch.Tensor | None) -> int | None:

@@ -214,7 +214,7 @@ class _DocAttention(torch.autograd.Function):
         B, Hq, S, D = q.shape
         Hkv = k.shape[1]
         if out_mem is None:
-            out_mem = torch.empty((B, S, Hq, D), dtype=q.dtype, device=q.device)
+            out_mem = q.new_empty((B, S, Hq, D))
         out = out_mem.transpose(1, 2)
         lse = torch.empty((B, Hq, S), dtype=torch.float32, device=q.device)
         p = plans[FWD]
@@ -238,12 +238,12 @@ class _DocAttention(torch.autograd.Function):
         g = dout.to(torch.bfloat16)
         if g.stride(-1) != 1:
             g = g.contiguous()
-        dq = torch.empty((B, S, Hq, D), dtype=q.dtype, device=q.device).transpose(1, 2)
-        dk = torch.empty((B, S, Hkv, D), dtype=k.dtype, device=k.device).transpose(1, 2)
+        dq = q.new_empty((B, S, Hq, D)).transpose(1, 2)
+        dk = k.new_empty((B, S, Hkv, D)).transpose(1, 2)
         if ctx.dv_mem is not None:  # the caller's [B, S, Hkv, D] view (e.g. a gradient slot)
             dv = ctx.dv_mem.transpose(1, 2)
         else:
-            dv = torch.empty((B, S, Hkv, D), dtype=v.dtype, device=v.device).transpose(1, 2)
+            dv = v.new_empty((B, S, Hkv, D)).transpose(1, 2)
         ws = torch.empty(ctx.plans["workspace"], dtype=torch.uint8, device=q.device)
         pq, pkv = ctx.plans[BWD_Q], ctx.plans[BWD_KV]
         N.call("pb_attn_bwd", N.BHSD.of(q), N.BHSD.of(k), N.BHSD.of(v), N.BHSD.of(out),
@@ -261,7 +261,7 @@ class _DocAttentionF32(torch.autograd.Function):
     def forward(ctx, q, k, v, doc, scale):
         B, Hq, S, D = q.shape
         Hkv = k.shape[1]
-        out = torch.empty((B, S, Hq, D), dtype=torch.float32, device=q.device).transpose(1, 2)
+        out = q.new_empty((B, S, Hq, D)).transpose(1, 2)
         lse = torch.empty((B, Hq, S), dtype=torch.float32, device=q.device)
         N.call("pb_attn_fwd_f32", N.BHSD.of(q), N.BHSD.of(k), N.BHSD.of(v), N.BHSD.of(out),
                lse.data_ptr(), doc.data_ptr(), doc.stride(0), B, Hq, Hkv, S, D, float(scale),
@@ -276,9 +276,9 @@ class _DocAttentionF32(torch.autograd.Function):
         B, Hq, S, D = q.shape
         Hkv = k.shape[1]
         g = _bhsd(dout.to(torch.float32))
-        dq = torch.empty((B, S, Hq, D), dtype=torch.float32, device=q.device).transpose(1, 2)
-        dk = torch.empty((B, S, Hkv, D), dtype=torch.float32, device=q.device).transpose(1, 2)
-        dv = torch.empty((B, S, Hkv, D), dtype=torch.float32, device=q.device).transpose(1, 2)
+        dq = q.new_empty((B, S, Hq, D)).transpose(1, 2)
+        dk = k.new_empty((B, S, Hkv, D)).transpose(1, 2)
+        dv = v.new_empty((B, S, Hkv, D)).transpose(1, 2)
         ws = torch.empty(N.lib().pb_attn_bwd_f32_workspace_bytes(B, Hq, Hkv, S, D),
                          dtype=torch.uint8, device=q.device)
         N.call("pb_attn_bwd_f32", N.BHSD.of(q), N.BHSD.of(k), N.BHSD.of(v), N.BHSD.of(out),
