@@ -326,6 +326,21 @@ int pb_lmhead_ce_dlogits(const void *x, int64_t ldx, const void *w, int64_t ldw,
                          int64_t v0, int64_t vc, void *dl, int64_t ldl, void *dlt, int64_t ldlt,
                          int logits_dtype, const void *logits, int64_t ldlg, void *stream);
 
+/* The dx product of one vocab chunk on this library's split-K GEMM (the step
+ * of pb_lmhead_ce_bwd after pb_lmhead_ce_dlogits), for the shapes where the
+ * caller's GEMM library is slower:
+ *   acc (fp32 [n][d], contiguous) = or, without `first`, += dL [n][k] wt [d][k]^T;
+ *   with dx != NULL the sum is rounded to dx_dtype instead and acc only read
+ *   (not at all with `first`, and it may then be NULL).
+ * bf16 operands, 16-byte aligned with row strides % 8 == 0; the columns from
+ * k up to the next multiple of 8 are read and must be zero in both (as
+ * pb_lmhead_ce_dlogits and pb_pack_bf16 write them).  The workspace is 16-byte
+ * aligned, and may be NULL where its size is 0.                             */
+int64_t pb_lmhead_ce_dx_workspace_bytes(int64_t n, int64_t d, int64_t k);
+int pb_lmhead_ce_dx(const void *dl, int64_t ldl, const void *wt, int64_t ldwt, int64_t n,
+                    int64_t d, int64_t k, void *workspace, float *acc, int first, void *dx,
+                    int dx_dtype, int64_t lddx, void *stream);
+
 /* ---- Fused residual add + RMSNorm (per-operand dtypes) ------------------
  * Replaces the decoder's `hidden = hidden + sublayer_out` followed by the
  * next rmsnorm (packbalance/model/llama.py:122-125 with

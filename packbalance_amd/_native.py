@@ -123,6 +123,10 @@ SIGNATURES: dict[str, tuple] = {
         [_p, _i64, _p, _i64, _i64, _i64, _i64, _p, _i64, _f32, _p, _p, _i64, _i64, _p, _i64, _p,
          _i64, _i32, _p, _i64, _p],
     ),
+    "pb_lmhead_ce_dx_workspace_bytes": (_i64, [_i64, _i64, _i64]),
+    "pb_lmhead_ce_dx": (
+        _i32, [_p, _i64, _p, _i64, _i64, _i64, _i64, _p, _p, _i32, _p, _i32, _i64, _p],
+    ),
     "pb_pack_bf16": (_i32, [_p, _i32, _i64, _i64, _i64, _p, _i64, _i64, _i64, _i32, _p]),
     "pb_add_rmsnorm_fwd": (
         _i32,

@@ -11,8 +11,8 @@
 // (both operands K-contiguous, "NT"), with four epilogues.  gemm_nt_dma reads
 // LDS-DMA rings of swizzled K slices in one of three tile shapes; gemm_nt
 // (128 x 128 x 64, four waves of 64 x 64, register-staged) takes the dx / dW
-// products whose K is not whole 64-element slices, and rows too far apart for
-// a tile's 2 GiB of DMA offsets.  Epilogues:
+// products whose K is not a multiple of 8, and rows too far apart for a tile's
+// 2 GiB of DMA offsets.  Epilogues:
 //   kLse      A = W, B = x: C = logits^T, lane <-> token.  Per token, a
 //             (max, sum exp) partial over the tile's vocab rows and the
 //             target logit; the [tokens x vocab] tile is discarded, or also
@@ -76,9 +76,9 @@ struct GemmArgs {
   int out_dtype;
   int first, last;
   int accum_out;  // kStore: out is fp32 and the product is added to it
-  // kAccum split-K: blockIdx.y = split; each split covers k_per_split of K and
+  // kAccum split-K: each of `splits` (1 without) covers k_per_split of K and
   // writes fp32 partials part[split][M][N]; split_reduce folds them.
-  int k_per_split;
+  int k_per_split, splits;
   float *part;
 };
 
@@ -135,6 +135,18 @@ __device__ __forceinline__ void tile_of(int id, int ntm, int ntn, int &tm, int &
   tn = local / rows;
 }
 
+// kAccum with few tile columns: (split, tile row) units are dealt to the XCDs and a unit's
+// columns run side by side on one, so its rows of A -- all of the product's HBM traffic but
+// W^T -- are read once.  In tile_of's order each column read them again on another XCD and
+// HBM set the time: dx [4096, 576] over K 49152 368 -> 262 us, [4096, 768] over 32000 262 ->
+// 232 us, and with dx_splits' count [1999, 768] over 32000 180 -> 102 us (967 TFLOP/s).
+// From 9 columns on a unit would be most of an XCD, and B, which every unit reads, the
+// larger operand.
+constexpr int kUnitCols = 8;
+__host__ __device__ __forceinline__ unsigned unit_grid(int units, int ntn) {
+  return (unsigned)((units + 7) / 8 * 8 * ntn);
+}
+
 // Row of token n's target relative to vocab row v0 + m when it is one of the
 // `rows` rows from there (below M) and the token counts, else -1.
 __device__ __forceinline__ int target_row(const GemmArgs &g, int n, int m, int rows) {
@@ -162,7 +174,7 @@ __device__ __forceinline__ void gemm_epilogue(const GemmArgs &g, f32x16_t (&acc)
                                               int m0, int n0, bf16_t *stage,
                                               float (*red_m)[32 * JN * WN],
                                               float (*red_s)[32 * JN * WN],
-                                              bool preloaded = false) {
+                                              bool preloaded = false, int split = 0) {
   constexpr int NT = 64 * WM * WN, BNT = 32 * JN * WN, WR = 32 * IM, WC = 32 * JN;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int hh = lane >> 5, l32 = lane & 31;
@@ -392,7 +404,7 @@ __device__ __forceinline__ void gemm_epilogue(const GemmArgs &g, f32x16_t (&acc)
           float v = acc[i][j][r];
           if constexpr (MODE == kAccum) {
             if (g.part) {
-              g.part[((int64_t)blockIdx.y * g.M + m) * g.N + n] = v;
+              g.part[((int64_t)split * g.M + m) * g.N + n] = v;
               continue;
             }
             float *p = g.acc + (int64_t)m * g.ldc + n;
@@ -452,10 +464,19 @@ __global__ __launch_bounds__(SH::NT, SH::WPS) void gemm_nt_dma(GemmArgs g) {
   const int hh = lane >> 5, l32 = lane & 31;
   const int wm = wave / WN, wn = wave % WN;
   const int ntm = (g.M + BMT - 1) / BMT, ntn = (g.N + BNT - 1) / BNT;
-  int tm, tn;
-  tile_of((int)blockIdx.x, ntm, ntn, tm, tn);
+  int tm, tn, split = 0;
+  if (MODE == kAccum && ntn <= kUnitCols) {
+    const int j = (int)blockIdx.x >> 3, u = j / ntn * 8 + ((int)blockIdx.x & 7);
+    split = u / ntm;
+    tm = u - split * ntm;
+    tn = j % ntn;
+    if (split >= g.splits) return;
+  } else {
+    tile_of((int)blockIdx.x, ntm, ntn, tm, tn);
+    if (MODE == kAccum) split = blockIdx.y;
+  }
   const int m0 = tm * BMT, n0 = tn * BNT;
-  const int kb = MODE == kAccum && g.part ? blockIdx.y * g.k_per_split : 0;
+  const int kb = MODE == kAccum && g.part ? split * g.k_per_split : 0;
   const int ke = MODE == kAccum && g.part ? min(g.K, kb + g.k_per_split) : g.K;
   const int nk = TAIL ? (ke - kb + KW - 1) / KW : (ke - kb) / KW;  // >= 1, checked by the host
 
@@ -627,7 +648,7 @@ __global__ __launch_bounds__(SH::NT, SH::WPS) void gemm_nt_dma(GemmArgs g) {
     stage = (sl == 0 ? st0 : sl == 1 ? st1 : STAGES > 2 && sl == 2 ? st2 : st3) + wave % WPT * kDlStage;
   }
   gemm_epilogue<MODE, WM, WN, IM, JN>(g, acc, tm, m0, n0, reinterpret_cast<bf16_t *>(stage), red_m,
-                                      red_s, preload);
+                                      red_s, preload, split);
 }
 
 template <int MODE>
@@ -705,7 +726,8 @@ __global__ __launch_bounds__(256) void gemm_nt(GemmArgs g) {
   if (MODE == kDlogits) __syncthreads();  // every wave is done with the tiles
   static_assert(sizeof(smem) >= 4 * kDlStage, "dlogits staging");
   gemm_epilogue<MODE, 2, 2, 2, 2>(
-      g, acc, tm, m0, n0, MODE == kDlogits ? smem + wave * (kDlStage / 2) : smem, red_m, red_s);
+      g, acc, tm, m0, n0, MODE == kDlogits ? smem + wave * (kDlStage / 2) : smem, red_m, red_s,
+      false, MODE == kAccum ? (int)blockIdx.y : 0);
 }
 
 // out (+)= sum of the split-K partials (the kAccum epilogue, applied after a
@@ -943,6 +965,40 @@ __global__ __launch_bounds__(256) void pack_bf16(const T *__restrict__ src, int6
   }
 }
 
+// The transpose of pack_bf16 for bf16 rows of whole 16-byte vectors (both
+// matrices): vectors in, and transposing LDS reads (a lane gets eight source
+// rows of one column) give the vectors out, 128 bytes of each destination row.
+// HBM-bound.  [49152, 576] 35 -> 21 us, [128256, 2048] 415 -> 223 us (4.7 TB/s),
+// against one element a lane and LDS access.
+__global__ __launch_bounds__(256) void transpose_bf16(const bf16_t *__restrict__ src, int64_t lds,
+                                                      int rows, int cols, bf16_t *__restrict__ dst,
+                                                      int64_t ldd, int drows, int dcols) {
+  __shared__ __align__(16) bf16_t tile[64 * kDlPitch];
+  const int r0 = blockIdx.y * 64, c0 = blockIdx.x * 64;
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+#pragma unroll
+  for (int p = 0; p < 2; ++p) {
+    const int q = tid + 256 * p, r = q >> 3, c = (q & 7) * 8;
+    u32x4 v = {0u, 0u, 0u, 0u};
+    if (r0 + r < rows && c0 + c < cols)
+      v = *reinterpret_cast<const u32x4 *>(src + (int64_t)(r0 + r) * lds + c0 + c);
+    *reinterpret_cast<u32x4 *>(&tile[r * kDlPitch + c]) = v;
+  }
+  __syncthreads();
+  const int li = lane & 15, tg = 8 * (lane >> 4);
+#pragma unroll
+  for (int p = 0; p < 2; ++p) {
+    const int t0 = 32 * p + tg, mr = 16 * wave;
+    const bf16_t *s = &tile[(t0 + (li >> 2)) * kDlPitch + mr + 4 * (li & 3)];
+    const i16x4_t lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_i16x4_t *)(s));
+    const i16x4_t hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_i16x4_t *)(s + 4 * kDlPitch));
+    const i16x8_t v = {lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
+    const int orow = c0 + mr + li, ocol = r0 + t0;
+    if (orow < drows && ocol < dcols)
+      *reinterpret_cast<i16x8_t *>(dst + (int64_t)orow * ldd + ocol) = v;
+  }
+}
+
 unsigned tiles(int m, int n) { return (unsigned)(((m + BM - 1) / BM) * ((n + BN - 1) / BN)); }
 
 // Tile shapes of the DMA kernel.  A K step's LDS reads and DMA writes take, per
@@ -965,8 +1021,9 @@ template <class SH> unsigned dma_tiles(int m, int n) {
 }
 // A tile's rows lie within the 2 GiB of a DMA's byte offset.
 bool dma_rows(const GemmArgs &g) { return g.lda <= (1 << 22) && g.ldb <= (1 << 22); }
-// RowShape takes K in whole 64-element slices.
-bool dma_ok(const GemmArgs &g) { return g.K % 64 == 0 && dma_rows(g); }
+// The dx / dW products by DMA: whole 16-byte chunks of K (gemm_nt takes the rest; dW of
+// n 3000, d 576, V 49152 408 -> 274 us).
+bool dma_ok(const GemmArgs &g) { return g.K % 8 == 0 && dma_rows(g); }
 // WideShape for the logits products from K = `least` on, when its tiles give
 // every CU one: below, the epilogue weighs as much as the K loop.  Measured with
 // V 50304, WideShape / PairShape: lse at n 8192, d 128 220 / 195 us; n 2999,
@@ -977,15 +1034,17 @@ constexpr int kWideLse = 512, kWideDlogits = 1024;
 bool wide_ok(const GemmArgs &g, int least) {
   return g.K >= least && dma_tiles<WideShape>(g.M, g.N) > 256;
 }
-template <int MODE, class SH> void launch_dma(const GemmArgs &g, int splits, hipStream_t st) {
-  const dim3 grid(dma_tiles<SH>(g.M, g.N), (unsigned)splits), block(SH::NT);
-  if constexpr (SH::KW == 32) {
-    if (g.K % 32 != 0) {
-      hipLaunchKernelGGL((gemm_nt_dma<MODE, SH, true>), grid, block, 0, st, g);
-      return;
-    }
+template <int MODE, class SH> void launch_dma(const GemmArgs &g, hipStream_t st) {
+  dim3 grid(dma_tiles<SH>(g.M, g.N)), block(SH::NT);
+  if constexpr (MODE == kAccum) {
+    const int ntn = (g.N + SH::BNT - 1) / SH::BNT, ntm = (g.M + SH::BMT - 1) / SH::BMT;
+    if (ntn <= kUnitCols) grid.x = unit_grid(ntm * g.splits, ntn);
+    else grid.y = (unsigned)g.splits;
   }
-  hipLaunchKernelGGL((gemm_nt_dma<MODE, SH>), grid, block, 0, st, g);
+  if (g.K % SH::KW != 0)
+    hipLaunchKernelGGL((gemm_nt_dma<MODE, SH, true>), grid, block, 0, st, g);
+  else
+    hipLaunchKernelGGL((gemm_nt_dma<MODE, SH>), grid, block, 0, st, g);
 }
 
 }  // namespace ce
@@ -1015,6 +1074,12 @@ extern "C" int pb_pack_bf16(const void *src, int src_dtype, int64_t src_ld, int6
   const int64_t grid_r = transpose ? dst_cols : dst_rows, grid_c = transpose ? dst_rows : dst_cols;
   dim3 grid((unsigned)((grid_c + 63) / 64), (unsigned)((grid_r + 63) / 64));
   bf16_t *D = static_cast<bf16_t *>(dst);
+  if (transpose && src_dtype == PB_BF16 && k_aligned(src, src_ld) && k_aligned(dst, dst_ld) &&
+      cols % 8 == 0 && dst_cols % 8 == 0) {
+    hipLaunchKernelGGL(ce::transpose_bf16, grid, dim3(256), 0, st, static_cast<const bf16_t *>(src),
+                       src_ld, (int)rows, (int)cols, D, dst_ld, (int)dst_rows, (int)dst_cols);
+    return launch_status("pb_pack_bf16");
+  }
 #define PB_PACK(T)                                                                                  \
   if (transpose)                                                                                    \
     hipLaunchKernelGGL((ce::pack_bf16<T, true>), grid, dim3(256), 0, st, static_cast<const T *>(src), \
@@ -1082,11 +1147,11 @@ int lmhead_fwd(const void *x, int64_t ldx, const void *w, int64_t ldw, int64_t n
   if (!dma_rows(g))
     hipLaunchKernelGGL(gemm_nt<kLse>, dim3(tiles(g.M, g.N)), dim3(256), 0, st, g);
   else if (wide_ok(g, kWideLse))
-    launch_dma<kLse, WideShape>(g, 1, st);
-  else if (dma_ok(g) && dma_tiles<RowShape>(g.M, g.N) <= 256)
-    launch_dma<kLse, RowShape>(g, 1, st);
+    launch_dma<kLse, WideShape>(g, st);
+  else if (g.K % 64 == 0 && dma_tiles<RowShape>(g.M, g.N) <= 256)
+    launch_dma<kLse, RowShape>(g, st);
   else
-    launch_dma<kLse, PairShape>(g, 1, st);
+    launch_dma<kLse, PairShape>(g, st);
   int rc = launch_status("pb_lmhead_ce_fwd(gemm)");
   if (rc) return rc;
   hipLaunchKernelGGL(lse_combine, dim3((unsigned)((n + 63) / 64)), dim3(1024), 0, st, g.part_m,
@@ -1124,6 +1189,9 @@ extern "C" int pb_lmhead_ce_fwd_logits(const void *x, int64_t ldx, const void *w
 }
 
 namespace {
+// Most splits of pb_lmhead_ce_dx: 15 tiles (n 700, d 576) still fill the CUs.
+constexpr int64_t kDxSplits = 16;
+
 // Backward workspace: dL [n][vchunk] bf16, dL^T [vchunk][n8] bf16, the fp32
 // dx accumulator [n][d], the split-K partials [splits][n][d] (256-byte aligned
 // pieces).
@@ -1131,6 +1199,30 @@ struct BwdWs {
   int64_t ldl, ldlt, off_dlt, off_acc, off_part, bytes;
   int splits, k_per_split;
 };
+
+// Splits of the dx GEMM's K (the vocab chunk) when its 256 x 128 tiles cannot
+// fill the GPU: of 1..most splits of at least kmin columns, the one of least
+// estimated time, fewer splits on a tie.  In units of one K column of a tile
+// (13 ns of a CU): each round of 32 workgroups an XCD takes its columns and
+// kFixed (prologue and epilogue), and the partials' way through HBM and
+// split_reduce kMerge per tile and split.
+void dx_splits(int64_t n, int64_t d, int64_t k, int64_t most, int *splits, int *k_per_split) {
+  const int64_t ntm = (n + 255) / 256, ntn = (d + 127) / 128;
+  constexpr int64_t kCus = 32, kmin = 1024, kFixed = 300, kMerge = 1;
+  auto kps = [&](int64_t s) {
+    return ((k + s - 1) / s + pb::ce::BK - 1) / pb::ce::BK * pb::ce::BK;
+  };
+  auto cost = [&](int64_t s) {
+    const int64_t per_xcd =
+        ntn <= pb::ce::kUnitCols ? (ntm * s + 7) / 8 * ntn : (ntm * ntn * s + 7) / 8;
+    return (per_xcd + kCus - 1) / kCus * (kps(s) + kFixed) + (s > 1 ? kMerge * ntm * ntn * s : 0);
+  };
+  int64_t use = 1;
+  for (int64_t s = 2; s <= most && k / s >= kmin; ++s)
+    if (cost(s) < cost(use)) use = s;
+  *splits = (int)use;
+  *k_per_split = (int)kps(use);
+}
 
 BwdWs bwd_ws(int64_t n, int64_t v, int64_t d, int64_t vchunk) {
   auto al = [](int64_t x) { return (x + 255) / 256 * 256; };
@@ -1140,29 +1232,8 @@ BwdWs bwd_ws(int64_t n, int64_t v, int64_t d, int64_t vchunk) {
   w.off_dlt = al(n * vchunk * 2);
   w.off_acc = w.off_dlt + al(vchunk * w.ldlt * 2);
   w.off_part = w.off_acc + al(n * d * 4);
-  // Split the dx GEMM's K (vocab chunk) when its tile grid (counted in the
-  // DMA kernel's 256 x 128 tiles, one workgroup per CU) cannot fill the
-  // GPU: of 1..8 splits of at least kmin columns, the one whose grid takes the
-  // least time as (rounds of 256 workgroups) x (K columns per split), fewer
-  // splits on a tie.  E.g. 96 tiles: 8 splits = 3 full rounds of 4032
-  // columns against 6 splits = 2.25 rounds (a quarter-full third round) of
-  // 5376.
-  const int64_t tiles = ((n + 255) / 256) * ((d + 127) / 128);
-  constexpr int64_t kCus = 256, kmin = 1024;
-  auto kps = [&](int64_t s) {
-    return ((vchunk + s - 1) / s + pb::ce::BK - 1) / pb::ce::BK * pb::ce::BK;
-  };
-  int64_t splits = 1, best = (tiles + kCus - 1) / kCus * kps(1);
-  for (int64_t s = 2; s <= 8 && vchunk / s >= kmin; ++s) {
-    const int64_t cost = (tiles * s + kCus - 1) / kCus * kps(s);
-    if (cost < best) {
-      best = cost;
-      splits = s;
-    }
-  }
-  w.splits = (int)splits;
-  w.k_per_split = (int)kps(splits);
-  w.bytes = w.off_part + (splits > 1 ? al(splits * n * d * 4) : 0);
+  dx_splits(n, d, vchunk, 8, &w.splits, &w.k_per_split);
+  w.bytes = w.off_part + (w.splits > 1 ? al((int64_t)w.splits * n * d * 4) : 0);
   return w;
 }
 }  // namespace
@@ -1223,10 +1294,31 @@ int dlogits_chunk(const void *x, int64_t ldx, const void *w, int64_t ldw, int64_
   if (!dma_rows(g))
     hipLaunchKernelGGL(gemm_nt<kDlogits>, dim3(tiles(g.M, g.N)), dim3(256), 0, st, g);
   else if (wide_ok(g, kWideDlogits))
-    launch_dma<kDlogits, WideShape>(g, 1, st);
+    launch_dma<kDlogits, WideShape>(g, st);
   else
-    launch_dma<kDlogits, PairShape>(g, 1, st);
+    launch_dma<kDlogits, PairShape>(g, st);
   return launch_status("pb_lmhead_ce(dlogits)");
+}
+
+void launch_dx(const pb::ce::GemmArgs &g, hipStream_t st) {
+  using namespace pb::ce;
+  if (dma_ok(g))
+    launch_dma<kAccum, RowShape>(g, st);
+  else
+    hipLaunchKernelGGL(gemm_nt<kAccum>, dim3(tiles(g.M, g.N), g.splits), dim3(256), 0, st, g);
+  if (g.part) {
+    const int64_t cnt = (int64_t)g.M * g.N;
+    hipLaunchKernelGGL(split_reduce, dim3((unsigned)((cnt + 255) / 256)), dim3(256), 0, st, g,
+                       g.splits);
+  }
+}
+
+void launch_dw(const pb::ce::GemmArgs &g, hipStream_t st) {
+  using namespace pb::ce;
+  if (dma_ok(g))
+    launch_dma<kStore, RowShape>(g, st);
+  else
+    hipLaunchKernelGGL(gemm_nt<kStore>, dim3(tiles(g.M, g.N)), dim3(256), 0, st, g);
 }
 
 int lmhead_bwd(const void *x, int64_t ldx, const void *w, int64_t ldw, const void *xt,
@@ -1283,16 +1375,8 @@ int lmhead_bwd(const void *x, int64_t ldx, const void *w, int64_t ldw, const voi
     gx.last = c == nchunks - 1;
     gx.part = part;
     gx.k_per_split = L.k_per_split;
-    const int splits = part ? (vc + L.k_per_split - 1) / L.k_per_split : 1;
-    if (dma_ok(gx))
-      launch_dma<kAccum, RowShape>(gx, splits, st);
-    else
-      hipLaunchKernelGGL(gemm_nt<kAccum>, dim3(tiles(gx.M, gx.N), splits), dim3(256), 0, st, gx);
-    if (part) {
-      const int64_t cnt = (int64_t)gx.M * gx.N;
-      hipLaunchKernelGGL(split_reduce, dim3((unsigned)((cnt + 255) / 256)), dim3(256), 0, st, gx,
-                         splits);
-    }
+    gx.splits = part ? (vc + L.k_per_split - 1) / L.k_per_split : 1;
+    launch_dx(gx, st);
     // 3) dW[v0:v0+vc] = dL^T x: A = dL^T [vc][n], B = x^T rows d.
     GemmArgs gw = {};
     gw.A = dlt;
@@ -1304,10 +1388,7 @@ int lmhead_bwd(const void *x, int64_t ldx, const void *w, int64_t ldw, const voi
     gw.ldo = lddw;
     gw.out_dtype = dw_dtype;
     gw.accum_out = dw_accumulate != 0;
-    if (dma_ok(gw))
-      launch_dma<kStore, RowShape>(gw, 1, st);
-    else
-      hipLaunchKernelGGL(gemm_nt<kStore>, dim3(tiles(gw.M, gw.N)), dim3(256), 0, st, gw);
+    launch_dw(gw, st);
     rc = launch_status("pb_lmhead_ce_bwd(dx/dw)");
     if (rc) return rc;
   }
@@ -1382,4 +1463,50 @@ extern "C" int pb_lmhead_ce_dlogits(const void *x, int64_t ldx, const void *w, i
                        grad_out, v0, (int)vc, static_cast<bf16_t *>(dl), ldl,
                        static_cast<bf16_t *>(dlt), ldlt, logits_dtype == PB_BF16, logits, ldlg,
                        as_stream(stream));
+}
+
+extern "C" int64_t pb_lmhead_ce_dx_workspace_bytes(int64_t n, int64_t d, int64_t k) {
+  if (n <= 0 || d <= 0 || k <= 0) return 0;
+  int splits, kps;
+  dx_splits(n, d, k, kDxSplits, &splits, &kps);
+  return splits > 1 ? (int64_t)splits * n * d * 4 : 0;
+}
+
+extern "C" int pb_lmhead_ce_dx(const void *dl, int64_t ldl, const void *wt, int64_t ldwt, int64_t n,
+                               int64_t d, int64_t k, void *workspace, float *acc, int first,
+                               void *dx, int dx_dtype, int64_t lddx, void *stream) {
+  using namespace pb;
+  using namespace pb::ce;
+  clear_error();
+  PB_CHECK_ARG(n >= 1 && d >= 1 && k >= 1, "pb_lmhead_ce_dx: bad shape");
+  PB_CHECK_SUPPORTED(n < (1LL << 31) && d < (1LL << 31) && k < (1LL << 30),
+                     "pb_lmhead_ce_dx: too large");
+  PB_CHECK_ARG(dl && wt && (dx || acc) && (acc || first), "pb_lmhead_ce_dx: null argument");
+  PB_CHECK_ARG(dx == nullptr || (valid_dtype(dx_dtype) && lddx >= d),
+               "pb_lmhead_ce_dx: bad dx dtype or stride");
+  const int64_t k8 = (k + 7) / 8 * 8;
+  PB_CHECK_ARG(k_aligned(dl, ldl) && k_aligned(wt, ldwt) && ldl >= k8 && ldwt >= k8,
+               "pb_lmhead_ce_dx: operand rows must be 16-byte aligned and hold k rounded up to 8");
+  GemmArgs g = {};
+  g.A = static_cast<const bf16_t *>(dl);
+  g.lda = ldl;
+  g.B = static_cast<const bf16_t *>(wt);
+  g.ldb = ldwt;
+  g.M = (int)n; g.N = (int)d; g.K = (int)k8;
+  g.acc = acc;
+  g.ldc = d;
+  g.out = dx;
+  g.ldo = lddx;
+  g.out_dtype = dx_dtype;
+  g.first = first != 0;
+  g.last = dx != nullptr;
+  dx_splits(n, d, k, kDxSplits, &g.splits, &g.k_per_split);
+  if (g.splits > 1) {
+    PB_CHECK_ARG(k_aligned(workspace, 8) && workspace != nullptr,
+                 "pb_lmhead_ce_dx: a 16-byte aligned workspace is required for this shape");
+    g.part = static_cast<float *>(workspace);
+    g.splits = (int)((k8 + g.k_per_split - 1) / g.k_per_split);
+  }
+  launch_dx(g, as_stream(stream));
+  return launch_status("pb_lmhead_ce_dx");
 }

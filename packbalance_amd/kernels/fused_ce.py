@@ -23,7 +23,8 @@ one dlogits chunk of all tokens under ``CHUNK_BUDGET`` elements -- 1 GiB of
 bf16 per layout -- but at least 8192): the chunk's dlogits (bf16) come from
 one memory-bound pass over the stored logits, or from a GEMM that recomputes
 them (the kernel of ``pb_lmhead_ce_dlogits``), then two plain library GEMMs
-(torch on hipBLASLt) accumulate dx and write the chunk's dW rows; the C
+(torch on hipBLASLt) accumulate dx and write the chunk's dW rows (dx of few
+output tiles runs on this build's GEMM instead, ``own_dx``); the C
 boundary's ``pb_lmhead_ce_bwd`` runs the same steps with this build's own
 GEMMs for C callers, and so does ``linear_cross_entropy_accumulate`` (the
 training step's form, run on two streams at once inside a captured graph).  Fewer, longer chunks mean fewer passes over the fp32 dx
@@ -184,12 +185,23 @@ def _ce_backward(xb, wb, t, lse, go, lg, lg_dtype, n, v, d8, ignore_index, z, vc
     dW_chunk (+)= dL^T x as library GEMMs (torch -> hipBLASLt, fp32 accumulation),
     which run these plain products faster than this build's own DMA GEMM
     (``pb_lmhead_ce_bwd``; at a cfg4 chunk dx 977 vs 1,110 us and dW 809 vs 967 us)
-    and read x and W as they are, with no transposed copies."""
+    and read x and W as they are, with no transposed copies.  dx of few output tiles
+    (``own_dx``) runs on this build's split-K GEMM (``pb_lmhead_ce_dx``), which reads a
+    transposed copy of the chunk's W rows."""
     dev = xb.device
     stream = N.stream_ptr(xb)
     dl = torch.empty((n, vchunk), dtype=torch.bfloat16, device=dev)
     dlt = torch.empty((vchunk, _round8(n)), dtype=torch.bfloat16, device=dev)
-    acc = dx if dx.dtype == torch.float32 else torch.empty((n, d8), dtype=torch.float32,
+    own = own_dx(n, d8)
+    ws = None
+    if own:
+        # the last chunk is shorter and may be split otherwise
+        nbytes = max(N.lib().pb_lmhead_ce_dx_workspace_bytes(n, d8, k)
+                     for k in (min(vchunk, v), v - (v - 1) // vchunk * vchunk))
+        ws = torch.empty(nbytes, dtype=torch.uint8, device=dev) if nbytes else None
+    acc = dx
+    if dx.dtype != torch.float32:
+        acc = None if own and vchunk >= v else torch.empty((n, d8), dtype=torch.float32,
                                                            device=dev)
     for c, v0 in enumerate(range(0, v, vchunk)):
         vc = min(vchunk, v - v0)
@@ -198,9 +210,16 @@ def _ce_backward(xb, wb, t, lse, go, lg, lg_dtype, n, v, d8, ignore_index, z, vc
                dl.data_ptr(), dl.stride(0), dlt.data_ptr(), dlt.stride(0), _lg_code(lg_dtype),
                N.ptr(lg), lg.stride(0) if lg is not None else 0, stream)
         dlc, dltc, dwc = dl[:, :vc], dlt[:vc, :n], dw[v0:v0 + vc]
-        # beta 0 on the first chunk: the accumulator's old contents are not read
-        torch.addmm(acc, dlc, wb[v0:v0 + vc], beta=0 if c == 0 else 1,
-                    out_dtype=torch.float32, out=acc)
+        if own:
+            wt = _transpose_bf16(wb[v0:v0 + vc])
+            last = dx is not acc and v0 + vc == v
+            N.call("pb_lmhead_ce_dx", dl.data_ptr(), dl.stride(0), wt.data_ptr(), wt.stride(0),
+                   n, d8, vc, N.ptr(ws), N.ptr(acc), int(c == 0), dx.data_ptr() if last else None,
+                   N.dtype_code(dx), dx.stride(0), stream)
+        else:
+            # beta 0 on the first chunk: the accumulator's old contents are not read
+            torch.addmm(acc, dlc, wb[v0:v0 + vc], beta=0 if c == 0 else 1,
+                        out_dtype=torch.float32, out=acc)
         if dw_accumulate or dwc.dtype == torch.float32:
             torch.addmm(dwc, dltc, xb, beta=1 if dw_accumulate else 0, out_dtype=torch.float32,
                         out=dwc)
@@ -209,8 +228,20 @@ def _ce_backward(xb, wb, t, lse, go, lg, lg_dtype, n, v, d8, ignore_index, z, vc
         else:  # fp16 weights: the product in fp32, rounded once
             dwc.copy_(torch.addmm(torch.empty((vc, d8), dtype=torch.float32, device=dev), dltc, xb,
                                   beta=0, out_dtype=torch.float32))
-    if acc is not dx:
+    if acc is not dx and not own:
         dx.copy_(acc)
+
+
+def own_dx(n: int, d8: int) -> bool:
+    """True when ``dx = dL W`` of a chunk runs on this build's split-K GEMM: up to 128 of its
+    256 x 128 output tiles (the vocabulary is split to fill the CUs) and at most 8 of them
+    side by side, which share one XCD's reads of dL.  Library product against split-K GEMM
+    and transposed copy of W, in us: d 576, V 49152: n 520 193 / 74, n 2999 370 / 214, n 6001
+    465 / 396; d 768, V 50257: n 2999 443 / 391, n 4096 518 / 487, but n 6001 649 / 685;
+    d 1000, V 32000: n 4096 377 / 283, n 6001 376 / 444.  Wider rows make the copy the larger
+    part: d 2048, V 128256: n 1999 1556 / 1226, n 2999 1324 / 1755; d 4096, V 32000: n 520
+    269 / 320, n 2999 643 / 864."""
+    return d8 <= 1024 and -(-n // 256) * -(-d8 // 128) <= 128
 
 
 def vocab_chunk(n: int, v: int) -> int:

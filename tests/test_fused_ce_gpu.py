@@ -97,6 +97,45 @@ _CE_CASES = [
 ]
 
 # fp32 x and W take the fp32 path, which keeps no kernel logits: recompute only.
+# (n, v, d, vocab rows per chunk): dx products of up to 128 output tiles (this build's split-K
+# GEMM) and of more (the library's); vocabulary chunks that are not whole K slices, split and
+# not, one chunk and several with a last one of other splits.  The same product as
+# test_fused_ce_matches_oracle's, at its tolerances.
+@pytest.mark.parametrize("xdt", [torch.bfloat16, torch.float32], ids=["bf16", "fp32x"])
+@pytest.mark.parametrize("n,v,d,vchunk", [
+    (1, 9, 8, 16), (257, 5000, 72, 5000), (300, 8200, 128, 4096), (700, 2100, 64, 1040),
+    (8192, 517, 512, 520), (8193, 517, 512, 520), (129, 6150, 264, 3080)])
+def test_dx_products_match_oracle(n, v, d, vchunk, xdt, dev) -> None:
+    x, w, t = _case((n,), v, d, xdt, torch.bfloat16, dev, seed=n + v, ignore_every=9,
+                    wstd=0.05 if d >= 256 else 1.0)
+    t[-1] = v - 1
+    with FC.vocab_chunk_rows(vchunk):
+        _check(x, w, t, 0.01, f"n {n} v {v} d {d} chunk {vchunk}")
+
+
+# The C boundary's products (the accumulate form) at K of whole 16-byte chunks but not of
+# whole slices: 1000 tokens, 1032 vocab rows.
+def test_accumulate_products_k_tail(dev) -> None:
+    n, v, d = 1000, 1032, 72
+    x, w, t = _case((n,), v, d, torch.bfloat16, torch.bfloat16, dev, seed=5, ignore_every=9)
+    wb, wt = FC.lmhead_weight_bf16(w)
+    xr = x.detach().requires_grad_(True)
+    acc = torch.zeros(v, d, device=dev)
+    FC.linear_cross_entropy_accumulate(xr, wb, wt, acc, t).backward()
+    _, dx_ref, dw_ref = OK.linear_ce(x, w, t, logits_dtype=torch.bfloat16)
+    assert _rel_fro(xr.grad, dx_ref) < 1e-2 and _rel_fro(acc, dw_ref) < 1e-2
+
+
+@pytest.mark.parametrize("rows,cols,pad", [(1, 8, 0), (63, 72, 8), (64, 64, 0), (129, 200, 16),
+                                           (1000, 136, 0)])
+def test_transposed_copy_is_exact(rows, cols, pad, dev) -> None:
+    src = torch.full((rows, cols + pad), float("nan"), dtype=torch.bfloat16, device=dev)
+    src[:, :cols] = torch.randn(rows, cols, device=dev)
+    out = FC._transpose_bf16(src[:, :cols])
+    assert torch.equal(out[:, :rows], src[:, :cols].t())
+    assert not out[:, rows:].any()
+
+
 _CE_PARAMS = [pytest.param(*c, stored, id=f"{i}-{'stored' if stored else 'recompute'}")
               for i, c in enumerate(_CE_CASES) for stored in (True, False)
               if not (stored and c[3] == torch.float32 and c[4] == torch.float32)]
