@@ -663,13 +663,12 @@ void attn_bwd_dkdv_pipe(BwdArgs a) {
 // on one XCD (consecutive KV tiles of one pack and KV head) then read the same
 // Q / dO tiles at about the same time, from that XCD's L2 (cfg3 backward
 // 4.94 -> 4.82 ms against walking up from each KV tile's diagonal).
-// At most kPairsMaxSteps steps per KV tile (G * S / 32); longer problems take the
+// Every step's 32 query rows lie inside the sequence: no buffer bound.  At
+// most kPairsMaxSteps steps per KV tile (G * S / 32); longer problems take the
 // 2-wave kernel above.
 constexpr int kPairsMaxSteps = 1024;
 
-// GEN: any sequence length and any head dim 72 .. 128 that is a multiple of 8
-// (zero rows and columns as in attn_bwd_dkdv_pipe).
-template <int DP, bool DS, bool GEN>
+template <int DP, bool DS>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2)))
 void attn_bwd_dkdv_pairs(BwdArgs a) {
   constexpr int NT = 256, NB = 2, BN = 32 * NB;
@@ -730,10 +729,8 @@ void attn_bwd_dkdv_pairs(BwdArgs a) {
   {
     const bf16_t *row = pwave ? a.k.row(b, hk, kvr) : a.v.row(b, hk, kvr);
 #pragma unroll
-    for (int dk = 0; dk < NDK; ++dk) {
-      if (GEN && 16 * dk + 8 * hh >= a.D) kvf[dk] = bf16x8_t{};
-      else kvf[dk] = *reinterpret_cast<const bf16x8_t *>(row + 16 * dk + 8 * hh);
-    }
+    for (int dk = 0; dk < NDK; ++dk)
+      kvf[dk] = *reinterpret_cast<const bf16x8_t *>(row + 16 * dk + 8 * hh);
   }
   f32x16_t acc[NDB];  // dV (P-wave) or dK (dP-wave)
 #pragma unroll
@@ -744,17 +741,13 @@ void attn_bwd_dkdv_pairs(BwdArgs a) {
   // chunk i * 128 + tid, rows 8 i + tid / 16, and the swizzle repeats every
   // 16 rows, so chunks i and i + 2 share a lane offset): the dP-waves, whose
   // dS stores share the in-order vmcnt, then never wait on a DMA.
-  // GEN: rows past the sequence end and columns past the head dim are zeros
-  // (kDmaZero); instruction i's row is drow + i * (rows per instruction).
   uint32_t qoff[NCH], goff[NCH];
-  const int drow = (DS ? tid & 127 : tid) / (DP / 8);
 #pragma unroll
   for (int i = 0; i < NCH; ++i) {
     int r, c;
     SwzTile<DP>::at(DS ? i * 128 + (tid & 127) : i * NT + tid, r, c);
-    const bool in = !GEN || c * 8 < a.D;
-    qoff[i] = in ? (uint32_t)((r * a.q.ss + c * 8) * 2) : kDmaZero;
-    goff[i] = in ? (uint32_t)((r * a.dout.ss + c * 8) * 2) : kDmaZero;
+    qoff[i] = (uint32_t)((r * a.q.ss + c * 8) * 2);
+    goff[i] = (uint32_t)((r * a.dout.ss + c * 8) * 2);
   }
   int roffs[NDK], coffs[NDB][2];
   {
@@ -810,22 +803,10 @@ void attn_bwd_dkdv_pairs(BwdArgs a) {
   auto dma_step = [&](int si, auto Rc) {
     const uint32_t q0 = si & 0xfffff, g = (si >> 20) & 0xff;
     const uint32_t ro = (g * (uint32_t)S + q0) * 4u;
-    const int left = S - (int)q0;
-    if constexpr (GEN) {  // 4 bytes per lane (see attn_bwd_dkdv_pipe)
-      const uint32_t rv = l32 < left ? 4u * l32 : kDmaZero;
-      if (wave == 0 && lane < 32) dma4_rs(lrs, ro, rv, lslot(Rc));
-      if (wave == 0 && lane >= 32) dma4_rs(trs, ro, rv, lslot(Rc));
-      if (wave == 1) dma_docs_gen(drs, (int)q0, S, lane, dslot(Rc));
-    } else {
-      if (wave == 0 && lane < 8) dma16_rs(lrs, ro, 16 * lane, lslot(Rc));
-      if (wave == 0 && lane >= 8 && lane < 16) dma16_rs(trs, ro, 16 * (lane - 8), lslot(Rc));
-      if (wave == 1 && lane < 16) dma16_rs(drs, q0 * 8u, 16 * lane, dslot(Rc));
-    }
+    if (wave == 0 && lane < 8) dma16_rs(lrs, ro, 16 * lane, lslot(Rc));
+    if (wave == 0 && lane >= 8 && lane < 16) dma16_rs(trs, ro, 16 * (lane - 8), lslot(Rc));
+    if (wave == 1 && lane < 16) dma16_rs(drs, q0 * 8u, 16 * lane, dslot(Rc));
     const uint32_t qo = g * qsh2 + q0 * qss2, go = g * gsh2 + q0 * gss2;
-    // Rows of one instruction: 128 or 256 lanes of 16 bytes.
-    auto in_row = [&](int i, uint32_t off) {
-      return !GEN || drow < left - i * ((DS ? 128 : NT) / (DP / 8)) ? off : kDmaZero;
-    };
     if constexpr (DS) {
       if (pwave) {
         // The LDS destinations are formed here, not hoisted out of the loop
@@ -834,18 +815,16 @@ void attn_bwd_dkdv_pairs(BwdArgs a) {
         asm volatile("" : "+s"(wb));
 #pragma unroll
         for (int i = 0; i < 2 * NCH; ++i)
-          dma16_rs(qrs, qo + (i >> 1) * 16 * qss2, in_row(i, qoff[i & 1]), qslot(Rc) + i * 2048 + wb);
+          dma16_rs(qrs, qo + (i >> 1) * 16 * qss2, qoff[i & 1], qslot(Rc) + i * 2048 + wb);
 #pragma unroll
         for (int i = 0; i < 2 * NCH; ++i)
-          dma16_rs(grs, go + (i >> 1) * 16 * gss2, in_row(i, goff[i & 1]), gslot(Rc) + i * 2048 + wb);
+          dma16_rs(grs, go + (i >> 1) * 16 * gss2, goff[i & 1], gslot(Rc) + i * 2048 + wb);
       }
     } else {
 #pragma unroll
-      for (int i = 0; i < NCH; ++i)
-        dma16_rs(qrs, qo, in_row(i, qoff[i]), qslot(Rc) + (i * 4 + wave) * 1024);
+      for (int i = 0; i < NCH; ++i) dma16_rs(qrs, qo, qoff[i], qslot(Rc) + (i * 4 + wave) * 1024);
 #pragma unroll
-      for (int i = 0; i < NCH; ++i)
-        dma16_rs(grs, go, in_row(i, goff[i]), gslot(Rc) + (i * 4 + wave) * 1024);
+      for (int i = 0; i < NCH; ++i) dma16_rs(grs, go, goff[i], gslot(Rc) + (i * 4 + wave) * 1024);
     }
   };
   const int kvmax = kt * BN + blk * 32 + 31;
@@ -959,7 +938,6 @@ void attn_bwd_dkdv_pairs(BwdArgs a) {
 #pragma unroll
     for (int db = 0; db < NDB; ++db) {
       const int d = 32 * db + l32;
-      if (GEN && d >= a.D) continue;
 #pragma unroll
       for (int j = 0; j < 16; ++j) {
         const int kvw = kt * BN + blk * 32 + 8 * (j >> 2) + 4 * hh + (j & 3);
@@ -1059,7 +1037,6 @@ void attn_bwd_dkdv_pairs(BwdArgs a) {
 #pragma unroll
     for (int db = 0; db < NDB; ++db) {
       const int d = 32 * db + l32;
-      if (GEN && d >= a.D) continue;
 #pragma unroll
       for (int j = 0; j < 16; ++j) {
         const int kvw = kt * BN + blk * 32 + 8 * (j >> 2) + 4 * hh + (j & 3);
@@ -1667,8 +1644,7 @@ __global__ __launch_bounds__(64 * WAVES) void attn_bwd_dq_wide(BwdArgs a) {
 // non-temporal (dO and O are streamed once; at cfg3 185 -> 179 us with four
 // rows instead of eight, 221 -> 185 us non-temporal instead of cached).
 constexpr int kDeltaRowsPerGroup = 4;
-// Lanes past the head dim (GEN) add zeros.
-template <int DP, bool GEN>
+template <int DP>
 __global__ __launch_bounds__(256) void attn_bwd_delta(BwdArgs a) {
   constexpr int TPR = DP / 8, RPP = 256 / TPR, NP = kDeltaRowsPerGroup;
   const int64_t rows = (int64_t)a.B * a.Hq * a.S;
@@ -1678,8 +1654,7 @@ __global__ __launch_bounds__(256) void attn_bwd_delta(BwdArgs a) {
 #pragma unroll
   for (int p = 0; p < NP; ++p) {
     r[p] = ((int64_t)blockIdx.x * NP + p) * RPP + threadIdx.x / TPR;
-    gv[p] = ov[p] = u32x4{0u, 0u, 0u, 0u};
-    if (r[p] < rows && (!GEN || 8 * sub < a.D)) {
+    if (r[p] < rows) {
       const int s = (int)(r[p] % a.S);
       const int64_t bh = r[p] / a.S;
       const int h = (int)(bh % a.Hq), b = (int)(bh / a.Hq);
@@ -1716,8 +1691,7 @@ __global__ __launch_bounds__(256) void attn_bwd_delta(BwdArgs a) {
 // (2 bytes per pair and head) from HBM.
 constexpr int kDsMaxTiles = kPairsMaxSteps / 8;  // 64-row KV tiles per list (G >= 4)
 
-// GEN: any sequence length and any head dim 72 .. 128 that is a multiple of 8.
-template <int DP, bool GEN>
+template <int DP>
 __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4, 4)))
 void attn_bwd_dq_ds(BwdArgs a) {
   static_assert(DP == 128, "head dim 128");
@@ -1778,9 +1752,7 @@ void attn_bwd_dq_ds(BwdArgs a) {
   const uint32_t tri = (uint32_t)(qt * (qt + 1) / 2);
   const uint32_t blkb = (uint32_t)(G * 8192), halfb = (uint32_t)(G * 4096), quadb = (uint32_t)(g0 * 4096);
   uint32_t koff[1];
-  int drow = 0;  // GEN: this thread's row of a K half
-  if constexpr (GEN) drow = Dma::offsets_gen(a.k.ss, wave, lane, a.D, koff);
-  else Dma::offsets(a.k.ss, wave, lane, koff);
+  Dma::offsets(a.k.ss, wave, lane, koff);
   const uint32_t soff0 = (uint32_t)((wave * 64 + lane) * 16), soff1 = soff0 + 8 * 1024;
   // ds_read_b64_tr_b16 addresses (see lds_col_frag): K^T of head-dim block
   // db (swizzled K half), dS^T of this wave's sub-block (64-byte pitch).
@@ -1811,9 +1783,7 @@ void attn_bwd_dq_ds(BwdArgs a) {
     const int uu = u < U ? u : U - 1;
     const int e = __builtin_amdgcn_readfirstlane(ents[uu >> 1]);
     const uint32_t kt = (uint32_t)plan_tile(e), half = (uint32_t)(uu & 1);
-    const uint32_t kv0 = kt * 64 + half * 32;
-    if constexpr (GEN) Dma::copy_gen(krs, kv0 * kss2, koff, drow, a.S - (int)kv0, kslot(Rc), wave);
-    else Dma::copy_rs(krs, kv0 * kss2, koff, kslot(Rc), wave);
+    Dma::copy_rs(krs, (kt * 64 + half * 32) * kss2, koff, kslot(Rc), wave);
     const uint32_t so = (tri + kt) * blkb + half * halfb + quadb;
     dma16_rs_nt(drs, so, soff0, sslot(Rc) + wave * 1024);
     dma16_rs_nt(drs, so, soff1, sslot(Rc) + (8 + wave) * 1024);
@@ -1859,13 +1829,11 @@ void attn_bwd_dq_ds(BwdArgs a) {
   // query half), register j <-> head-dim row 8 (j / 4) + 4 hh + j % 4.
   const int sl = lane & 31;
   const int q = qt * 64 + qs * 32 + 8 * ((sl & 15) >> 2) + 4 * (sl >> 4) + (sl & 3);
-  if (GEN && q >= a.S) return;
   bf16_t *qrow = a.dq.row(b, h, q);
 #pragma unroll
   for (int db = 0; db < NDB; ++db)
 #pragma unroll
     for (int jq = 0; jq < 4; ++jq) {
-      if (GEN && 32 * db + 8 * jq >= a.D) continue;
       typedef __bf16 bf16x4_t __attribute__((ext_vector_type(4)));
       bf16x4_t o4;
 #pragma unroll
@@ -1993,24 +1961,22 @@ extern "C" int pb_attn_bwd(const pb_bhsd *q, const pb_bhsd *k, const pb_bhsd *v,
       ((G - 1) * std::max(q->stride_h, dout->stride_h) + s * std::max(q->stride_s, dout->stride_s)) *
               2 < (1LL << 31) &&
       G * s * 4 < (1LL << 31);
-  const bool pairs = pipe && cfg.pairs && 2 * G * ((s + 63) / 64) <= kPairsMaxSteps && pairs_fit;
+  const bool pairs = pipe && !gen && cfg.pairs && G * s / 32 <= kPairsMaxSteps && pairs_fit;
   if (pairs && cfg.ds) {
     // Kept dS: D, then dK/dV storing dS, then dQ = scale * dS K.
     a.ds = ws + delta_bytes;
     a.ds_pair = ds_pair_bytes(G, s);
     const int64_t rows = b * hq * s;
     const int64_t drows = (int64_t)kDeltaRowsPerGroup * (256 / (128 / 8));  // rows per workgroup
-    const dim3 g_d((unsigned)((rows + drows - 1) / drows)), g_ds((unsigned)(b * (hq / 4) * a.nqt_dq));
-    if (gen) hipLaunchKernelGGL((attn_bwd_delta<128, true>), g_d, dim3(256), 0, st, a);
-    else hipLaunchKernelGGL((attn_bwd_delta<128, false>), g_d, dim3(256), 0, st, a);
+    hipLaunchKernelGGL(attn_bwd_delta<128>, dim3((unsigned)((rows + drows - 1) / drows)), dim3(256),
+                       0, st, a);
     rc = launch_status("pb_attn_bwd(delta)");
     if (rc) return rc;
-    if (gen) hipLaunchKernelGGL((attn_bwd_dkdv_pairs<128, true, true>), g_kv, dim3(256), 0, st, a);
-    else hipLaunchKernelGGL((attn_bwd_dkdv_pairs<128, true, false>), g_kv, dim3(256), 0, st, a);
+    hipLaunchKernelGGL((attn_bwd_dkdv_pairs<128, true>), g_kv, dim3(256), 0, st, a);
     rc = launch_status("pb_attn_bwd(dkdv)");
     if (rc) return rc;
-    if (gen) hipLaunchKernelGGL((attn_bwd_dq_ds<128, true>), g_ds, dim3(512), 0, st, a);
-    else hipLaunchKernelGGL((attn_bwd_dq_ds<128, false>), g_ds, dim3(512), 0, st, a);
+    hipLaunchKernelGGL(attn_bwd_dq_ds<128>, dim3((unsigned)(b * (hq / 4) * a.nqt_dq)), dim3(512), 0,
+                       st, a);
     return launch_status("pb_attn_bwd(dq)");
   }
   if (pipe && cfg.dq_chunk > 0) {
@@ -2039,11 +2005,11 @@ extern "C" int pb_attn_bwd(const pb_bhsd *q, const pb_bhsd *k, const pb_bhsd *v,
     else                                                                                         \
       hipLaunchKernelGGL((attn_bwd_dkdv_pipe<DP, W, SP, false>), g_kv, dim3(64 * W), 0, st, a);  \
   } while (0)
-    if (pairs && gen)
-      hipLaunchKernelGGL((attn_bwd_dkdv_pairs<128, false, true>), g_kv, dim3(256), 0, st, a);
-    else if (pairs)
-      hipLaunchKernelGGL((attn_bwd_dkdv_pairs<128, false, false>), g_kv, dim3(256), 0, st, a);
-    else if (cfg.kv_waves == 4) PB_KVP(64, 4, false);  // (wider head dims take 64-row KV tiles)
+    if (pairs)
+      hipLaunchKernelGGL((attn_bwd_dkdv_pairs<128, false>), g_kv, dim3(256), 0, st, a);
+    else if (cfg.kv_waves == 4 && d > 64)  // (the unbounded form of these shapes is the paired one)
+      hipLaunchKernelGGL((attn_bwd_dkdv_pipe<128, 4, false, true>), g_kv, dim3(256), 0, st, a);
+    else if (cfg.kv_waves == 4) PB_KVP(64, 4, false);
     else if (cfg.split) {
       // Lists of >= kKvChunkSteps steps are walked as two halves by two workgroups.
       a.kv_chunk = kKvChunkSteps;

@@ -304,10 +304,7 @@ inline bool views_vectorizable(int64_t d, std::initializer_list<const pb_bhsd *>
 // sub-block holds query row 8 ((s % 16) / 4) + 4 (s / 16) + s % 4 (the row
 // order of the dK/dV kernel's dS accumulators).
 constexpr int64_t kDsMaxBytes = 32LL << 30;
-inline int64_t ds_tri(int64_t s) {
-  const int64_t t = (s + 63) / 64;
-  return t * (t + 1) / 2;
-}
+inline int64_t ds_tri(int64_t s) { return (s / 64) * (s / 64 + 1) / 2; }
 inline int64_t ds_pair_bytes(int64_t g, int64_t s) { return ds_tri(s) * g * 8192; }
 inline int64_t ds_bytes(int64_t b, int64_t hq, int64_t hkv, int64_t s) {
   return b * hkv * ds_pair_bytes(hq / hkv, s);
@@ -315,7 +312,7 @@ inline int64_t ds_bytes(int64_t b, int64_t hq, int64_t hkv, int64_t s) {
 
 struct AttnConfig {
   int fwd_waves, dq_waves, kv_waves, split;
-  int pairs;  // head dim 72 .. 128 on a full grid: dK/dV by attn_bwd_dkdv_pairs on 64-row KV tiles
+  int pairs;  // head dim 128 on a full grid: dK/dV by attn_bwd_dkdv_pairs on 64-row KV tiles
   // dS kept: the paired dK/dV kernel stores its bf16 dS tiles and dQ = scale * dS K
   // is a streaming pass over them (attn_bwd_dq_ds) instead of a kernel that
   // recomputes S and dP; D = rowsum(dO * O) then comes from attn_bwd_delta.
@@ -364,9 +361,11 @@ inline AttnConfig attn_config(int64_t b, int64_t hq, int64_t hkv, int64_t s, int
   c.dq_waves = big_q ? 4 : 2;
   c.kv_waves = b * hkv * tiles(128) >= kFill ? 4 : 2;
   c.split = (c.kv_waves == 2 && b * hkv * tiles(64) < kFill && hq > hkv) ? 1 : 0;
-  // Head dims padded to 128 on a full grid: two (P, dP) wave pairs per 64-row
-  // KV tile, two workgroups per CU (the KV tile of the 2-wave kernels).
-  c.pairs = (d > 64 && d % 8 == 0 && c.kv_waves == 4) ? 1 : 0;
+  // Head dim 128 on a full grid: two (P, dP) wave pairs per 64-row KV tile,
+  // two workgroups per CU (the KV tile of the 2-wave kernels).  Only whole
+  // 64-row tiles: the pair passes P as bf16, the kernels of every other shape
+  // form dS from the fp32 P.
+  c.pairs = (d == 128 && s % 64 == 0 && c.kv_waves == 4) ? 1 : 0;
   if (c.pairs) c.kv_waves = 2;
   c.ds = (c.pairs && (hq / hkv) % 4 == 0 && ds_pair_bytes(hq / hkv, s) < (1LL << 31) &&
           ds_bytes(b, hq, hkv, s) <= kDsMaxBytes) ? 1 : 0;

@@ -239,6 +239,32 @@ def test_ragged_matches_padded(B, Hq, Hkv, S, D, dev) -> None:
 
 
 @pytest.mark.parametrize(
+    "B,Hq,Hkv,S,D",
+    [
+        (9, 32, 8, 1025, 128),  # a full grid of a length that is no multiple of 64
+        (9, 32, 8, 1024, 96),  # of a padded head dim
+    ],
+)
+def test_ds_from_fp32_p_on_full_grids(B, Hq, Hkv, S, D, dev) -> None:
+    """Outside whole 64-row tiles of head dim 128 the backward forms dS from the fp32 P.
+    Rounding a normal value to bf16 leaves 1.66e-3 of its 2-norm (2^-8 / sqrt(3) of the
+    mantissa's scale), so dq and dk, which see the rounding of dS, their own and a little
+    of O's through delta, are sqrt(2) of that and some: 2.5e-3.  P rounded first would
+    make it sqrt(3) and as much again: over 2.9e-3.  The bound lies between, at 2^-8.5."""
+    packs = [W.fill_sequential(np.random.default_rng(S + b), S, np.log(300), 1.0, 1, S)
+             for b in range(B)]
+    doc = W.doc_ids_from_lengths(packs, S).to(dev)
+    q, k, v, do = _inputs(B, Hq, Hkv, S, D, dev, seed=S)
+    _, dq, dk, _ = _run(q, k, v, do, doc)
+    b, g, G = 4, 3, Hq // Hkv
+    sl, hs = slice(b, b + 1), slice(G * g, G * (g + 1))
+    ref = OA.attention(q[sl, hs], k[sl, g : g + 1], v[sl, g : g + 1], doc[sl].cpu(), do[sl, hs])
+    for name, got, want in (("dq", dq[sl, hs], ref["dq"]), ("dk", dk[sl, g : g + 1], ref["dk"])):
+        err = float((got.cpu().double() - want).norm() / want.norm())
+        assert err <= 2 ** -8.5, f"{name}: {err:.2e}"
+
+
+@pytest.mark.parametrize(
     "B,Hq,Hkv,S,D,mu,misaligned",
     [
         (1, 4, 2, 4096, 64, 1e9, False),  # one document: the longest lists, 64 steps a wave
