@@ -24,6 +24,9 @@ struct FwdArgs {
   int B, Hq, Hkv, S, D, nqt, nkt;
   float sl2;  // softmax scale * log2(e)
   int vec;    // 16-byte global access allowed
+  // Growth of a row's running max (log2 units) that attn_fwd_wave leaves in the
+  // exponentials; 0 keeps the max exact (see softmax state in attn_fwd_pipe).
+  float tau;
   // KV split (pipelined kernel): chunk = KV tiles per workgroup (0: whole
   // list); bm = query rows per tile; partial outputs [split][B][Hq][S][D]
   // and log-sum-exps [split][B][Hq][S], fp32.

@@ -455,9 +455,25 @@ void attn_fwd_pipe(FwdArgs a) {
   // max of S(u), the move rule (max > m_run + kTau), and, if a lane moved,
   // the O / l rescale and the exponentials again against the new max.
   typedef __bf16 bf16x2_t __attribute__((ext_vector_type(2)));
+  // GEN takes the exact running max instead, from S(u) before its exponentials
+  // (take_max), so that a row's largest P is 1 and rounds to bf16 without an
+  // error; commit rescales when a lane moved.  These shapes' outputs are as
+  // close to float64 as the register-staged kernel's (scores of standard
+  // deviation 4, relative 2-norm: 1.71e-3, with kTau 2.02e-3), for 5% (short
+  // documents) to 16% (one document) of the time.
   constexpr float kLim = 256.0f;  // 2^kTau
   static_assert(kTau == 8.0f, "kLim is 2^kTau");
-  float m_use[NQB], lim[NQB], lt[NQB];
+  float m_use[NQB], m_next[NQB], lim[NQB], lt[NQB];
+  auto take_max = [&](const f32x16_t (&sv)[NQB]) {
+#pragma unroll
+    for (int qb = 0; qb < NQB; ++qb) {
+      float m0 = sv[qb][0];
+#pragma unroll
+      for (int j = 1; j < 16; ++j) m0 = fmaxf(m0, sv[qb][j]);
+      m_next[qb] = fmaxf(m_run[qb], xor32_max(m0) * sl2);
+      m_use[qb] = m_next[qb] == -INFINITY ? 0.f : m_next[qb];
+    }
+  };
 #pragma unroll
   for (int qb = 0; qb < NQB; ++qb) {
     m_use[qb] = 0.f;
@@ -493,6 +509,25 @@ void attn_fwd_pipe(FwdArgs a) {
   // End of sub-tile u (after PV(u-1), which used the old max): the rare slow
   // path, then the sums.
   auto softmax_commit = [&](const f32x16_t (&sv)[NQB], bf16x8_t (&pf)[NQB][2]) {
+    if constexpr (GEN) {
+      bool moved = false;
+#pragma unroll
+      for (int qb = 0; qb < NQB; ++qb) moved |= m_next[qb] != m_run[qb];
+      if (__builtin_amdgcn_ballot_w64(moved) != 0) {
+#pragma unroll
+        for (int qb = 0; qb < NQB; ++qb) {
+          // (both -inf: the difference would be NaN)
+          const float alpha = m_next[qb] == m_run[qb] ? 1.f : fast_exp2(m_run[qb] - m_next[qb]);
+          l_run[qb] *= alpha;
+#pragma unroll
+          for (int db = 0; db < NDB; ++db) oacc[qb][db] *= alpha;
+          m_run[qb] = m_next[qb];
+        }
+      }
+#pragma unroll
+      for (int qb = 0; qb < NQB; ++qb) l_run[qb] += lt[qb];
+      return;
+    }
     bool slow = false;
 #pragma unroll
     for (int qb = 0; qb < NQB; ++qb) slow |= !(lt[qb] <= lim[qb]);
@@ -628,6 +663,7 @@ void attn_fwd_pipe(FwdArgs a) {
       for (int k = 0; k < kAhead; ++k) read_step(k);
 #pragma unroll
       for (int qb = 0; qb < NQB; ++qb) sn[qb] = zero16();
+      if constexpr (GEN) take_max(sc);  // (while the first fragments are on their way)
       __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
       for (int dk = 0; dk < NDK; ++dk) {
@@ -704,6 +740,7 @@ void attn_fwd_pipe(FwdArgs a) {
     bf16x8_t vf[NVF], pf[NQB][2];
 #pragma unroll
     for (int f = 0; f < NVF; ++f) vf[f] = vfrag_of(f, vprev);
+    if constexpr (GEN) take_max(sc);
 #pragma unroll
     for (int step = 0; step < NDK; ++step) {
       pv_step(step, vf[step], pfp);
@@ -849,9 +886,10 @@ extern "C" int pb_attn_fwd(const pb_bhsd *q, const pb_bhsd *k, const pb_bhsd *v,
   // the pack's document ids must span < 2 GiB.
   const bool pipe = a.vec && s * std::max(k->stride_s, v->stride_s) * 2 < (1LL << 31) &&
                     s * 8 < (1LL << 31);
-  if (pipe && cfg.wave_fwd) return launch_fwd_wave(a, st);
   const bool gen = !((d == 64 || d == 128) && s % 64 == 0 &&
                      (reinterpret_cast<uintptr_t>(doc_ids) & 15) == 0 && doc_stride % 2 == 0);
+  a.tau = gen ? 0.f : 8.f;  // (as attn_fwd_pipe: GEN exact, else kTau)
+  if (pipe && cfg.wave_fwd) return launch_fwd_wave(a, st);
   if (pipe && cfg.fwd_chunk > 0) {
     PB_CHECK_ARG(workspace != nullptr, "pb_attn_fwd: workspace is required for this shape");
     a.chunk = cfg.fwd_chunk;

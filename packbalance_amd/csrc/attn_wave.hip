@@ -169,8 +169,8 @@ __device__ __forceinline__ void settle() {
 }
 
 // ---------------------------------------------------------------- forward
-// Per step: S^T = K Q^T, online softmax with the running max moved only when
-// it grows by more than 8 (log2 units), O^T += V^T P^T.  The next step's K goes
+// Per step: S^T = K Q^T, online softmax with the running max moved when it
+// grows by more than FwdArgs::tau (log2 units), O^T += V^T P^T.  The next step's K goes
 // to the one K slot as soon as S has read it, its V to the other of two V
 // slots: 12 KiB a wave, three waves per SIMD.  (K fragments loaded straight
 // into registers, 32 rows of 16 bytes an instruction, measured 2x slower.)
@@ -238,7 +238,7 @@ void attn_fwd_wave(FwdArgs a) {
 #pragma unroll
     for (int j = 1; j < 16; ++j) m0 = fmaxf(m0, s[j]);
     const float m1 = xor32_max(m0) * sl2;
-    const bool move = m1 > m_run + 8.0f;
+    const bool move = m1 > m_run + a.tau;
     if (__builtin_amdgcn_ballot_w64(move) != 0) {
       const float mn = move ? m1 : m_run;
       const float alpha = mn == m_run ? 1.f : fast_exp2(m_run - mn);
