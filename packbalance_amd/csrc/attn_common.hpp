@@ -333,12 +333,25 @@ struct AttnConfig {
 // When the wave kernels serve a shape (see attn_wave.hip): head dims to 64 and
 // a small grid, counted in 128-row query tiles over all heads; kWaveMaxS bounds
 // the list entries a wave can hold.  The lines lie where the wave kernels win
-// for short and for whole-sequence documents alike, with the head counts of
-// [B, S], 12 / 4 heads, D 64 in us, workgroup -> wave kernels:
+// for short documents and lose at most 3%, at [1, 4096] up to 8%, with one
+// document of the whole sequence (in brackets).  [B, S], 12 / 4 heads, D 64 in
+// us, workgroup -> wave kernels:
 //   forward   [4, 2048] 42 -> 27 (one document: 68 -> 60), [8, 2048] 72 -> 52,
 //             but [16, 2048] 107 -> 94 (one document: 179 -> 204)
 //   backward  [4, 2048] 112 -> 66 (249 -> 149), [16, 2048] 299 -> 241 (535 ->
-//             491), but [16, 4096] 752 -> 765 (1648 -> 1804)
+//             491), but [16, 4096] 752 -> 765 (1648 -> 1804); dQ + dK/dV
+// The backward's dK/dV kernel has a workgroup per KV tile and KV head, which
+// walks the query heads of the group one after the other, where the workgroup
+// kernels split them.  So it wins with enough (pack, KV head) pairs for the
+// group, whole-sequence documents, us, workgroup -> wave kernels:
+//   12 / 3 heads, [1, 2048] 74 -> 64, [1, 4096] 176 -> 159; 20 / 4, [1, 2048]
+//   105 -> 81; 64 / 8, [1, 2048] 210 -> 200; but 4 / 1, [1, 1024] 29 -> 34; 16 / 1,
+//   [1, 2048] 85 -> 229; 71 / 1, [1, 2048] 315 -> 961; 49 / 7, [1, 4096] 0.84x; packs
+//   that differ, 8 / 1, [8, 2048], documents of about 400 0.87x
+// and always where those do not split (512 tiles of 64 KV rows: 64 / 8, [1, 4096]
+// 919 -> 619), up to as many tiles, times their length, as
+//   [4, 4096], 16 / 8 583 -> 601 and [3, 4096], 16 / 16 453 -> 454 (187 -> 137 with
+//   short documents), but [6, 4096], 16 / 16 849 -> 919; [12, 2048] 492 -> 530
 constexpr int kWaveLeast = 6;  // least steps of a list worth another wave
 constexpr int64_t kWaveMaxS = 4096;
 inline int64_t wave_tiles(int64_t b, int64_t hq, int64_t s, int64_t d) {
@@ -348,8 +361,12 @@ inline int64_t wave_tiles(int64_t b, int64_t hq, int64_t s, int64_t d) {
 inline bool wave_fwd_grid(int64_t b, int64_t hq, int64_t s, int64_t d) {
   return wave_tiles(b, hq, s, d) <= (s <= 2048 ? 1536 : 1024);
 }
-inline bool wave_bwd_grid(int64_t b, int64_t hq, int64_t s, int64_t d) {
-  return wave_tiles(b, hq, s, d) <= 3072;
+inline bool wave_bwd_grid(int64_t b, int64_t hq, int64_t hkv, int64_t s, int64_t d) {
+  const int64_t t = wave_tiles(b, hq, s, d), tk = wave_tiles(b, hkv, s, d);
+  if (t > 3072 || t + tk > 4096 || t * s > 2048 * 4096 || tk * s > 1536 * 4096) return false;
+  const int64_t g = hq / hkv, pairs = b * hkv;
+  if (g == 1 || pairs * ((s + 63) / 64) >= 512) return true;
+  return g <= (s <= 2048 ? 8 : 6) && 4 * pairs >= 3 * g && (hkv > 1 || g <= 4);
 }
 
 inline AttnConfig attn_config(int64_t b, int64_t hq, int64_t hkv, int64_t s, int64_t d) {
@@ -371,7 +388,7 @@ inline AttnConfig attn_config(int64_t b, int64_t hq, int64_t hkv, int64_t s, int
           ds_bytes(b, hq, hkv, s) <= kDsMaxBytes) ? 1 : 0;
   if (c.ds) c.dq_waves = 2;  // dQ on the 64-row query tiles of the dS blocks
   c.wave_fwd = wave_fwd_grid(b, hq, s, d) ? 1 : 0;
-  c.wave_bwd = wave_bwd_grid(b, hq, s, d) ? 1 : 0;
+  c.wave_bwd = wave_bwd_grid(b, hq, hkv, s, d) ? 1 : 0;
   if (c.wave_fwd) c.fwd_waves = 1;
   if (c.wave_bwd) {
     c.dq_waves = c.kv_waves = 1;

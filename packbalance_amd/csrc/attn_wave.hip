@@ -9,8 +9,8 @@
 // [4, 2048], 12 / 4 heads: dK/dV 107 us for 108 steps of the longest list
 // where the mean is 36.
 //
-// Here a workgroup of four waves owns ONE 32-row tile (of queries, or of KV
-// rows for dK/dV).  Plans are 32 x 32, so only tiles that hold a pair are
+// Here a workgroup of one to eight waves owns ONE 32-row tile (of queries, or of
+// KV rows for dK/dV).  Plans are 32 x 32, so only tiles that hold a pair are
 // visited.  The list is shared out evenly over the waves (wave_share), each
 // wave streams its own share with its own LDS ring (DMA one step ahead, waited
 // for with vmcnt alone) and no barrier, and the waves' results meet once, in
@@ -34,11 +34,16 @@ namespace pb {
 namespace attn {
 namespace {
 
-// Waves per workgroup of the forward and dQ.  Two were the fastest or within
-// 3% of it from 768 to 12288 tiles, short and long lists ([4, 2048], 12 heads:
-// forward 30 / 27 / 34 us and dQ 35 / 33 / 42 us with 1 / 2 / 4 waves): more
-// leave most of a workgroup's LDS to waves without a share.
-constexpr int kNWq = 2;
+// Waves per workgroup of the forward and dQ, and the least steps worth another
+// wave.  Two were the fastest or within 3% of it from 768 to 12288 tiles, short
+// and long lists ([4, 2048], 12 heads: forward 30 / 27 / 34 us and dQ 35 / 33 /
+// 42 us with 1 / 2 / 4 waves): more leave most of a workgroup's LDS to waves
+// without a share.  Up to kFewQ tiles (three per CU) the CUs have room, the
+// longest list sets the time, and four are faster: forward of [1, 2048], 4
+// heads, one document 21.2 -> 13.4 us (the workgroup kernels 18.7), [1, 2048],
+// 12 heads 22.5 -> 17.1 (30.3); at 1152 tiles ([1, 3072], 12 heads, documents of
+// about 100) 14.1 -> 15.3.
+constexpr int kFewQ = 768;
 constexpr int kTB = 32 * 64 * 2;   // bytes of one 32 x 64 bf16 tile
 constexpr int NDK = 4, NDB = 2;    // 16-wide k steps and 32-wide blocks of the head dim
 using Dma = TileDma<64, 32, 64>;   // one wave copies a tile: four 1 KiB instructions
@@ -48,11 +53,11 @@ typedef __bf16 bf16x4_t __attribute__((ext_vector_type(4)));
 typedef float f32x4_t __attribute__((ext_vector_type(4)));
 
 // Wave w's part [i0, i1) of n >= 1 steps: at most NW waves of at least
-// kWaveLeast steps (all but the first wave cost a prologue and a merge).
+// LEAST steps (all but the first wave cost a prologue and a merge).
 // Returns the number of waves that have a share.
-template <int NW>
+template <int NW, int LEAST = kWaveLeast>
 __device__ __forceinline__ int wave_share(int n, int w, int &i0, int &i1) {
-  const int nw = max(1, min(NW, n / kWaveLeast));
+  const int nw = max(1, min(NW, n / LEAST));
   i0 = n * w / nw;
   i1 = n * (w + 1) / nw;
   return nw;
@@ -174,18 +179,19 @@ __device__ __forceinline__ void settle() {
 // to the one K slot as soon as S has read it, its V to the other of two V
 // slots: 12 KiB a wave, three waves per SIMD.  (K fragments loaded straight
 // into registers, 32 rows of 16 bytes an instruction, measured 2x slower.)
-__global__ __launch_bounds__(64 * kNWq) __attribute__((amdgpu_waves_per_eu(3, 3)))
+template <int NW, int LEAST>
+__global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(3, 3)))
 void attn_fwd_wave(FwdArgs a) {
-  __shared__ __align__(16) char ks[kNWq][kTB], vs0[kNWq][kTB], vs1[kNWq][kTB];
-  __shared__ __align__(16) int64_t kd0[kNWq][32], kd1[kNWq][32];
-  __shared__ float ml[kNWq][2][64];
+  __shared__ __align__(16) char ks[NW][kTB], vs0[NW][kTB], vs1[NW][kTB];
+  __shared__ __align__(16) int64_t kd0[NW][32], kd1[NW][32];
+  __shared__ float ml[NW][2][64];
   const int lane = threadIdx.x & 63, hh = lane >> 5, l32 = lane & 31;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   int qt, b, h;
   decode_q_major((int)blockIdx.x, a.nqt, a.B, a.Hq, a.Hkv, qt, b, h);
   const int n = a.cnt[b * a.nqt + qt];  // >= 1: every row sees itself
   int i0, i1;
-  const int nw = wave_share<kNWq>(n, wave, i0, i1);
+  const int nw = wave_share<NW, LEAST>(n, wave, i0, i1);
   if (wave >= nw) return;
   const int m = i1 - i0;  // at most 64: n <= kWaveMaxS / 32 over two waves
   const int S = a.S, hk = h / (a.Hq / a.Hkv);
@@ -309,17 +315,18 @@ void attn_fwd_wave(FwdArgs a) {
 // Per step: S^T = K Q^T and dP^T = V dO^T, dS^T = P (dP - delta), dQ^T += K^T
 // dS^T with K^T read from the same K tile.  The next step's V goes to the one
 // V slot as soon as dP has read it, its K to the other of two K slots.
-__global__ __launch_bounds__(64 * kNWq) __attribute__((amdgpu_waves_per_eu(3, 3)))
+template <int NW, int LEAST>
+__global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(3, 3)))
 void attn_bwd_dq_wave(BwdArgs a) {
-  __shared__ __align__(16) char ks0[kNWq][kTB], ks1[kNWq][kTB], vs[kNWq][kTB];
-  __shared__ __align__(16) int64_t kd0[kNWq][32], kd1[kNWq][32];
+  __shared__ __align__(16) char ks0[NW][kTB], ks1[NW][kTB], vs[NW][kTB];
+  __shared__ __align__(16) int64_t kd0[NW][32], kd1[NW][32];
   const int lane = threadIdx.x & 63, hh = lane >> 5, l32 = lane & 31;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   int qt, b, h;
   decode_q_major((int)blockIdx.x, a.nqt_dq, a.B, a.Hq, a.Hkv, qt, b, h);
   const int n = a.qcnt[b * a.nqt_dq + qt];
   int i0, i1;
-  const int nw = wave_share<kNWq>(n, wave, i0, i1);
+  const int nw = wave_share<NW, LEAST>(n, wave, i0, i1);
   if (wave >= nw) return;
   const int m = i1 - i0;
   const int S = a.S, hk = h / (a.Hq / a.Hkv);
@@ -593,24 +600,35 @@ void attn_bwd_dkdv_wave(BwdArgs a) {
 }  // namespace
 
 int launch_fwd_wave(const FwdArgs &a, hipStream_t st) {
-  hipLaunchKernelGGL(attn_fwd_wave, dim3((unsigned)(a.nqt * a.B * a.Hq)), dim3(64 * kNWq), 0, st, a);
+  const int tiles = a.nqt * a.B * a.Hq;
+  const dim3 g((unsigned)tiles);
+  if (tiles <= kFewQ) hipLaunchKernelGGL((attn_fwd_wave<4, 4>), g, dim3(256), 0, st, a);
+  else hipLaunchKernelGGL((attn_fwd_wave<2, kWaveLeast>), g, dim3(128), 0, st, a);
   return launch_status("pb_attn_fwd");
 }
 
 int launch_bwd_wave(const BwdArgs &a, hipStream_t st) {
   // dQ first: it also writes delta = rowsum(dO * O), which dK/dV reads.
-  hipLaunchKernelGGL(attn_bwd_dq_wave, dim3((unsigned)(a.nqt_dq * a.B * a.Hq)), dim3(64 * kNWq), 0,
-                     st, a);
+  const int qtiles = a.nqt_dq * a.B * a.Hq;
+  const dim3 gq((unsigned)qtiles);
+  if (qtiles <= kFewQ) hipLaunchKernelGGL((attn_bwd_dq_wave<4, 4>), gq, dim3(256), 0, st, a);
+  else hipLaunchKernelGGL((attn_bwd_dq_wave<2, kWaveLeast>), gq, dim3(128), 0, st, a);
   const int rc = launch_status("pb_attn_bwd(dq)");
   if (rc) return rc;
   // Waves per workgroup by the number of KV tiles: at 1024 tiles (2048 waves
   // are resident) the longest list still sets the time and four waves are
   // fastest ([2, 2048], 12 / 4 heads: 71 / 41 / 27 us with 1 / 2 / 4 waves;
   // [4, 2048]: 63 / 39 / 37 us), at 4096 two ([16, 2048]: 151 / 140 / 165 us),
-  // beyond that one ([8, 2048], 16 / 16 heads: 87 / 120 / 185 us).
+  // beyond that one ([8, 2048], 16 / 16 heads: 87 / 120 / 185 us).  Up to one
+  // workgroup per CU eight, and to 384 tiles with long lists: one document, dQ and
+  // dK/dV with 4 / 8: [1, 2048], 9 / 3 heads 65 / 53 us (workgroup kernels 67);
+  // 384 tiles: [1, 3072], 16 / 4 132 / 109 (125), but [1, 2048], 6 / 6 38 / 45.
   const int64_t tiles = (int64_t)a.nkt_kv * a.B * a.Hkv;
   const dim3 gk((unsigned)tiles);
-  if (tiles <= 1024) hipLaunchKernelGGL(attn_bwd_dkdv_wave<4>, gk, dim3(256), 0, st, a);
+  const int longest = a.nqt_kv * (a.Hq / a.Hkv);  // steps
+  if (tiles <= 256 || (tiles <= 384 && longest >= 288))
+    hipLaunchKernelGGL(attn_bwd_dkdv_wave<8>, gk, dim3(512), 0, st, a);
+  else if (tiles <= 1024) hipLaunchKernelGGL(attn_bwd_dkdv_wave<4>, gk, dim3(256), 0, st, a);
   else if (tiles <= 4096) hipLaunchKernelGGL(attn_bwd_dkdv_wave<2>, gk, dim3(128), 0, st, a);
   else hipLaunchKernelGGL(attn_bwd_dkdv_wave<1>, gk, dim3(64), 0, st, a);
   return launch_status("pb_attn_bwd(dkdv)");

@@ -297,12 +297,17 @@ def test_exact_max_of_peaked_scores(dense, B, Hq, Hkv, S, D, dev) -> None:
 @pytest.mark.parametrize(
     "B,Hq,Hkv,S,D,mu,misaligned",
     [
-        (1, 4, 2, 4096, 64, 1e9, False),  # one document: the longest lists, 64 steps a wave
-        (1, 2, 1, 4096, 64, 40, False),  # short lists: single waves
+        (1, 4, 2, 4096, 64, 1e9, False),  # few tiles: four waves a query tile, eight a KV tile
+        (2, 4, 2, 4096, 64, 1e9, False),  # two, 64 steps a wave; four
+        (1, 2, 1, 4096, 64, 40, False),  # few heads a group: the backward splits them instead
+        (1, 9, 3, 2047, 56, 1e9, False),  # eight waves a KV tile, a ragged length
+        (1, 16, 4, 3072, 64, 900, False),  # the most KV tiles of eight waves
         (2, 12, 4, 2048, 64, 200, False),  # dK/dV lists shared by four waves
         (4, 16, 16, 2017, 64, 500, False),  # by two
-        (9, 16, 16, 2048, 48, 150, False),  # by none
-        (5, 8, 1, 777, 64, 90, False),  # G = 8
+        (8, 16, 16, 2048, 48, 150, False),  # by none
+        (9, 16, 16, 2048, 48, 150, False),  # past the backward's largest grid
+        (1, 64, 8, 4096, 40, 700, False),  # G = 8, the longest walks of four waves
+        (5, 8, 1, 777, 64, 90, False),  # G = 8, split by head in the backward
         (8, 12, 4, 2048, 64, 300, False),  # the largest forward grid of these kernels
         (9, 12, 4, 2048, 64, 300, False),  # past it: another forward, the same backward
         (2, 4, 2, 333, 64, 60, True),  # rows without 16-byte alignment: register-staged

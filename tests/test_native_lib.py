@@ -6,6 +6,8 @@ import ctypes
 import re
 from pathlib import Path
 
+import pytest
+
 from packbalance_amd import _native as N
 
 ROOT = Path(__file__).resolve().parents[1]
@@ -127,3 +129,27 @@ def test_attention_kept_ds_config_on_host() -> None:
         c = attn_config(*shape)
         assert c["tiles"][2] == (128, 64) and c["workspace"] == (8 * shape[1] * shape[3] * 4), shape
 
+
+@pytest.mark.parametrize(
+    "shape,wave",
+    [
+        ((4, 12, 4, 2048, 64), True),
+        ((1, 20, 4, 4096, 64), True),
+        ((1, 64, 8, 4096, 64), True),  # no split by head there
+        ((2, 2, 2, 700, 40), True),  # nothing to split
+        ((1, 4, 1, 2048, 64), False),  # one KV head: too few walks to fill the GPU
+        ((1, 32, 2, 2048, 64), False),
+        ((1, 71, 1, 2048, 64), False),
+        ((8, 8, 1, 2048, 64), False),
+        ((6, 16, 16, 4096, 64), False),  # a full grid
+        ((12, 16, 16, 2048, 64), False),
+        ((1, 4, 4, 4097, 64), False),  # longer lists than a wave holds
+    ],
+)
+def test_attention_wave_backward_config_on_host(shape, wave) -> None:
+    """pb_attn_config: the backward's 32 x 32 tiles (a workgroup per KV tile and KV head,
+    query heads in turn) only with enough KV heads for the group."""
+    from packbalance_amd.model.attention import BWD_KV, BWD_Q, attn_config
+
+    t = attn_config(*shape)["tiles"]
+    assert (t[BWD_KV] == (32, 32)) == wave and (t[BWD_Q] == (32, 32)) == wave, t
