@@ -70,6 +70,41 @@ struct BwdArgs {
   int vec;
 };
 
+// Views that the wave kernels cannot take (rows that are not 16-byte aligned, or
+// too far apart for the DMA's offsets) are copied to dense [B][H][S][D] rows
+// first, outputs back afterwards: on 32 x 32 plans nothing else runs, and the
+// register-staged kernels with one wave per 32-row tile took up to twice as long
+// as on their own tiles.  Misaligned [4, 2048], 12 / 4 heads, D 64, one document,
+// us, register-staged on 64 x 64 tiles / on 32 x 32 / copied: forward 174 / 367 /
+// 74, backward 842 / 1350 / 174.
+struct RowCopies {
+  struct Item {
+    bf16_t *view, *dense;
+    int64_t sb, sh, ss;
+    int heads;
+  } c[5];
+  int n, B, S, D;
+  char *next;  // first free byte of the workspace
+
+  RowCopies(int b, int s, int d, void *ws) : n(0), B(b), S(s), D(d) {
+    next = reinterpret_cast<char *>((reinterpret_cast<uintptr_t>(ws) + 15) & ~(uintptr_t)15);
+  }
+  // Adds a view; returns its dense rows, whose strides it writes to sb, sh, ss.
+  bf16_t *add_at(char *at, const pb_bhsd &v, int heads, int64_t &sb, int64_t &sh, int64_t &ss) {
+    bf16_t *dense = reinterpret_cast<bf16_t *>(at);
+    c[n++] = {static_cast<bf16_t *>(v.data), dense, v.stride_b, v.stride_h, v.stride_s, heads};
+    ss = D;
+    sh = (int64_t)S * D;
+    sb = heads * sh;
+    next = at + B * sb * 2;
+    return dense;
+  }
+  bf16_t *add(const pb_bhsd &v, int heads, int64_t &sb, int64_t &sh, int64_t &ss) {
+    return add_at(next, v, heads, sb, sh, ss);
+  }
+};
+int launch_row_copies(const RowCopies &c, bool to_dense, hipStream_t st);
+
 // The wave kernels (AttnConfig::wave): forward, and dQ then dK/dV.
 int launch_fwd_wave(const FwdArgs &a, hipStream_t st);
 int launch_bwd_wave(const BwdArgs &a, hipStream_t st);

@@ -45,11 +45,10 @@ namespace attn {
 constexpr int kKvChunkSteps = 16;
 
 // ---------------------------------------------------------------- dK, dV
-// BM = query rows per plan tile.
-template <int DP, int WAVES, bool SPLIT, int BM>
+template <int DP, int WAVES, bool SPLIT>
 __global__ __launch_bounds__(64 * WAVES) void attn_bwd_dkdv(BwdArgs a) {
   constexpr int NT = 64 * WAVES;
-  constexpr int BN = 32 * WAVES;
+  constexpr int BN = 32 * WAVES, BM = kQStep;
   constexpr int QP = DP + 8;  // row-major pitch (elements)
   constexpr int NDK = DP / 16, NDB = DP / 32, CH = DP / 8;
   constexpr int NCH = BM * CH;             // 16-byte chunks of one [BM x DP] tile
@@ -152,10 +151,10 @@ __global__ __launch_bounds__(64 * WAVES) void attn_bwd_dkdv(BwdArgs a) {
     __syncthreads();
     if (step + 1 < steps) fetch(step + 1);
 
-    // S = Q K^T, dP = dO V^T: 32-query blocks x this wave's 32 KV rows.
-    bf16x8_t pf[BM / 16], dsf[BM / 16];
+    // S = Q K^T, dP = dO V^T: two 32-query blocks x this wave's 32 KV rows.
+    bf16x8_t pf[4], dsf[4];
 #pragma unroll
-    for (int qb = 0; qb < BM / 32; ++qb) {
+    for (int qb = 0; qb < 2; ++qb) {
       f32x16_t sacc = zero16(), pacc = zero16();
 #pragma unroll
       for (int dk = 0; dk < NDK; ++dk) {
@@ -177,7 +176,7 @@ __global__ __launch_bounds__(64 * WAVES) void attn_bwd_dkdv(BwdArgs a) {
 #pragma unroll
     for (int db = 0; db < NDB; ++db)
 #pragma unroll
-      for (int qk = 0; qk < BM / 16; ++qk) {
+      for (int qk = 0; qk < 4; ++qk) {
         dv_acc[db] = mfma32(pf[qk], lds_col_frag(Gs, QP, 16 * qk, 32 * db, lane), dv_acc[db]);
         dk_acc[db] = mfma32(dsf[qk], lds_col_frag(Qs, QP, 16 * qk, 32 * db, lane), dk_acc[db]);
       }
@@ -1123,11 +1122,10 @@ __global__ __launch_bounds__(256) void attn_bwd_reduce(BwdArgs a) {
 }
 
 // ---------------------------------------------------------------- dQ
-// BN = KV rows per plan tile.
-template <int DP, int WAVES, int BN>
+template <int DP, int WAVES>
 __device__ __forceinline__ void dq_body(const BwdArgs &a) {
   constexpr int NT = 64 * WAVES;
-  constexpr int BM = 32 * WAVES;
+  constexpr int BM = 32 * WAVES, BN = kKvStep;
   constexpr int KP = DP + 8;
   constexpr int NDK = DP / 16, NDB = DP / 32, CH = DP / 8;
   constexpr int NLD = BN * CH / NT;
@@ -1205,9 +1203,9 @@ __device__ __forceinline__ void dq_body(const BwdArgs &a) {
 
     const int kv0 = plan_tile(e) * BN;
     const bool full = plan_full(e);
-    bf16x8_t dsf[BN / 16];
+    bf16x8_t dsf[4];
 #pragma unroll
-    for (int blk = 0; blk < BN / 32; ++blk) {
+    for (int blk = 0; blk < 2; ++blk) {
       f32x16_t sacc = zero16(), pacc = zero16();
 #pragma unroll
       for (int dk = 0; dk < NDK; ++dk) {
@@ -1228,7 +1226,7 @@ __device__ __forceinline__ void dq_body(const BwdArgs &a) {
 #pragma unroll
     for (int db = 0; db < NDB; ++db)
 #pragma unroll
-      for (int kk = 0; kk < BN / 16; ++kk)
+      for (int kk = 0; kk < 4; ++kk)
         dq_acc[db] = mfma32(lds_col_frag(Ks, KP, 16 * kk, 32 * db, lane), dsf[kk], dq_acc[db]);
   }
   if (!qvalid) return;
@@ -1626,15 +1624,15 @@ __global__ __launch_bounds__(256) void attn_bwd_reduce_both(BwdArgs a, int bm, i
 
 // Two entry points over one body: two waves per SIMD (so one wave's softmax
 // overlaps the other's MFMAs) wherever the registers fit without spilling.
-template <int DP, int WAVES, int BN>
+template <int DP, int WAVES>
 __global__ __launch_bounds__(64 * WAVES) __attribute__((amdgpu_waves_per_eu(2, 2))) void
 attn_bwd_dq(BwdArgs a) {
-  dq_body<DP, WAVES, BN>(a);
+  dq_body<DP, WAVES>(a);
 }
 
 template <int DP, int WAVES>
 __global__ __launch_bounds__(64 * WAVES) void attn_bwd_dq_wide(BwdArgs a) {
-  dq_body<DP, WAVES, kKvStep>(a);
+  dq_body<DP, WAVES>(a);
 }
 
 // ---------------------------------------------------------------- kept-dS dQ
@@ -1932,12 +1930,9 @@ extern "C" int pb_attn_bwd(const pb_bhsd *q, const pb_bhsd *k, const pb_bhsd *v,
     if (DP == 128 && W == 2)                                                        \
       hipLaunchKernelGGL((attn_bwd_dq_wide<DP, W>), g_q, dim3(64 * W), 0, st, a);   \
     else                                                                            \
-      hipLaunchKernelGGL((attn_bwd_dq<DP, W, W == 1 ? 32 : kKvStep>), g_q, dim3(64 * W), 0, st, a);     \
+      hipLaunchKernelGGL((attn_bwd_dq<DP, W>), g_q, dim3(64 * W), 0, st, a);        \
   } while (0)
-#define PB_KV(DP, W, SP)                                                                    \
-  hipLaunchKernelGGL((attn_bwd_dkdv<DP, W, SP, W == 1 ? 32 : kQStep>), g_kv, dim3(64 * W), 0, st, a)
-#define PB_BY_D64(M, ...) \
-  do { if (d <= 32) M(32, __VA_ARGS__); else M(64, __VA_ARGS__); } while (0)
+#define PB_KV(DP, W, SP) hipLaunchKernelGGL((attn_bwd_dkdv<DP, W, SP>), g_kv, dim3(64 * W), 0, st, a)
 #define PB_BY_D(M, ...) \
   do { if (d <= 32) M(32, __VA_ARGS__); else if (d <= 64) M(64, __VA_ARGS__); else M(128, __VA_ARGS__); } while (0)
   // DMA-pipelined kernels where views, documents and the sequence length allow.
@@ -1948,7 +1943,22 @@ extern "C" int pb_attn_bwd(const pb_bhsd *q, const pb_bhsd *k, const pb_bhsd *v,
                     ((hq / hkv - 1) * std::max(q->stride_h, dout->stride_h) +
                      s * std::max(q->stride_s, dout->stride_s)) * 2 < (1LL << 31) &&
                     (hq / hkv) * s * 4 < (1LL << 31) && s * 8 < (1LL << 31);
-  if (pipe && cfg.wave_bwd) return launch_bwd_wave(a, st);
+  if (cfg.wave_bwd) {
+    if (pipe) return launch_bwd_wave(a, st);
+    RowCopies in(a.B, a.S, a.D, ws + delta_bytes), back(a.B, a.S, a.D, nullptr);
+    auto dense = [&](View &t, const pb_bhsd &view, int heads) {
+      t.p = in.add(view, heads, t.sb, t.sh, t.ss);
+    };
+    dense(a.q, *q, a.Hq);
+    dense(a.k, *k, a.Hkv);
+    dense(a.v, *v, a.Hkv);
+    dense(a.o, *out, a.Hq);
+    dense(a.dout, *dout, a.Hq);
+    a.dq.p = back.add_at(in.next, *dq, a.Hq, a.dq.sb, a.dq.sh, a.dq.ss);  // (dK, dV: scalar stores)
+    rc = launch_row_copies(in, true, st);
+    if (!rc) rc = launch_bwd_wave(a, st);
+    return rc ? rc : launch_row_copies(back, false, st);
+  }
   // The forms without bounds; every other length, head dim and alignment of
   // the documents and lse takes the GEN forms.
   const bool gen = !((d == 64 || d == 128) && s % 64 == 0 &&
@@ -1993,7 +2003,6 @@ extern "C" int pb_attn_bwd(const pb_bhsd *q, const pb_bhsd *k, const pb_bhsd *v,
     else { if (d > 64) PB_DQP(128, 2); else PB_DQP(64, 2); }
 #undef PB_DQP
   } else if (cfg.dq_waves == 4) PB_BY_D(PB_DQ, 4);
-  else if (cfg.dq_waves == 1) PB_BY_D64(PB_DQ, 1);  // the tiles of the wave kernels
   else PB_BY_D(PB_DQ, 2);
   rc = launch_status("pb_attn_bwd(dq)");
   if (rc) return rc;
@@ -2019,11 +2028,9 @@ extern "C" int pb_attn_bwd(const pb_bhsd *q, const pb_bhsd *k, const pb_bhsd *v,
     else { if (d > 64) PB_KVP(128, 2, false); else PB_KVP(64, 2, false); }
 #undef PB_KVP
   } else if (cfg.kv_waves == 4) PB_BY_D(PB_KV, 4, false);
-  else if (cfg.kv_waves == 1) PB_BY_D64(PB_KV, 1, false);
   else if (cfg.split) PB_BY_D(PB_KV, 2, true);
   else PB_BY_D(PB_KV, 2, false);
 #undef PB_BY_D
-#undef PB_BY_D64
 #undef PB_KV
 #undef PB_DQ
   rc = launch_status("pb_attn_bwd(dkdv)");

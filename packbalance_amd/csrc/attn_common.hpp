@@ -320,7 +320,7 @@ struct AttnConfig {
   int fwd_chunk, fwd_splits;  // 0 / 1: no forward KV split
   int dq_chunk, dq_splits;    // the same for the (q-major) dQ kernel
   // Head dims to 64 on small grids: the wave kernels (attn_wave.hip) on 32 x 32
-  // tiles.  Views they cannot take run the register-staged kernels on the same tiles.
+  // tiles.  Views they cannot take are copied first (RowCopies).
   int wave_fwd, wave_bwd;
   int fwd_kv_step() const { return wave_fwd ? 32 : kKvStep; }
   int dq_kv_step() const { return wave_bwd ? 32 : kKvStep; }
@@ -420,10 +420,12 @@ inline AttnConfig attn_config(int64_t b, int64_t hq, int64_t hkv, int64_t s, int
 }
 
 // Workspace of pb_attn_fwd: with a KV split, the partial outputs
-// [splits, b, hq, s, d] and log-sum-exps [splits, b, hq, s], fp32.
+// [splits, b, hq, s, d] and log-sum-exps [splits, b, hq, s], fp32; on the wave
+// kernels the dense copies of q, k, v and out (RowCopies, 16-byte aligned).
 inline int64_t attn_fwd_workspace(int64_t b, int64_t hq, int64_t hkv, int64_t s, int64_t d) {
   const AttnConfig c = attn_config(b, hq, hkv, s, d);
-  if (c.fwd_chunk == 0 || c.wave_fwd) return 0;
+  if (c.wave_fwd) return 2 * (hq + hkv) * b * s * d * 2 + 16;
+  if (c.fwd_chunk == 0) return 0;
   const int64_t rows = (int64_t)c.fwd_splits * b * hq * s;
   return (rows * d * 4 + 255) / 256 * 256 + (rows * 4 + 255) / 256 * 256;
 }
@@ -432,7 +434,8 @@ inline int64_t attn_fwd_workspace(int64_t b, int64_t hq, int64_t hkv, int64_t s,
 // partials [b, hq, s, d] fp32 each and a second such pair (the second halves
 // of long KV lists), then (dQ KV split) dQ partials [dq_splits, b, hq, s, d]
 // fp32; with kept dS (AttnConfig::ds, which excludes both splits) the dS
-// blocks follow delta.
+// blocks follow delta, on the wave kernels the dense copies of q, k, v, out,
+// dout and dq (RowCopies).
 inline int64_t attn_bwd_dq_part_offset(int64_t b, int64_t hq, int64_t s, int64_t d, bool split) {
   int64_t bytes = (b * hq * s * 4 + 255) / 256 * 256;
   // split: dK and dV partials, and a second pair for lists walked in two halves
@@ -443,6 +446,7 @@ inline int64_t attn_bwd_dq_part_offset(int64_t b, int64_t hq, int64_t s, int64_t
 inline int64_t attn_bwd_workspace(int64_t b, int64_t hq, int64_t hkv, int64_t s, int64_t d) {
   const AttnConfig c = attn_config(b, hq, hkv, s, d);
   int64_t bytes = attn_bwd_dq_part_offset(b, hq, s, d, c.split != 0);
+  if (c.wave_bwd) bytes += (4 * hq + 2 * hkv) * b * s * d * 2 + 16;
   if (c.ds) bytes += ds_bytes(b, hq, hkv, s);  // the kept dS blocks after delta
   if (c.dq_chunk) bytes += (int64_t)c.dq_splits * b * hq * s * d * 4;
   return bytes;

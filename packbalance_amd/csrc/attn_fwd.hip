@@ -38,11 +38,10 @@ namespace attn {
 
 // Generic path: any head dim <= 128, any strides / alignment (element-wise
 // loads where 16-byte access is not allowed), K/V staged through registers.
-// BN = KV rows per plan tile.
-template <int DP, int WAVES, int BN>
+template <int DP, int WAVES>
 __global__ __launch_bounds__(64 * WAVES) __attribute__((amdgpu_waves_per_eu(2, 2))) void attn_fwd_generic(FwdArgs a) {
   constexpr int NT = 64 * WAVES;
-  constexpr int BM = 32 * WAVES, NBLK = BN / 32;
+  constexpr int BM = 32 * WAVES, BN = kKvStep;
   constexpr int KP = DP + 8;  // K / V row pitch in LDS (elements)
   constexpr int NDK = DP / 16;
   constexpr int NDB = DP / 32;
@@ -117,10 +116,10 @@ __global__ __launch_bounds__(64 * WAVES) __attribute__((amdgpu_waves_per_eu(2, 2
     __syncthreads();
     if (it + 1 < cnt) fetch(lst[it + 1]);
 
-    // S^T = K Q^T for the 32-row blocks of the tile.
-    f32x16_t sacc[NBLK];
+    // S^T = K Q^T for the two 32-row halves of the tile.
+    f32x16_t sacc[2];
 #pragma unroll
-    for (int blk = 0; blk < NBLK; ++blk) {
+    for (int blk = 0; blk < 2; ++blk) {
       sacc[blk] = zero16();
 #pragma unroll
       for (int dk = 0; dk < NDK; ++dk) {
@@ -136,7 +135,7 @@ __global__ __launch_bounds__(64 * WAVES) __attribute__((amdgpu_waves_per_eu(2, 2
     float mloc = -INFINITY;
     if (!full) {
 #pragma unroll
-      for (int blk = 0; blk < NBLK; ++blk)
+      for (int blk = 0; blk < 2; ++blk)
 #pragma unroll
         for (int j = 0; j < 16; ++j) {
           const int kr_ = 32 * blk + 8 * (j >> 2) + 4 * hh + (j & 3);
@@ -146,7 +145,7 @@ __global__ __launch_bounds__(64 * WAVES) __attribute__((amdgpu_waves_per_eu(2, 2
         }
     }
 #pragma unroll
-    for (int blk = 0; blk < NBLK; ++blk)
+    for (int blk = 0; blk < 2; ++blk)
 #pragma unroll
       for (int j = 0; j < 16; ++j) mloc = fmaxf(mloc, sacc[blk][j]);
     mloc = fmaxf(mloc, __shfl_xor(mloc, 32)) * a.sl2;
@@ -160,9 +159,9 @@ __global__ __launch_bounds__(64 * WAVES) __attribute__((amdgpu_waves_per_eu(2, 2
 #pragma unroll
       for (int j = 0; j < 16; ++j) oacc[db][j] *= alpha;
 
-    bf16x8_t pf[2 * NBLK];
+    bf16x8_t pf[4];
 #pragma unroll
-    for (int blk = 0; blk < NBLK; ++blk)
+    for (int blk = 0; blk < 2; ++blk)
 #pragma unroll
       for (int j = 0; j < 16; ++j) {
         const float p = fast_exp2(fmaf(sacc[blk][j], a.sl2, -m_use));
@@ -175,7 +174,7 @@ __global__ __launch_bounds__(64 * WAVES) __attribute__((amdgpu_waves_per_eu(2, 2
 #pragma unroll
     for (int db = 0; db < NDB; ++db)
 #pragma unroll
-      for (int kk = 0; kk < 2 * NBLK; ++kk)
+      for (int kk = 0; kk < 4; ++kk)
         oacc[db] = mfma32(lds_col_frag(Vs, KP, 16 * kk, 32 * db, lane), pf[kk], oacc[db]);
   }
 
@@ -889,7 +888,19 @@ extern "C" int pb_attn_fwd(const pb_bhsd *q, const pb_bhsd *k, const pb_bhsd *v,
   const bool gen = !((d == 64 || d == 128) && s % 64 == 0 &&
                      (reinterpret_cast<uintptr_t>(doc_ids) & 15) == 0 && doc_stride % 2 == 0);
   a.tau = gen ? 0.f : 8.f;  // (as attn_fwd_pipe: GEN exact, else kTau)
-  if (pipe && cfg.wave_fwd) return launch_fwd_wave(a, st);
+  if (cfg.wave_fwd) {
+    if (pipe) return launch_fwd_wave(a, st);
+    PB_CHECK_ARG(workspace != nullptr,
+                 "pb_attn_fwd: workspace is required for views without 16-byte aligned rows");
+    RowCopies in(a.B, a.S, a.D, workspace), back(a.B, a.S, a.D, nullptr);
+    a.q = in.add(*q, a.Hq, a.q_sb, a.q_sh, a.q_ss);
+    a.k = in.add(*k, a.Hkv, a.k_sb, a.k_sh, a.k_ss);
+    a.v = in.add(*v, a.Hkv, a.v_sb, a.v_sh, a.v_ss);
+    a.o = back.add_at(in.next, *out, a.Hq, a.o_sb, a.o_sh, a.o_ss);
+    int rc = launch_row_copies(in, true, st);
+    if (!rc) rc = launch_fwd_wave(a, st);
+    return rc ? rc : launch_row_copies(back, false, st);
+  }
   if (pipe && cfg.fwd_chunk > 0) {
     PB_CHECK_ARG(workspace != nullptr, "pb_attn_fwd: workspace is required for this shape");
     a.chunk = cfg.fwd_chunk;
@@ -921,13 +932,10 @@ extern "C" int pb_attn_fwd(const pb_bhsd *q, const pb_bhsd *k, const pb_bhsd *v,
       else hipLaunchKernelGGL(attn_fwd_combine<0>, cgrid, dim3(256), 0, st, a);
     }
   } else {
-    // Generic kernel: 32 query rows per wave, same tiles as the plan.
+    // Generic kernel: 32 query rows per wave, same query tile as the plan.
     const int w = cfg.fwd_q_tile() / 32;
-#define PB_FWD(DP, W)                                                                          \
-  hipLaunchKernelGGL((attn_fwd_generic<DP, W, W == 1 ? 32 : kKvStep>), grid, dim3(64 * W), 0, st, a)
-    if (w == 1) {  // the tiles of attn_fwd_wave (d <= 64)
-      if (d <= 32) PB_FWD(32, 1); else PB_FWD(64, 1);
-    } else if (w == 4) {
+#define PB_FWD(DP, W) hipLaunchKernelGGL((attn_fwd_generic<DP, W>), grid, dim3(64 * W), 0, st, a)
+    if (w == 4) {
       if (d <= 32) PB_FWD(32, 4); else if (d <= 64) PB_FWD(64, 4); else PB_FWD(128, 4);
     } else {
       if (d <= 32) PB_FWD(32, 2); else if (d <= 64) PB_FWD(64, 2); else PB_FWD(128, 2);

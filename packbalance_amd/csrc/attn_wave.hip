@@ -597,7 +597,43 @@ void attn_bwd_dkdv_wave(BwdArgs a) {
   }
 }
 
+// A thread moves eight elements of a row.
+template <bool TO_DENSE>
+__global__ __launch_bounds__(256) void copy_rows(RowCopies a) {
+  const RowCopies::Item &c = a.c[blockIdx.y];
+  const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  const int chunks = a.D / 8;
+  int64_t r = i / chunks;
+  const int x = (int)(i - r * chunks) * 8;
+  if (r >= (int64_t)a.B * c.heads * a.S) return;
+  const int s = (int)(r % a.S);
+  r /= a.S;
+  const int h = (int)(r % c.heads), b = (int)(r / c.heads);
+  bf16_t *p = c.view + b * c.sb + h * c.sh + s * c.ss + x;
+  bf16x8_t *d = reinterpret_cast<bf16x8_t *>(c.dense + 8 * i);
+  bf16x8_t v;
+  if constexpr (TO_DENSE) {
+#pragma unroll
+    for (int j = 0; j < 8; ++j) v[j] = p[j];
+    *d = v;
+  } else {
+    v = *d;
+#pragma unroll
+    for (int j = 0; j < 8; ++j) p[j] = v[j];
+  }
+}
+
 }  // namespace
+
+int launch_row_copies(const RowCopies &c, bool to_dense, hipStream_t st) {
+  int heads = 0;
+  for (int i = 0; i < c.n; ++i) heads = c.c[i].heads > heads ? c.c[i].heads : heads;
+  const int64_t n = (int64_t)c.B * heads * c.S * (c.D / 8);
+  const dim3 g((unsigned)((n + 255) / 256), (unsigned)c.n);
+  if (to_dense) hipLaunchKernelGGL(copy_rows<true>, g, dim3(256), 0, st, c);
+  else hipLaunchKernelGGL(copy_rows<false>, g, dim3(256), 0, st, c);
+  return launch_status("pb_attn(row copies)");
+}
 
 int launch_fwd_wave(const FwdArgs &a, hipStream_t st) {
   const int tiles = a.nqt * a.B * a.Hq;

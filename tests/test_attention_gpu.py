@@ -310,8 +310,10 @@ def test_exact_max_of_peaked_scores(dense, B, Hq, Hkv, S, D, dev) -> None:
         (5, 8, 1, 777, 64, 90, False),  # G = 8, split by head in the backward
         (8, 12, 4, 2048, 64, 300, False),  # the largest forward grid of these kernels
         (9, 12, 4, 2048, 64, 300, False),  # past it: another forward, the same backward
-        (2, 4, 2, 333, 64, 60, True),  # rows without 16-byte alignment: register-staged
+        (2, 4, 2, 333, 64, 60, True),  # rows without 16-byte alignment: copied first
         (2, 4, 2, 333, 32, 60, True),
+        (4, 12, 4, 1999, 40, 300, True),
+        (1, 32, 2, 1024, 64, 300, True),  # register-staged in the backward
     ],
 )
 def test_small_grid_matches_padded_head_dim(B, Hq, Hkv, S, D, mu, misaligned, dev) -> None:
