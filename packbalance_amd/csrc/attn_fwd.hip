@@ -883,13 +883,18 @@ extern "C" int pb_attn_fwd(const pb_bhsd *q, const pb_bhsd *k, const pb_bhsd *v,
   hipStream_t st = as_stream(stream);
   // DMA offsets are 32-bit: one (pack, KV head) view of K / V (S rows) and
   // the pack's document ids must span < 2 GiB.
-  const bool pipe = a.vec && s * std::max(k->stride_s, v->stride_s) * 2 < (1LL << 31) &&
-                    s * 8 < (1LL << 31);
+  const bool dma = a.vec && s * std::max(k->stride_s, v->stride_s) * 2 < (1LL << 31) &&
+                   s * 8 < (1LL << 31);
+  // Head dim 32, padded to 64 in the pipeline, is the one that the register-staged
+  // kernel is instantiated for: it keeps the larger grids (one document, us, staged /
+  // pipeline: [8, 8192], 12 / 4 heads 1007 / 1044, [1, 8192] 137 / 163; documents of
+  // about 500 350 / 282).  From head dim 24 down the pipeline wins (1212 / 1035).
+  const bool pipe = dma && d != 32;
   const bool gen = !((d == 64 || d == 128) && s % 64 == 0 &&
                      (reinterpret_cast<uintptr_t>(doc_ids) & 15) == 0 && doc_stride % 2 == 0);
   a.tau = gen ? 0.f : 8.f;  // (as attn_fwd_pipe: GEN exact, else kTau)
   if (cfg.wave_fwd) {
-    if (pipe) return launch_fwd_wave(a, st);
+    if (dma) return launch_fwd_wave(a, st);
     PB_CHECK_ARG(workspace != nullptr,
                  "pb_attn_fwd: workspace is required for views without 16-byte aligned rows");
     RowCopies in(a.B, a.S, a.D, workspace), back(a.B, a.S, a.D, nullptr);
