@@ -52,8 +52,9 @@ typedef __bf16 bf16x2_t __attribute__((ext_vector_type(2)));
 typedef __bf16 bf16x4_t __attribute__((ext_vector_type(4)));
 typedef float f32x4_t __attribute__((ext_vector_type(4)));
 
-// Wave w's part [i0, i1) of n >= 1 steps: at most NW waves of at least
-// LEAST steps (all but the first wave cost a prologue and a merge).
+// Wave w's part [i0, i1) of n steps: at most NW waves of at least LEAST steps
+// (all but the first wave cost a prologue and a merge).  pb_attn_plan leaves no
+// list empty, but a caller's plan may: the first wave then has no step.
 // Returns the number of waves that have a share.
 template <int NW, int LEAST = kWaveLeast>
 __device__ __forceinline__ int wave_share(int n, int w, int &i0, int &i1) {
@@ -189,7 +190,7 @@ void attn_fwd_wave(FwdArgs a) {
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   int qt, b, h;
   decode_q_major((int)blockIdx.x, a.nqt, a.B, a.Hq, a.Hkv, qt, b, h);
-  const int n = a.cnt[b * a.nqt + qt];  // >= 1: every row sees itself
+  const int n = a.cnt[b * a.nqt + qt];
   int i0, i1;
   const int nw = wave_share<NW, LEAST>(n, wave, i0, i1);
   if (wave >= nw) return;
@@ -197,7 +198,7 @@ void attn_fwd_wave(FwdArgs a) {
   const int S = a.S, hk = h / (a.Hq / a.Hkv);
   const float sl2 = a.sl2;
   const int32_t *lst = a.list + ((int64_t)b * a.nqt + qt) * a.nkt + i0;
-  const int ev = lst[min(lane, m - 1)];
+  const int ev = lst[max(min(lane, m - 1), 0)];
   auto entry = [&](int i) { return __builtin_amdgcn_readlane(ev, min(i, m - 1)); };
   const auto krs = buf_rsrc(a.k + b * a.k_sb + hk * a.k_sh, 0x7fffffff);
   const auto vrs = buf_rsrc(a.v + b * a.v_sb + hk * a.v_sh, 0x7fffffff);
@@ -271,7 +272,7 @@ void attn_fwd_wave(FwdArgs a) {
 #pragma unroll
       for (int db = 0; db < NDB; ++db) oacc[db] = mfma32(fo.cfrag(vt, kk, db), pf[kk], oacc[db]);
   };
-  fetch(0, v0, kd0[wave]);
+  if (m > 0) fetch(0, v0, kd0[wave]);
   int i = 0;
   for (; i + 2 <= m; i += 2) {
     step(i, v0, kd0[wave], v1, kd1[wave]);
@@ -332,7 +333,7 @@ void attn_bwd_dq_wave(BwdArgs a) {
   const int S = a.S, hk = h / (a.Hq / a.Hkv);
   const float sl2 = a.sl2;
   const int32_t *lst = a.qlist + ((int64_t)b * a.nqt_dq + qt) * a.nkt_dq + i0;
-  const int ev = lst[min(lane, m - 1)];
+  const int ev = lst[max(min(lane, m - 1), 0)];
   auto entry = [&](int i) { return __builtin_amdgcn_readlane(ev, min(i, m - 1)); };
   const auto krs = buf_rsrc(a.k.row(b, hk, 0), 0x7fffffff);
   const auto vrs = buf_rsrc(a.v.row(b, hk, 0), 0x7fffffff);
@@ -397,7 +398,7 @@ void attn_bwd_dq_wave(BwdArgs a) {
 #pragma unroll
       for (int db = 0; db < NDB; ++db) acc[db] = mfma32(fo.cfrag(kt, kk, db), ds[kk], acc[db]);
   };
-  fetch(0, k0, kd0[wave]);
+  if (m > 0) fetch(0, k0, kd0[wave]);
   int i = 0;
   for (; i + 2 <= m; i += 2) {
     step(i, k0, kd0[wave], k1, kd1[wave]);
@@ -447,7 +448,7 @@ void attn_bwd_dkdv_wave(BwdArgs a) {
     pair = (int)blockIdx.x - kt * npairs;
   }
   const int b = pair / a.Hkv, hk = pair - b * a.Hkv;
-  const int cnt = a.kcnt[b * a.nkt_kv + kt];  // >= 1
+  const int cnt = a.kcnt[b * a.nkt_kv + kt];
   int t0, t1;
   const int nw = wave_share<NW>(cnt * G, wave, t0, t1);
   if (wave >= nw) return;
@@ -456,7 +457,8 @@ void attn_bwd_dkdv_wave(BwdArgs a) {
   // This wave's query tiles: list entries u0 .. (at most 128 of them).
   const int u0 = t0 / G;
   const int32_t *lst = a.klist + ((int64_t)b * a.nkt_kv + kt) * a.nqt_kv;
-  const int ev0 = lst[min(u0 + lane, cnt - 1)], ev1 = lst[min(u0 + 64 + lane, cnt - 1)];
+  const int ev0 = lst[max(min(u0 + lane, cnt - 1), 0)];
+  const int ev1 = lst[max(min(u0 + 64 + lane, cnt - 1), 0)];
   auto entry = [&](int i) { return __builtin_amdgcn_readlane(i < 64 ? ev0 : ev1, i & 63); };
   const int h0 = hk * G;
   const auto qrs = buf_rsrc(a.q.row(b, h0, 0), 0x7fffffff);
@@ -545,7 +547,7 @@ void attn_bwd_dkdv_wave(BwdArgs a) {
   };
   char *q0 = qs0[wave], *q1 = qs1[wave], *g0 = gs0[wave], *g1 = gs1[wave];
   const int m = t1 - t0;
-  fetch(q0, g0, ld0[wave], qd0[wave]);
+  if (m > 0) fetch(q0, g0, ld0[wave], qd0[wave]);
   int i = 0;
   for (; i + 2 <= m; i += 2) {
     fetch(q1, g1, ld1[wave], qd1[wave]);

@@ -568,3 +568,33 @@ def test_kept_ds_backward_graph_replays(dev) -> None:
         for name, got, w in zip(("dq", "dk", "dv"), outs[:3], want):
             assert torch.equal(got, w), f"replay {rep}: {name} differs from the eager call"
         _ = (q.float() * 2).sum().item()  # eager work between replays
+
+
+@pytest.mark.parametrize("D", [64, 128])
+def test_empty_plan_rows(D, dev) -> None:
+    """A caller's plan may leave a tile's list empty (pb_attn_plan never does): the rows of
+    that query tile get zero outputs, lse -inf and zero dQ, the KV rows zero dK and dV, and
+    the other tiles what they get with the full plan, on the 32 x 32 tiles of head dim 64 as
+    on the workgroup kernels."""
+    from packbalance_amd.model import attention as A
+
+    B, Hq, Hkv, S = 1, 4, 4, 512
+    doc = W.doc_ids_from_lengths([[300, 212]], S).to(dev)
+    q, k, v, do = _inputs(B, Hq, Hkv, S, D, dev, seed=5)
+    full, _ = _fwd_abi(q, k, v, doc)
+    mask = A.DocPlans(doc)
+    plans = A._plans(mask.doc_ids, Hq, Hkv, D, mask)
+    qt, kt = A.attn_config(B, Hq, Hkv, S, D)["tiles"][A.FWD][0], plans[A.BWD_KV].kv_tile
+    assert qt == plans[A.BWD_Q].q_tile and (qt == 32) == (D == 64)
+    for p in {id(p): p for p in (plans[A.FWD], plans[A.BWD_Q])}.values():
+        p.counts[0, 1] = 0
+    plans[A.BWD_KV].counts[0, 2] = 0
+    qr, kr, vr = (t.detach().requires_grad_(True) for t in (q, k, v))
+    out = doc_attention(qr, kr, vr, mask.doc_ids, block_mask=mask)
+    out.backward(do)
+    rows = torch.zeros(S, dtype=torch.bool, device=dev)
+    rows[qt:2 * qt] = True
+    assert (out[:, :, rows] == 0).all() and torch.equal(out[:, :, ~rows], full[:, :, ~rows])
+    assert torch.isfinite(out.float()).all()
+    assert (kr.grad[:, :, 2 * kt:3 * kt] == 0).all() and (vr.grad[:, :, 2 * kt:3 * kt] == 0).all()
+    assert (qr.grad[:, :, rows] == 0).all() and (qr.grad[:, :, ~rows] != 0).any()
