@@ -906,7 +906,9 @@ extern "C" int pb_attn_fwd(const pb_bhsd *q, const pb_bhsd *k, const pb_bhsd *v,
     if (!rc) rc = launch_fwd_wave(a, st);
     return rc ? rc : launch_row_copies(back, false, st);
   }
-  if (pipe && cfg.fwd_chunk > 0) {
+  // (The bounded form walks whole lists without a workspace, as the register-staged
+  // kernel that took its shapes did.)
+  if (pipe && cfg.fwd_chunk > 0 && (workspace || !gen)) {
     PB_CHECK_ARG(workspace != nullptr, "pb_attn_fwd: workspace is required for this shape");
     a.chunk = cfg.fwd_chunk;
     const int64_t prow = (int64_t)cfg.fwd_splits * b * hq * s;

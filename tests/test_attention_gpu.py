@@ -598,3 +598,26 @@ def test_empty_plan_rows(D, dev) -> None:
     assert torch.isfinite(out.float()).all()
     assert (kr.grad[:, :, 2 * kt:3 * kt] == 0).all() and (vr.grad[:, :, 2 * kt:3 * kt] == 0).all()
     assert (qr.grad[:, :, rows] == 0).all() and (qr.grad[:, :, ~rows] != 0).any()
+
+
+@pytest.mark.parametrize("S,D", [(801, 128), (1472, 96), (4200, 40)])
+def test_forward_without_workspace(S, D, dev) -> None:
+    """Lengths and head dims of the bounded forward need no workspace: without one a list is
+    not cut into chunks.  Either way rounds P and the output to bf16 once, so the two differ
+    by at most two such roundings (2 x 2^-9 in the 2-norm)."""
+    from packbalance_amd import _native as N
+    from packbalance_amd.model import attention as A
+
+    B, Hq, Hkv = 1, 4, 2
+    doc = W.doc_ids_from_lengths([[S - 100, 100]], S).to(dev)
+    q, k, v, _ = _inputs(B, Hq, Hkv, S, D, dev, seed=6)
+    want, want_lse = _fwd_abi(q, k, v, doc)
+    plans = A._plans(doc, Hq, Hkv, D, None)
+    assert plans["fwd_workspace"] > 0 and A.attn_config(B, Hq, Hkv, S, D)["fwd_chunk"] > 0
+    out, lse = torch.empty_like(want), torch.empty_like(want_lse)
+    p = plans[A.FWD]
+    N.call("pb_attn_fwd", N.BHSD.of(q), N.BHSD.of(k), N.BHSD.of(v), N.BHSD.of(out),
+           lse.data_ptr(), None, doc.data_ptr(), doc.stride(0), p.counts.data_ptr(),
+           p.lists.data_ptr(), B, Hq, Hkv, S, D, 1.0 / math.sqrt(D), N.PB_BF16, N.stream_ptr(q))
+    assert (out.double() - want.double()).norm() <= 2 ** -8 * want.double().norm()
+    torch.testing.assert_close(lse, want_lse, atol=1e-4, rtol=0)
