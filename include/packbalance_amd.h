@@ -174,11 +174,11 @@ typedef struct pb_bhsd {
 /* Launch configuration of the attention kernels for one problem shape (no
  * reference counterpart).  out[0..9] = forward query tile, forward KV tile,
  * dK/dV query tile, dK/dV KV tile, dQ query tile, dQ KV tile, pb_attn_bwd
- * workspace bytes, dK/dV split flag (a KV tile's work is shared by several
- * workgroups or waves), pb_attn_fwd workspace bytes, forward KV chunk (KV
- * tiles of a list before another workgroup or wave shares it; 0 = whole
- * lists).  Plans passed to pb_attn_fwd / pb_attn_bwd must be built with these
- * tile sizes.                                                               */
+ * workspace bytes, dK/dV head-split flag, pb_attn_fwd workspace bytes,
+ * forward KV chunk (KV tiles per workgroup; 0 = whole lists).  32 x 32 tiles
+ * name the kernels that share a list among the waves of one workgroup: there
+ * the flag and the chunk are 0.  Plans passed to pb_attn_fwd / pb_attn_bwd must
+ * be built with these tile sizes.                                           */
 int pb_attn_config(int64_t b, int64_t hq, int64_t hkv, int64_t s, int64_t d, int64_t *out);
 
 /* Tile plan of a packed batch (no counterpart table in the reference; it is

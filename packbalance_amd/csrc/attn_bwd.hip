@@ -1868,7 +1868,7 @@ extern "C" int pb_attn_config(int64_t b, int64_t hq, int64_t hkv, int64_t s, int
   out[4] = c.dq_q_tile();
   out[5] = c.dq_kv_step();
   out[6] = attn_bwd_workspace(b, hq, hkv, s, d);
-  out[7] = c.split || c.wave_bwd;
+  out[7] = c.split;
   out[8] = attn_fwd_workspace(b, hq, hkv, s, d);
   out[9] = c.fwd_chunk;
   return PB_OK;

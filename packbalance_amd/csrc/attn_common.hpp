@@ -352,7 +352,6 @@ struct AttnConfig {
 // 919 -> 619), up to as many tiles, times their length, as
 //   [4, 4096], 16 / 8 583 -> 601 and [3, 4096], 16 / 16 453 -> 454 (187 -> 137 with
 //   short documents), but [6, 4096], 16 / 16 849 -> 919; [12, 2048] 492 -> 530
-constexpr int kWaveLeast = 6;  // least steps of a list worth another wave
 constexpr int64_t kWaveMaxS = 4096;
 inline int64_t wave_tiles(int64_t b, int64_t hq, int64_t s, int64_t d) {
   if (d > 64 || d % 8 || s > kWaveMaxS) return INT64_MAX;
@@ -410,10 +409,8 @@ inline AttnConfig attn_config(int64_t b, int64_t hq, int64_t hkv, int64_t s, int
       splits_out = (int)((nkt + chunk - 1) / chunk);
     }
   };
-  c.fwd_chunk = kWaveLeast;  // (KV tiles of a list before a second wave shares it)
-  c.fwd_splits = 1;
-  c.dq_chunk = 0;
-  c.dq_splits = 1;
+  c.fwd_chunk = c.dq_chunk = 0;
+  c.fwd_splits = c.dq_splits = 1;
   if (!c.wave_fwd) kv_split(c.fwd_q_tile(), c.fwd_chunk, c.fwd_splits);
   if (!c.wave_bwd) kv_split(c.dq_q_tile(), c.dq_chunk, c.dq_splits);
   return c;

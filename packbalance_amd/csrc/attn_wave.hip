@@ -44,6 +44,7 @@ namespace {
 // 12 heads 22.5 -> 17.1 (30.3); at 1152 tiles ([1, 3072], 12 heads, documents of
 // about 100) 14.1 -> 15.3.
 constexpr int kFewQ = 768;
+constexpr int kWaveLeast = 6;  // (four waves of the forward and dQ: 4)
 constexpr int kTB = 32 * 64 * 2;   // bytes of one 32 x 64 bf16 tile
 constexpr int NDK = 4, NDB = 2;    // 16-wide k steps and 32-wide blocks of the head dim
 using Dma = TileDma<64, 32, 64>;   // one wave copies a tile: four 1 KiB instructions

@@ -216,10 +216,10 @@ def test_benchmarked_cfg2_step_graph_matches_eager(dev) -> None:
     """The step exactly as bench.py times it -- cfg2 (100M, [2, 2048] micro-batches on
     2 streams, packs built on the device, captured and replayed as one HIP graph) --
     against an eager twin of the same configuration over four replays (loss sum
-    and pre-clip gradient norm to 1e-3).  At this shape the attention takes its
-    split-KV forward / dQ and the dK/dV head split, and the LM head its split-K
-    dx, none of which the cfg1 tests reach.  The embedding backward adds rows
-    with atomics, so the twins differ by fp32 summation order; AdamW's
+    and pre-clip gradient norm to 1e-3).  At this shape the attention runs on 32 x 32
+    tiles, its lists shared by two waves in the forward and dQ and four in dK/dV,
+    and the LM head takes its split-K dx, none of which the cfg1 tests reach.  The
+    embedding backward adds rows with atomics, so the twins differ by fp32 summation order; AdamW's
     sign-like early updates amplify that from step to step (at lr 3e-4 the
     gradient norms drifted 4e-4, 7e-4, 1.5e-3 apart over replays 2-4), so the
     twins train at lr 3e-5 here -- every kernel, the optimizer state and the
@@ -229,7 +229,7 @@ def test_benchmarked_cfg2_step_graph_matches_eager(dev) -> None:
 
     cfg = cfg2_model()
     cfgs = A.attn_config(2, cfg.n_heads, cfg.n_kv_heads, 2048, cfg.head_dim)
-    assert cfgs["split"] and cfgs["fwd_chunk"] > 0  # the small-grid branches are exercised
+    assert set(cfgs["tiles"].values()) == {(32, 32)} and not cfgs["split"]
     plan, store, tables = _cfg2_store(cfg, dev, 5)
     eager = TrainStep(cfg, dev, store=store, streams=2, packs_per_micro_batch=2, lr=3e-5)
     graph = TrainStep(cfg, dev, store=store, streams=2, packs_per_micro_batch=2, lr=3e-5)

@@ -149,7 +149,11 @@ def test_attention_kept_ds_config_on_host() -> None:
 def test_attention_wave_backward_config_on_host(shape, wave) -> None:
     """pb_attn_config: the backward's 32 x 32 tiles (a workgroup per KV tile and KV head,
     query heads in turn) only with enough KV heads for the group."""
-    from packbalance_amd.model.attention import BWD_KV, BWD_Q, attn_config
+    from packbalance_amd.model.attention import BWD_KV, BWD_Q, FWD, attn_config
 
-    t = attn_config(*shape)["tiles"]
+    c = attn_config(*shape)
+    t = c["tiles"]
     assert (t[BWD_KV] == (32, 32)) == wave and (t[BWD_Q] == (32, 32)) == wave, t
+    b, hq, hkv, s, _ = shape
+    split = not wave and hq > hkv and b * hkv * -(-s // 64) < 512
+    assert c["split"] == split and (t[FWD] != (32, 32) or c["fwd_chunk"] == 0), c
