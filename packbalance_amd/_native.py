@@ -241,10 +241,16 @@ def require_device(*tensors: torch.Tensor, op: str) -> None:
     lib()
 
 
+# The current stream's handle without a Stream object, which costs 4 us of a call's host
+# time.  Not a public entry of torch: absent, the Stream object is made.
+_raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+
+
 def stream_ptr(t: torch.Tensor) -> int:
-    """The current stream of t's device (its handle, without a Stream object: that costs
-    4 us of a call's host time)."""
-    return torch._C._cuda_getCurrentRawStream(t.device.index)
+    """The handle of the current stream of t's device."""
+    if _raw_stream is None:
+        return torch.cuda.current_stream(t.device).cuda_stream
+    return _raw_stream(t.device.index)
 
 
 def ptr(t: torch.Tensor | None) -> int | None:

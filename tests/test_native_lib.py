@@ -5,8 +5,10 @@ from __future__ import annotations
 import ctypes
 import re
 from pathlib import Path
+from types import SimpleNamespace
 
 import pytest
+import torch
 
 from packbalance_amd import _native as N
 
@@ -157,3 +159,14 @@ def test_attention_wave_backward_config_on_host(shape, wave) -> None:
     b, hq, hkv, s, _ = shape
     split = not wave and hq > hkv and b * hkv * -(-s // 64) < 512
     assert c["split"] == split and (t[FWD] != (32, 32) or c["fwd_chunk"] == 0), c
+
+
+def test_stream_ptr_without_the_raw_getter(monkeypatch) -> None:
+    """torch builds without the private stream getter take the public one."""
+    t = SimpleNamespace(device=torch.device("cuda", 1))
+    monkeypatch.setattr(N, "_raw_stream", None)
+    monkeypatch.setattr(torch.cuda, "current_stream",
+                        lambda d: SimpleNamespace(cuda_stream=100 + d.index))
+    assert N.stream_ptr(t) == 101
+    monkeypatch.setattr(N, "_raw_stream", lambda index: 200 + index)
+    assert N.stream_ptr(t) == 201
