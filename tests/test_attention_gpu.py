@@ -93,12 +93,12 @@ def test_reference_flex_test_case(dev) -> None:
         (3, 4, 4, 130, 100, [64, 66]),  # head dim not a multiple of 16
         (1, 4, 2, 130, 100, [64, 66]),  # split dK/dV, element-wise reduce (D % 8 != 0)
         (1, 8, 2, 1024, 128, [300, 1, 400, -323]),  # pipelined path, 32 query rows per wave
-        (2, 16, 4, 2048, 64, "cfg2"),  # pipelined path, 64 query rows per wave, D 64
+        (2, 16, 4, 2048, 64, "cfg2"),  # 32 x 32 tiles, lists shared by two and four waves
+        (1, 12, 4, 2048, 64, [2048]),  # one dense document: lists of up to 64 tiles
+        (2, 6, 2, 1536, 64, [1000, 536]),
         # head-split dK/dV with KV lists of >= 16 steps (kKvChunkSteps) walked
         # as two halves:
-        (1, 12, 4, 2048, 64, [2048]),  # one dense document (64-step lists)
-        (1, 8, 2, 2048, 128, [1100, -948]),  # D 128, a long document then padding
-        (2, 6, 2, 1536, 64, [1000, 536]),  # two packs, both documents over the threshold
+        (1, 8, 2, 2048, 128, [1100, -948]),  # a long document then padding
         # the threshold itself: the 512-token document's first KV tile has a
         # 16-step list (two halves), every other tile 14 steps or fewer (whole)
         (1, 8, 2, 1024, 64, [512, 448, -64]),
@@ -109,7 +109,7 @@ def test_reference_flex_test_case(dev) -> None:
         (2, 3, 1, 95, 128, [90, -5]),
         (1, 4, 4, 97, 96, [33, 64]),
         (2, 6, 2, 191, 40, [100, 91]),
-        (1, 12, 4, 1999, 64, [1200, 300, 499]),  # split lists of a ragged length
+        (1, 12, 4, 1999, 64, [1200, 300, 499]),  # shared lists of a ragged length
     ],
 )
 def test_attention_matches_oracle(B, Hq, Hkv, S, D, docs, dev) -> None:
@@ -198,9 +198,9 @@ def test_attention_deterministic(dev) -> None:
         (9, 32, 8, 1087, 96),  # the same, head dim padded, one row short of a tile
         (10, 16, 8, 1056, 128),  # paired dK/dV without kept dS, a sub-tile wholly past the end
         (9, 12, 12, 639, 72),
-        (12, 24, 8, 1000, 64),  # four-wave kernels at head dim 64
-        (3, 12, 4, 2047, 56),  # the smaller grids: lists in chunks
-        (1, 9, 3, 1350, 64),  # dK/dV split by head, long lists in two halves
+        (12, 24, 8, 1000, 64),  # head dim 64: 128-row query tiles, the backward on 32 x 32
+        (3, 12, 4, 2047, 56),  # 32 x 32 tiles in both
+        (1, 9, 3, 1350, 64),
         (1, 4, 1, 801, 120),
     ],
 )
@@ -292,6 +292,60 @@ def test_exact_max_of_peaked_scores(dense, B, Hq, Hkv, S, D, dev) -> None:
     ref = OA.attention(q[:1, G:2 * G], k[:1, 1:2], v[:1, 1:2], doc[:1].cpu(), do[:1, G:2 * G])["out"]
     err = float((out[:1, G:2 * G].cpu().double() - ref).norm() / ref.norm())
     assert err <= 1.85e-3, f"{err:.2e}"
+
+
+@pytest.mark.parametrize(
+    "B,Hq,Hkv,S,D,misaligned,kv_tile,split",
+    [
+        (1, 4, 2, 4160, 64, False, 64, True),  # whole tiles: lists in chunks, heads split
+        (1, 4, 2, 4161, 64, False, 64, True),  # the same with bounds
+        (1, 6, 2, 4200, 40, False, 64, True),
+        (1, 4, 1, 4100, 24, False, 64, True),
+        (1, 4, 1, 4100, 32, False, 64, True),  # (the forward register-staged)
+        (1, 16, 1, 1024, 64, False, 64, True),  # one KV head of a short sequence
+        (1, 16, 1, 1023, 48, False, 64, True),
+        (1, 8, 8, 4160, 64, False, 64, False),  # two waves a KV tile, whole lists
+        (1, 8, 8, 4133, 56, False, 64, False),
+        (2, 8, 8, 4160, 64, False, 128, False),  # four
+        (2, 8, 8, 4161, 64, False, 128, False),
+        (1, 4, 2, 4161, 64, True, 64, True),  # rows without 16-byte alignment
+        (1, 8, 8, 4133, 32, True, 64, False),
+        (2, 8, 8, 4161, 48, True, 128, False),
+    ],
+)
+def test_workgroup_kernels_to_head_dim_64(B, Hq, Hkv, S, D, misaligned, kv_tile, split, dev) -> None:
+    """Head dims to 64 past the 32 x 32 tiles' grids, in every form that serves them: the
+    tiles and the head split that pb_attn_config names, and all four results of one KV head
+    against the oracle.  Outputs and gradients round bf16 values at most twice (P or dS, and
+    the result; 1.66e-3 of the 2-norm each), dQ and dK see O's rounding through delta too:
+    within 2^-8.5."""
+    from packbalance_amd.model import attention as A
+
+    c = A.attn_config(B, Hq, Hkv, S, D)
+    assert c["tiles"][A.BWD_KV] == (64, kv_tile) and c["tiles"][A.BWD_Q][1] == 64
+    assert c["split"] == split
+    if S > 4096:
+        assert c["tiles"][A.FWD][1] == 64 and c["fwd_chunk"] > 0
+    packs = [W.fill_sequential(np.random.default_rng(S + b), S, np.log(700), 1.0, 1, S)
+             for b in range(B)]
+    doc = W.doc_ids_from_lengths(packs, S).to(dev)
+    q, k, v, do = _inputs(B, Hq, Hkv, S, D, dev, seed=S + Hq)
+    if misaligned:
+        def odd(t):
+            mem = torch.zeros(B, S, t.shape[1], D + 1, dtype=t.dtype, device=dev)
+            mem[..., :D] = t.transpose(1, 2)
+            return mem[..., :D].transpose(1, 2)
+
+        q, k, v, do = odd(q), odd(k), odd(v), odd(do)
+    got = _run(q, k, v, do, doc)
+    b, g, G = B - 1, Hkv - 1, Hq // Hkv
+    sl, hs, ks = slice(b, b + 1), slice(G * g, G * (g + 1)), slice(g, g + 1)
+    ref = OA.attention(q[sl, hs], k[sl, ks], v[sl, ks], doc[sl].cpu(), do[sl, hs])
+    for name, t in zip(("out", "dq", "dk", "dv"), got):
+        want = ref[name]
+        err = float((t[sl, hs if name in ("out", "dq") else ks].detach().cpu().double()
+                     - want).norm() / want.norm())
+        assert err <= 2 ** -8.5, f"{name}: {err:.2e}"
 
 
 @pytest.mark.parametrize(
@@ -441,15 +495,16 @@ def test_attention_kept_ds_two_quads_per_kv_head(dev) -> None:
     assert torch.isfinite(dq.float()).all()
 
 
-@pytest.mark.parametrize("D", [64, 128])
+@pytest.mark.parametrize("S,D", [(1024, 64), (1024, 128), (4160, 64)])
 @pytest.mark.parametrize("profile", ["rising", "falling"])
-def test_attention_running_max_moves(profile, D, dev) -> None:
+def test_attention_running_max_moves(profile, S, D, dev) -> None:
     """Scores that rise along the sequence (the forward's running max moves
     every few sub-tiles, by up to ~40 log2 units, taking the rescaling slow
     path) or fall (the first valid sub-tile holds the max, every later one
     takes the fast path), with documents that leave some lanes' first
-    sub-tiles fully masked, on the pipelined kernels (S % 64 == 0)."""
-    B, Hq, Hkv, S = 1, 4, 2, 1024
+    sub-tiles fully masked: on 32 x 32 tiles (head dim 64, short sequences) and on
+    the pipelined kernels."""
+    B, Hq, Hkv = 1, 4, 2
     g = torch.Generator().manual_seed(31 + D)
     pos = torch.arange(S, dtype=torch.float32) / S
     ramp = 6.0 * (pos if profile == "rising" else 1.0 - pos)
@@ -458,7 +513,7 @@ def test_attention_running_max_moves(profile, D, dev) -> None:
     v = torch.randn(B, S, Hkv, D, generator=g)
     do = torch.randn(B, S, Hq, D, generator=g)
     q, k, v, do = (t.to(dev, torch.bfloat16).transpose(1, 2) for t in (q, k, v, do))
-    doc = W.doc_ids_from_lengths([[40, 300, 1, 400]], S).to(dev)  # 283 pad tokens
+    doc = W.doc_ids_from_lengths([[40, 300, 1, 400]], S).to(dev)  # then pad tokens
     out, dq, dk, dv = _run(q, k, v, do, doc)
     ref = OA.attention(q, k, v, doc.cpu(), do)
     what = f"{profile} scores, D {D}"

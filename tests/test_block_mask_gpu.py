@@ -166,3 +166,47 @@ def test_plan_rows_match_dense(q_tile, kv_tile, s, kind, dev) -> None:
         for r in range(w.shape[0]):
             row = [(c << 2) | int(k) for c, k in enumerate(w[r]) if k >= 0]
             assert lists[0, r, :int(counts[0, r])].tolist() == row, (by_kv, r)
+
+
+def test_rows_of_more_tiles_than_fit_in_lds(dev) -> None:
+    """Plan rows and block tables of more than 16384 tiles (classes in the workspace first),
+    against the mask itself: tiles of 1024 x 1 tokens both ways, and 1-token blocks."""
+    from packbalance_amd import _native as N
+
+    s, own = 16500, 1024
+    rng = np.random.default_rng(8)
+    d = np.sort(rng.integers(0, s // 90, s)).astype(np.int64)
+    d[-30:] = -1
+    doc = torch.from_numpy(d)[None].to(dev)
+    pos = torch.arange(s, device=dev)
+    n = -(-s // own)
+    for by_kv in (0, 1):
+        # row r: the own tile's tokens against every token of the other axis
+        nq, nk, qt, kt = (s, n, 1, own) if by_kv else (n, s, own, 1)
+        counts = torch.empty((1, n), dtype=torch.int32, device=dev)
+        lists = torch.full((1, n, s), -7, dtype=torch.int32, device=dev)
+        ws = torch.empty(nq * nk, dtype=torch.uint8, device=dev)
+        N.call("pb_attn_plan", doc.data_ptr(), doc.stride(0), 1, s, qt, kt, by_kv,
+               counts.data_ptr(), lists.data_ptr(), ws.data_ptr(), N.stream_ptr(doc))
+        for r in range(n):
+            o = pos[r * own:(r + 1) * own]
+            causal = (o[:, None] <= pos[None]) if by_kv else (o[:, None] >= pos[None])
+            same = doc[0, o][:, None] == doc[0][None]
+            full = (causal & same).all(0) & (len(o) == own)
+            kind = torch.where(full, 1, torch.where((same | ~causal).all(0), 2, 0))
+            cols = torch.nonzero((causal & same).any(0))[:, 0]
+            want = ((cols << 2) | kind[cols]).to(torch.int32)
+            assert int(counts[0, r]) == len(want), (by_kv, r)
+            assert torch.equal(lists[0, r, :len(want)], want), (by_kv, r)
+    s = 16385
+    t = doc_block_tables(doc[:, :s].contiguous(), 1, 1)
+    pos = pos[:s]
+    for q_rows in (False, True):  # (a 1-token tile is full or empty, never partial)
+        a = "q" if q_rows else "kv"
+        assert not t[f"{a}_num_blocks"].any()
+        for r in (0, 1, 4095, 9000, s - 31, s - 2, s - 1):
+            on = (doc[0, :s] == doc[0, r]) & ((pos >= r) if q_rows else (pos <= r))
+            want = torch.cat([pos[on], pos[~on]]).to(torch.int32)
+            assert int(t[f"full_{a}_num_blocks"][0, 0, r]) == int(on.sum()), (a, r)
+            assert torch.equal(t[f"full_{a}_indices"][0, 0, r], want), (a, r)
+            assert torch.equal(t[f"{a}_indices"][0, 0, r], pos.to(torch.int32)), (a, r)

@@ -96,7 +96,6 @@ _CE_CASES = [
     ((3,), 5000, 64, torch.bfloat16, torch.bfloat16, 0.01),  # DMA tiles almost all past N
 ]
 
-# fp32 x and W take the fp32 path, which keeps no kernel logits: recompute only.
 # (n, v, d, vocab rows per chunk): dx products of up to 128 output tiles (this build's split-K
 # GEMM) and of more (the library's); vocabulary chunks that are not whole K slices, split and
 # not, one chunk and several with a last one of other splits.  The same product as
@@ -136,6 +135,7 @@ def test_transposed_copy_is_exact(rows, cols, pad, dev) -> None:
     assert not out[:, rows:].any()
 
 
+# fp32 x and W take the fp32 path, which keeps no kernel logits: recompute only.
 _CE_PARAMS = [pytest.param(*c, stored, id=f"{i}-{'stored' if stored else 'recompute'}")
               for i, c in enumerate(_CE_CASES) for stored in (True, False)
               if not (stored and c[3] == torch.float32 and c[4] == torch.float32)]

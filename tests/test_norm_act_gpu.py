@@ -312,7 +312,7 @@ def test_swiglu_rejects_cpu() -> None:
         (2048, 768, torch.float32, torch.bfloat16, torch.bfloat16, torch.float32),  # cfg2 flow
         (300, 2048, torch.float32, torch.bfloat16, torch.bfloat16, torch.float32),  # 4 vectors/lane
         (64, 512, torch.bfloat16, torch.bfloat16, torch.bfloat16, torch.bfloat16),
-        (40, 4096, torch.float32, torch.float32, torch.bfloat16, torch.float32),  # loop kernel
+        (40, 4096, torch.float32, torch.float32, torch.bfloat16, torch.float32),
         (37, 100, torch.float32, torch.float16, torch.float32, torch.float32),  # n % 8 != 0
         # a workgroup per row: the first and last widths of each shape, rows in a loop
         (5, 2056, torch.float32, torch.bfloat16, torch.bfloat16, torch.float32),
