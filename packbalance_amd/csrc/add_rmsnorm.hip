@@ -26,7 +26,7 @@
 #include <utility>
 
 #include "common.hpp"
-#include "lds_dma.hpp"
+#include "row_sum.hpp"
 
 namespace pb {
 namespace {
@@ -207,18 +207,6 @@ __global__ __launch_bounds__(kThreads) void add_rmsnorm_fwd_reg(AddNormFwd a) {
 // flow (fp32 residual and weight, bf16 the rest) at compile time.
 // At [8192, 4096], fp32 residual, bf16 delta and y: 68 us (5.9 TB/s); with the
 // backward 917 us on the scalar two-pass kernels below, 170 us here.
-template <int THREADS>
-__device__ __forceinline__ float row_sum(float v, float (*red)[THREADS / 64], int slot) {
-  v = wave_sum_full(v);
-  if ((threadIdx.x & 63) == 0) red[slot][threadIdx.x >> 6] = v;
-  __builtin_amdgcn_s_waitcnt(0xC07F);  // the LDS write is done (lgkmcnt(0))
-  block_sync_nofence();
-  float s = red[slot][0];
-#pragma unroll
-  for (int k = 1; k < THREADS / 64; ++k) s += red[slot][k];
-  return s;
-}
-
 template <int NV, int THREADS, bool STD>
 __global__ __launch_bounds__(THREADS) void add_rmsnorm_fwd_wide(AddNormFwd a) {
   __shared__ float red[2][THREADS / 64];

@@ -15,7 +15,7 @@
 #include <mutex>
 
 #include "common.hpp"
-#include "lds_dma.hpp"
+#include "row_sum.hpp"
 
 namespace pb {
 namespace {
@@ -137,19 +137,6 @@ inline unsigned fwd_reg_grid(int64_t rows) {
 // the next row's loads, issued before it, stay in flight across the reduction
 // and the stores.  HBM-bound.  Against the two-pass scalar kernel below
 // ([8192, 8192] bf16): forward 118 -> 46 us (5.9 TB/s).
-template <int THREADS>
-__device__ __forceinline__ float row_sum(float v, float (*red)[THREADS / 64], int slot) {
-  constexpr int W = THREADS / 64;
-  v = wave_sum_full(v);
-  if ((threadIdx.x & 63) == 0) red[slot][threadIdx.x >> 6] = v;
-  __builtin_amdgcn_s_waitcnt(0xC07F);  // the LDS write is done (lgkmcnt(0))
-  block_sync_nofence();
-  float s = red[slot][0];
-#pragma unroll
-  for (int k = 1; k < W; ++k) s += red[slot][k];
-  return s;
-}
-
 template <typename TX, typename TW, int NV, int THREADS>
 __global__ __launch_bounds__(THREADS) void rmsnorm_fwd_wide(
     const TX *__restrict__ x, int64_t xs, const TW *__restrict__ w, TX *__restrict__ y, int64_t ys,

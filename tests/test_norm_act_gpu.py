@@ -305,6 +305,19 @@ def test_swiglu_rejects_cpu() -> None:
         swiglu(torch.randn(4), torch.randn(4))
 
 
+def test_rmsnorm_wide_row_sum_precision(dev) -> None:
+    """fp32 rows held by 16 waves: y has two roundings (x r, then w) of 4e-8 of the 2-norm
+    each, 5.65e-8 together, and 1.2e-8 from the row sum when the waves' sums are added
+    pairwise; one after the other the sum alone gives 3e-8, 6.4e-8 in all."""
+    g = torch.Generator(device=dev).manual_seed(3)
+    x = torch.randn(1000, 12288, device=dev, generator=g)
+    w = torch.randn(12288, device=dev, generator=g)
+    xd = x.double()
+    want = xd * (xd.square().mean(-1, keepdim=True) + 1e-5).rsqrt() * w.double()
+    err = float((rmsnorm(x, w, 1e-5).double() - want).norm() / want.norm())
+    assert err <= 6.1e-8, f"{err:.3e}"
+
+
 # ---------------------------------------------------------------- fused residual add + RMSNorm
 @pytest.mark.parametrize(
     "rows,n,xdt,ddt,ydt,wdt",
