@@ -80,6 +80,18 @@ def test_block_tables_random_layouts(seed, dev) -> None:
     _assert_tables({n: getattr(bm, n) for n in OB.TABLE_NAMES}, want, f"seed{seed}")
 
 
+@pytest.mark.parametrize("kind", ["distinct", "permuted", "short"])
+def test_block_tables_many_documents_a_block(kind, dev) -> None:
+    """Blocks of more documents than are compared one by one."""
+    s = 1300
+    doc = np.arange(s) // (5 if kind == "short" else 1)
+    if kind == "permuted":
+        doc = np.random.default_rng(4).permutation(doc // 3)
+    bm = build_doc_block_mask(torch.from_numpy(doc).to(dev), 2)
+    want = OB.tables_dense(doc, 2, bm.BLOCK_SIZE[0])
+    _assert_tables({n: getattr(bm, n) for n in OB.TABLE_NAMES}, want, kind)
+
+
 def test_build_doc_block_mask_rejects_batch(dev) -> None:
     with pytest.raises(ValueError):
         build_doc_block_mask(torch.zeros(2, 64, dtype=torch.long, device=dev), 2)
@@ -132,10 +144,12 @@ def test_attention_plans_match_oracle(q_tile, kv_tile, by_kv, dev) -> None:
 
 @pytest.mark.parametrize("q_tile,kv_tile", [(32, 32), (128, 64), (64, 128), (1024, 32), (7, 5)])
 @pytest.mark.parametrize("s,kind", [(1, "sorted"), (97, "sorted"), (1025, "sorted"), (700, "mixed"),
-                                    (1999, "padded")])
+                                    (1999, "padded"), (1999, "distinct"), (900, "permuted"),
+                                    (1500, "short"), (1100, "clash")])
 def test_plan_rows_match_dense(q_tile, kv_tile, s, kind, dev) -> None:
     """Both orientations of a plan against the dense mask: ids that recur in any order,
-    one id per token, tiles longer than a wave, and tiles cut by the sequence end."""
+    one id per token (in order and not, and ids that share the hash bits of the sieve over a
+    tile's runs), tiles longer than a wave, and tiles cut by the sequence end."""
     from packbalance_amd import _native as N
 
     rng = np.random.default_rng(s + q_tile)
@@ -144,6 +158,15 @@ def test_plan_rows_match_dense(q_tile, kv_tile, s, kind, dev) -> None:
         d = rng.permutation(d)
     if kind == "padded":
         d[-40:] = -1
+    if kind in ("distinct", "permuted", "clash"):
+        d = np.arange(s, dtype=np.int64)
+    if kind == "permuted":
+        d = rng.permutation(d)
+    if kind == "clash":  # times the inverse of the hash's multiplier: ids whose product is small
+        inv = pow(0x9E3779B97F4A7C15, -1, 1 << 64)
+        d = np.array([(int(x) * inv) % (1 << 64) for x in d], dtype=np.uint64).view(np.int64)
+    if kind == "short":
+        d = np.repeat(np.arange(s // 5 + 1, dtype=np.int64), 5)[:s]
     doc = torch.from_numpy(d)[None].to(dev)
     nq, nk = -(-s // q_tile), -(-s // kv_tile)
     pos = np.arange(s)
