@@ -1005,9 +1005,8 @@ unsigned tiles(int m, int n) { return (unsigned)(((m + BM - 1) / BM) * ((n + BN 
 // MFMA cycle of a SIMD, RowShape 1.4, PairShape 1.1, WideShape 1.0 cycles of
 // the CU's LDS: the larger the wave's block, the fewer.
 // RowShape: 256 x 128 tiles on 8 waves of 64 x 64 (two per SIMD), a three-slice
-// ring of 48 KiB slices.  The dx / dW products, and the lse product while one
-// workgroup per CU covers the grid (n 256, d 768, V 32000: 26.1 us, PairShape
-// 27.6).
+// ring of 48 KiB slices.  The dx / dW products, and the logits products of few
+// tokens (row_lse, row_dlogits).
 using RowShape = DmaShape<4, 2, 2, 2, 3>;
 // WideShape: 256 x 256 tiles on 8 waves of 128 x 64 (half the operand bytes per
 // flop), 32-wide K slices in a four-slice ring of 32 KiB.
@@ -1022,7 +1021,9 @@ template <class SH> unsigned dma_tiles(int m, int n) {
 // A tile's rows lie within the 2 GiB of a DMA's byte offset.
 bool dma_rows(const GemmArgs &g) { return g.lda <= (1 << 22) && g.ldb <= (1 << 22); }
 // The dx / dW products by DMA: whole 16-byte chunks of K (gemm_nt takes the rest; dW of
-// n 3000, d 576, V 49152 408 -> 274 us).
+// n 3000, d 576, V 49152 408 -> 274 us).  Of a few tokens dW stays on gemm_nt where
+// they don't fill the last K slice: the backward by DMA / by gemm_nt, n 200, d 1024,
+// V 50304 280 / 268 us; n 600 397 / 389; n 904 497 / 509.
 bool dma_ok(const GemmArgs &g) { return g.K % 8 == 0 && dma_rows(g); }
 // WideShape for the logits products from K = `least` on, when its tiles give
 // every CU one: below, the epilogue weighs as much as the K loop.  Measured with
@@ -1030,9 +1031,25 @@ bool dma_ok(const GemmArgs &g) { return g.K % 8 == 0 && dma_rows(g); }
 // d 576, V 49152 185 / 191; n 8192, d 768 604 / 658; n 4096, d 2048 723 / 810.
 // dlogits, whose stores add to the epilogue: n 8192, d 768 1006 / 948 us; n 4096,
 // d 1024 512 / 534; d 2048 839 / 940.
+// Not for so few tokens that the empty half of a last 256-column tile costs more
+// than the shape gains (lse, d 4096, V 128256, WideShape / RowShape: n 128 298 / 276 us,
+// n 300 456 / 412, n 512 530 / 550, n 600 683 / 661, n 900 911 / 1019).
 constexpr int kWideLse = 512, kWideDlogits = 1024;
 bool wide_ok(const GemmArgs &g, int least) {
+  if (g.N <= 768 && (g.N + RowShape::BNT - 1) / RowShape::BNT % 2 != 0) return false;
   return g.K >= least && dma_tiles<WideShape>(g.M, g.N) > 256;
+}
+// RowShape for the logits products of few tokens, whose reduction fills whole K
+// slices.  RowShape / PairShape, lse: n 256, d 768, V 32000 23.5 / 27.0 us (one
+// workgroup per CU covers the grid); n 300, d 1024, V 50304 57.3 / 54.2; n 600,
+// d 2048 131 / 142.  The whole backward: n 200, d 576, V 49152 205.9 / 210.9; n 600
+// 294.7 / 286.2; n 512, d 2048, V 50304 570.9 / 586.0 and with d 4096, V 128256
+// 2422 / 2476 (WideShape 2488); n 1024 3792 / 3918 (3725).
+bool row_lse(const GemmArgs &g) {
+  return g.K % 64 == 0 && (g.K >= 2048 || dma_tiles<RowShape>(g.M, g.N) <= 256);
+}
+bool row_dlogits(const GemmArgs &g) {
+  return g.K % 64 == 0 && g.N <= (g.K >= 2048 ? 768 : 256);
 }
 template <int MODE, class SH> void launch_dma(const GemmArgs &g, hipStream_t st) {
   dim3 grid(dma_tiles<SH>(g.M, g.N)), block(SH::NT);
@@ -1148,7 +1165,7 @@ int lmhead_fwd(const void *x, int64_t ldx, const void *w, int64_t ldw, int64_t n
     hipLaunchKernelGGL(gemm_nt<kLse>, dim3(tiles(g.M, g.N)), dim3(256), 0, st, g);
   else if (wide_ok(g, kWideLse))
     launch_dma<kLse, WideShape>(g, st);
-  else if (g.K % 64 == 0 && dma_tiles<RowShape>(g.M, g.N) <= 256)
+  else if (row_lse(g))
     launch_dma<kLse, RowShape>(g, st);
   else
     launch_dma<kLse, PairShape>(g, st);
@@ -1293,6 +1310,8 @@ int dlogits_chunk(const void *x, int64_t ldx, const void *w, int64_t ldw, int64_
   g.round_bf16 = round_bf16;
   if (!dma_rows(g))
     hipLaunchKernelGGL(gemm_nt<kDlogits>, dim3(tiles(g.M, g.N)), dim3(256), 0, st, g);
+  else if (row_dlogits(g))
+    launch_dma<kDlogits, RowShape>(g, st);
   else if (wide_ok(g, kWideDlogits))
     launch_dma<kDlogits, WideShape>(g, st);
   else
@@ -1315,7 +1334,7 @@ void launch_dx(const pb::ce::GemmArgs &g, hipStream_t st) {
 
 void launch_dw(const pb::ce::GemmArgs &g, hipStream_t st) {
   using namespace pb::ce;
-  if (dma_ok(g))
+  if (dma_ok(g) && (g.K % 64 == 0 || g.K > 640))
     launch_dma<kStore, RowShape>(g, st);
   else
     hipLaunchKernelGGL(gemm_nt<kStore>, dim3(tiles(g.M, g.N)), dim3(256), 0, st, g);

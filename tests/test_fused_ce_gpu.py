@@ -125,6 +125,26 @@ def test_accumulate_products_k_tail(dev) -> None:
     assert _rel_fro(xr.grad, dx_ref) < 1e-2 and _rel_fro(acc, dw_ref) < 1e-2
 
 
+# Few tokens: the logits products' 256 x 128 tiles on 8 waves (d of 2048 on, or up to 256
+# tokens), 256 x 256 tiles only where the last one's second half holds tokens, and dW off the
+# DMA up to 640 tokens that don't fill a K slice.  Loss and products as above.
+@pytest.mark.parametrize("n,v,d", [
+    (200, 1032, 2048), (296, 1032, 2048), (768, 1032, 2048), (776, 1032, 2048), (600, 1032, 64),
+    (640, 1032, 72), (648, 1032, 64), (120, 66056, 512), (136, 66056, 512)])
+def test_few_tokens_tile_shapes(n, v, d, dev) -> None:
+    x, w, t = _case((n,), v, d, torch.bfloat16, torch.bfloat16, dev, seed=n + d, ignore_every=9,
+                    wstd=0.05 if d >= 256 else 1.0)
+    t[1], t[-1] = 0, v - 1
+    wb, wt = FC.lmhead_weight_bf16(w)
+    xr = x.detach().requires_grad_(True)
+    acc = torch.zeros(v, d, device=dev)
+    loss = FC.linear_cross_entropy_accumulate(xr, wb, wt, acc, t)
+    loss.backward()
+    l_ref, dx_ref, dw_ref = OK.linear_ce(x, w, t, logits_dtype=torch.bfloat16)
+    torch.testing.assert_close(loss.double().cpu(), l_ref, rtol=1e-4, atol=1e-4)
+    assert _rel_fro(xr.grad, dx_ref) < 1e-2 and _rel_fro(acc, dw_ref) < 1e-2
+
+
 @pytest.mark.parametrize("rows,cols,pad", [(1, 8, 0), (63, 72, 8), (64, 64, 0), (129, 200, 16),
                                            (1000, 136, 0)])
 def test_transposed_copy_is_exact(rows, cols, pad, dev) -> None:
