@@ -21,11 +21,10 @@
 // from L2 instead of once per workgroup, which is why larger grids and longer
 // sequences keep the workgroup kernels (wave_tiles).
 //
-// Measured, workgroup -> wave kernels with their merges: [4, 2048], 12 / 4
-// heads, D 64: forward 42 -> 27 us, backward 112 -> 66 us; [2, 2048]: 24 -> 19
-// and 61 -> 46 us.  What is left is latency: at [16, 2048] the VALU is busy 38%
-// and the matrix cores 14% of the forward's time, 1.7 waves per SIMD resident
-// on average (short lists end before the next workgroups have started).
+// Measured in captured launches, workgroup -> wave kernels with their merges, 12 / 4
+// heads, D 64: [4, 2048] forward 41 -> 27 us, backward 135 -> 71 us; [2, 2048] 25 ->
+// 16 and 59 -> 43 us.  What is left is latency: there the VALU is active 19 to 23%
+// of the waves' time and the matrix cores 8 to 9% of the kernels'.
 //
 // MFMA layouts, masks and log2-domain lse as in attn_fwd.hip / attn_bwd.hip.
 #include "attn_args.hpp"
@@ -44,7 +43,7 @@ namespace {
 // 12 heads 22.5 -> 17.1 (30.3); at 1152 tiles ([1, 3072], 12 heads, documents of
 // about 100) 14.1 -> 15.3.
 constexpr int kFewQ = 768;
-constexpr int kWaveLeast = 6;  // (four waves of the forward and dQ: 4)
+constexpr int kWaveLeast = 6, kFewLeast = 4;  // kFewLeast: four waves of the forward and dQ
 constexpr int kTB = 32 * 64 * 2;   // bytes of one 32 x 64 bf16 tile
 constexpr int NDK = 4, NDB = 2;    // 16-wide k steps and 32-wide blocks of the head dim
 using Dma = TileDma<64, 32, 64>;   // one wave copies a tile: four 1 KiB instructions
@@ -638,11 +637,17 @@ int launch_row_copies(const RowCopies &c, bool to_dense, hipStream_t st) {
   return launch_status("pb_attn(row copies)");
 }
 
+// Rows too short for a second wave's part have one wave a query tile (forward of
+// one document, 16 / 2 heads: [32, 128] 13.7 -> 10.7 us, [16, 200] 13.6 -> 10.6).
 int launch_fwd_wave(const FwdArgs &a, hipStream_t st) {
   const int tiles = a.nqt * a.B * a.Hq;
   const dim3 g((unsigned)tiles);
-  if (tiles <= kFewQ) hipLaunchKernelGGL((attn_fwd_wave<4, 4>), g, dim3(256), 0, st, a);
-  else hipLaunchKernelGGL((attn_fwd_wave<2, kWaveLeast>), g, dim3(128), 0, st, a);
+  if (tiles <= kFewQ && a.nkt >= 2 * kFewLeast)
+    hipLaunchKernelGGL((attn_fwd_wave<4, kFewLeast>), g, dim3(256), 0, st, a);
+  else if (a.nkt >= 2 * kWaveLeast)
+    hipLaunchKernelGGL((attn_fwd_wave<2, kWaveLeast>), g, dim3(128), 0, st, a);
+  else
+    hipLaunchKernelGGL((attn_fwd_wave<1, kWaveLeast>), g, dim3(64), 0, st, a);
   return launch_status("pb_attn_fwd");
 }
 
@@ -650,8 +655,12 @@ int launch_bwd_wave(const BwdArgs &a, hipStream_t st) {
   // dQ first: it also writes delta = rowsum(dO * O), which dK/dV reads.
   const int qtiles = a.nqt_dq * a.B * a.Hq;
   const dim3 gq((unsigned)qtiles);
-  if (qtiles <= kFewQ) hipLaunchKernelGGL((attn_bwd_dq_wave<4, 4>), gq, dim3(256), 0, st, a);
-  else hipLaunchKernelGGL((attn_bwd_dq_wave<2, kWaveLeast>), gq, dim3(128), 0, st, a);
+  if (qtiles <= kFewQ && a.nkt_dq >= 2 * kFewLeast)
+    hipLaunchKernelGGL((attn_bwd_dq_wave<4, kFewLeast>), gq, dim3(256), 0, st, a);
+  else if (a.nkt_dq >= 2 * kWaveLeast)
+    hipLaunchKernelGGL((attn_bwd_dq_wave<2, kWaveLeast>), gq, dim3(128), 0, st, a);
+  else
+    hipLaunchKernelGGL((attn_bwd_dq_wave<1, kWaveLeast>), gq, dim3(64), 0, st, a);
   const int rc = launch_status("pb_attn_bwd(dq)");
   if (rc) return rc;
   // Waves per workgroup by the number of KV tiles: at 1024 tiles (2048 waves
@@ -662,13 +671,23 @@ int launch_bwd_wave(const BwdArgs &a, hipStream_t st) {
   // workgroup per CU eight, and to 384 tiles with long lists: one document, dQ and
   // dK/dV with 4 / 8: [1, 2048], 9 / 3 heads 65 / 53 us (workgroup kernels 67);
   // 384 tiles: [1, 3072], 16 / 4 132 / 109 (125), but [1, 2048], 6 / 6 38 / 45.
+  // No more waves than the longest list has parts of kWaveLeast steps (up to one
+  // workgroup per CU, where idle waves cost less, no twice as many).  Backward of
+  // one document, 12 / 4 heads, with these counts in dQ and dK/dV, before / after:
+  // [64, 128] (KV tiles of up to 12 steps) 43.8 / 35.5 us, [32, 200] 45.2 / 35.1,
+  // [1, 64] 15.5 / 14.5; [16, 384], 4 / 4 heads 28.9 / 26.1.
   const int64_t tiles = (int64_t)a.nkt_kv * a.B * a.Hkv;
   const dim3 gk((unsigned)tiles);
   const int longest = a.nqt_kv * (a.Hq / a.Hkv);  // steps
-  if (tiles <= 256 || (tiles <= 384 && longest >= 288))
-    hipLaunchKernelGGL(attn_bwd_dkdv_wave<8>, gk, dim3(512), 0, st, a);
-  else if (tiles <= 1024) hipLaunchKernelGGL(attn_bwd_dkdv_wave<4>, gk, dim3(256), 0, st, a);
-  else if (tiles <= 4096) hipLaunchKernelGGL(attn_bwd_dkdv_wave<2>, gk, dim3(128), 0, st, a);
+  int nw = tiles <= 256 || (tiles <= 384 && longest >= 288) ? 8
+           : tiles <= 1024                                  ? 4
+           : tiles <= 4096                                  ? 2
+                                                            : 1;
+  const int parts = longest / kWaveLeast;
+  while (nw > 1 && (tiles <= 256 ? nw / 2 >= parts : nw > parts)) nw /= 2;
+  if (nw == 8) hipLaunchKernelGGL(attn_bwd_dkdv_wave<8>, gk, dim3(512), 0, st, a);
+  else if (nw == 4) hipLaunchKernelGGL(attn_bwd_dkdv_wave<4>, gk, dim3(256), 0, st, a);
+  else if (nw == 2) hipLaunchKernelGGL(attn_bwd_dkdv_wave<2>, gk, dim3(128), 0, st, a);
   else hipLaunchKernelGGL(attn_bwd_dkdv_wave<1>, gk, dim3(64), 0, st, a);
   return launch_status("pb_attn_bwd(dkdv)");
 }

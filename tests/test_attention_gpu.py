@@ -403,6 +403,18 @@ def test_small_grid_matches_padded_head_dim(B, Hq, Hkv, S, D, mu, misaligned, de
         assert err <= 2 ** -8, f"{name}: {err:.2e}"
 
 
+# Rows so short that no list has a part for a second (fourth, eighth) wave: fewer waves a
+# workgroup.  Query tiles of 1, 7, 8, 11 and 12 list entries on small and large grids, KV
+# tiles of 1 to 24 steps.
+@pytest.mark.parametrize("B,Hq,Hkv,S,D", [
+    (1, 4, 4, 20, 64), (2, 4, 2, 224, 64), (2, 4, 2, 225, 40), (64, 4, 4, 352, 40),
+    (64, 4, 4, 353, 64), (64, 12, 4, 128, 64), (32, 12, 4, 200, 64), (1, 12, 4, 200, 64),
+    (32, 4, 4, 200, 48), (33, 16, 2, 65, 64)])
+def test_short_rows_match_padded_head_dim(B, Hq, Hkv, S, D, dev) -> None:
+    for mu in (1e9, 40):
+        test_small_grid_matches_padded_head_dim(B, Hq, Hkv, S, D, mu, False, dev)
+
+
 @pytest.mark.parametrize("pack", [1, 0])
 def test_attention_cfg3_pack(pack, dev) -> None:
     """cfg3 shape (S=8192, Hq=32, Hkv=8, D=128): all 8 packs run, one pack x one
