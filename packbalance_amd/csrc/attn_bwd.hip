@@ -249,8 +249,9 @@ constexpr int kAheadDkdv = DP == 64 ? 2 : DP / 16;
 // GEN: any sequence length and any head dim that is a multiple of 8 (see
 // attn_fwd_pipe).  Query rows past the end arrive as zero Q, dO, lse and delta,
 // so their P is at most 1, their dS 0, and both products add nothing.  Against
-// the register-staged kernels ([4, 1999], 12 / 4 heads, D 64): dK/dV 390 ->
-// 153 us, dQ 130 -> 47 us and a 7 us sum.
+// the register-staged kernels, dQ and dK/dV with their sums: [1, 6001], 12 / 4
+// heads, D 64, one document 870 -> 324 us, documents of about 200 178 -> 88 us;
+// [8, 8191], 32 / 8 heads, D 128 11.3 -> 4.0 ms (four waves, 128 KV rows).
 template <int DP, int WAVES, bool SPLIT, bool GEN>
 __global__ __launch_bounds__(64 * WAVES) __attribute__((amdgpu_waves_per_eu(DP == 64 ? 2 : 1, DP == 64 ? 2 : 1)))
 void attn_bwd_dkdv_pipe(BwdArgs a) {

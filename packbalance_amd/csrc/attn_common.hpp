@@ -336,10 +336,10 @@ struct AttnConfig {
 // for short documents and lose at most 3%, at [1, 4096] up to 8%, with one
 // document of the whole sequence (in brackets).  [B, S], 12 / 4 heads, D 64 in
 // us, workgroup -> wave kernels:
-//   forward   [4, 2048] 42 -> 27 (one document: 68 -> 60), [8, 2048] 72 -> 52,
-//             but [16, 2048] 107 -> 94 (one document: 179 -> 204)
-//   backward  [4, 2048] 112 -> 66 (249 -> 149), [16, 2048] 299 -> 241 (535 ->
-//             491), but [16, 4096] 752 -> 765 (1648 -> 1804); dQ + dK/dV
+//   forward   [4, 2048] 41 -> 27 (68 -> 54), [8, 2048] 72 -> 52, but [16, 2048]
+//             107 -> 94 (179 -> 204)
+//   backward  [4, 2048] 135 -> 71 (249 -> 142), [16, 2048] 279 -> 262 (534 ->
+//             488), but [16, 4096] 752 -> 765 (1648 -> 1804); dQ + dK/dV
 // The backward's dK/dV kernel has a workgroup per KV tile and KV head, which
 // walks the query heads of the group one after the other, where the workgroup
 // kernels split them.  So it wins with enough (pack, KV head) pairs for the

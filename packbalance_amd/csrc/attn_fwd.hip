@@ -237,9 +237,10 @@ __global__ __launch_bounds__(64 * WAVES) __attribute__((amdgpu_waves_per_eu(2, 2
 // past the sequence or the head dim (TileDma::copy_gen), documents move 4
 // bytes per lane, and the causal test masks the zero rows (a tile that reaches
 // past the end is always a diagonal one).  It costs a compare and a select per
-// DMA instruction, 169 -> 172 registers at D 64.  Against the register-staged
-// kernel above: [4, 1999], 12 / 4 heads, D 64: 84 -> 40 us and an 8 us merge;
-// [1, 6001], 32 / 8 heads, D 128: 404 -> 324 us with the merge.
+// DMA instruction, and the max of each sub-tile (take_max).  Against the
+// register-staged kernel above, with the merge, one document / documents of
+// about 200 (D 128: 512): [1, 6001], 12 / 4 heads, D 64 268 -> 110 / 45 -> 34 us,
+// 32 / 8 heads, D 128 449 -> 369 / 108 -> 95 us.
 template <int DP, int MQ, int WAVES, bool GEN>
 __global__ __launch_bounds__(64 * WAVES)
 __attribute__((amdgpu_waves_per_eu(MQ == 64 ? 1 : 2, MQ == 64 ? 1 : 2)))

@@ -5,7 +5,7 @@ Drop-in for the reference ``packbalance/model/attention.py``:
 * ``build_doc_block_mask(doc_ids, n_heads, block_size=128)`` (attention.py:25-54)
   returns a ``torch.nn.attention.flex_attention.BlockMask`` whose eight tables
   are bit-identical to ``create_block_mask``'s for the mask
-  ``doc[q] == doc[kv] and q >= kv``, but are built by two small HIP kernels
+  ``doc[q] == doc[kv] and q >= kv``, but are built by one small HIP kernel
   straight from ``doc_ids`` -- the dense [H, S, S] mask the reference
   materialises is never formed.  The returned object also carries ``doc_ids``
   and the attention kernel's own tile plan.
