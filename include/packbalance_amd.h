@@ -200,8 +200,8 @@ int pb_attn_plan(const int64_t *doc_ids, int64_t doc_stride, int64_t b, int64_t 
  * lse (fp32 [b, hq, s]) receives log2(sum_j exp2(scale*log2(e)*q.k)) for the
  * backward.  plan = pb_attn_plan(by_kv = 0) with the forward tiles of
  * pb_attn_config; workspace: out[8] bytes of pb_attn_config (may be NULL when
- * that is 0, and on 32 x 32 tiles when every row of q, k, v and out is 16-byte
- * aligned: there it holds copies of views that are not).                     */
+ * that is 0, and on 32 x 32 tiles: there it holds copies of views without
+ * 16-byte aligned rows, which run several times slower without it).          */
 int pb_attn_fwd(const pb_bhsd *q, const pb_bhsd *k, const pb_bhsd *v, const pb_bhsd *out,
                 float *lse, void *workspace, const int64_t *doc_ids, int64_t doc_stride,
                 const int32_t *plan_counts, const int32_t *plan_lists, int64_t b,

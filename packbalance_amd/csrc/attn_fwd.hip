@@ -41,7 +41,8 @@ namespace attn {
 template <int DP, int WAVES>
 __global__ __launch_bounds__(64 * WAVES) __attribute__((amdgpu_waves_per_eu(2, 2))) void attn_fwd_generic(FwdArgs a) {
   constexpr int NT = 64 * WAVES;
-  constexpr int BM = 32 * WAVES, BN = kKvStep;
+  constexpr int BM = 32 * WAVES, BN = WAVES == 1 ? 32 : kKvStep;  // (one wave: 32 x 32 plans)
+  constexpr int NBLK = BN / 32;
   constexpr int KP = DP + 8;  // K / V row pitch in LDS (elements)
   constexpr int NDK = DP / 16;
   constexpr int NDB = DP / 32;
@@ -116,10 +117,10 @@ __global__ __launch_bounds__(64 * WAVES) __attribute__((amdgpu_waves_per_eu(2, 2
     __syncthreads();
     if (it + 1 < cnt) fetch(lst[it + 1]);
 
-    // S^T = K Q^T for the two 32-row halves of the tile.
-    f32x16_t sacc[2];
+    // S^T = K Q^T for the 32-row blocks of the tile.
+    f32x16_t sacc[NBLK];
 #pragma unroll
-    for (int blk = 0; blk < 2; ++blk) {
+    for (int blk = 0; blk < NBLK; ++blk) {
       sacc[blk] = zero16();
 #pragma unroll
       for (int dk = 0; dk < NDK; ++dk) {
@@ -135,7 +136,7 @@ __global__ __launch_bounds__(64 * WAVES) __attribute__((amdgpu_waves_per_eu(2, 2
     float mloc = -INFINITY;
     if (!full) {
 #pragma unroll
-      for (int blk = 0; blk < 2; ++blk)
+      for (int blk = 0; blk < NBLK; ++blk)
 #pragma unroll
         for (int j = 0; j < 16; ++j) {
           const int kr_ = 32 * blk + 8 * (j >> 2) + 4 * hh + (j & 3);
@@ -145,7 +146,7 @@ __global__ __launch_bounds__(64 * WAVES) __attribute__((amdgpu_waves_per_eu(2, 2
         }
     }
 #pragma unroll
-    for (int blk = 0; blk < 2; ++blk)
+    for (int blk = 0; blk < NBLK; ++blk)
 #pragma unroll
       for (int j = 0; j < 16; ++j) mloc = fmaxf(mloc, sacc[blk][j]);
     mloc = fmaxf(mloc, __shfl_xor(mloc, 32)) * a.sl2;
@@ -159,9 +160,9 @@ __global__ __launch_bounds__(64 * WAVES) __attribute__((amdgpu_waves_per_eu(2, 2
 #pragma unroll
       for (int j = 0; j < 16; ++j) oacc[db][j] *= alpha;
 
-    bf16x8_t pf[4];
+    bf16x8_t pf[2 * NBLK];
 #pragma unroll
-    for (int blk = 0; blk < 2; ++blk)
+    for (int blk = 0; blk < NBLK; ++blk)
 #pragma unroll
       for (int j = 0; j < 16; ++j) {
         const float p = fast_exp2(fmaf(sacc[blk][j], a.sl2, -m_use));
@@ -174,7 +175,7 @@ __global__ __launch_bounds__(64 * WAVES) __attribute__((amdgpu_waves_per_eu(2, 2
 #pragma unroll
     for (int db = 0; db < NDB; ++db)
 #pragma unroll
-      for (int kk = 0; kk < 4; ++kk)
+      for (int kk = 0; kk < 2 * NBLK; ++kk)
         oacc[db] = mfma32(lds_col_frag(Vs, KP, 16 * kk, 32 * db, lane), pf[kk], oacc[db]);
   }
 
@@ -896,8 +897,11 @@ extern "C" int pb_attn_fwd(const pb_bhsd *q, const pb_bhsd *k, const pb_bhsd *v,
   a.tau = gen ? 0.f : 8.f;  // (as attn_fwd_pipe: GEN exact, else kTau)
   if (cfg.wave_fwd) {
     if (dma) return launch_fwd_wave(a, st);
-    PB_CHECK_ARG(workspace != nullptr,
-                 "pb_attn_fwd: workspace is required for views without 16-byte aligned rows");
+    if (!workspace) {  // the register-staged kernel reads any view
+      if (d <= 32) hipLaunchKernelGGL((attn_fwd_generic<32, 1>), grid, dim3(64), 0, st, a);
+      else hipLaunchKernelGGL((attn_fwd_generic<64, 1>), grid, dim3(64), 0, st, a);
+      return launch_status("pb_attn_fwd");
+    }
     RowCopies in(a.B, a.S, a.D, workspace), back(a.B, a.S, a.D, nullptr);
     a.q = in.add(*q, a.Hq, a.q_sb, a.q_sh, a.q_ss);
     a.k = in.add(*k, a.Hkv, a.k_sb, a.k_sh, a.k_ss);

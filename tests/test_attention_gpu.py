@@ -688,3 +688,35 @@ def test_forward_without_workspace(S, D, dev) -> None:
            p.lists.data_ptr(), B, Hq, Hkv, S, D, 1.0 / math.sqrt(D), N.PB_BF16, N.stream_ptr(q))
     assert (out.double() - want.double()).norm() <= 2 ** -8 * want.double().norm()
     torch.testing.assert_close(lse, want_lse, atol=1e-4, rtol=0)
+
+
+@pytest.mark.parametrize("B,S,D", [(1, 33, 32), (2, 700, 64), (3, 257, 40)])
+def test_misaligned_forward_without_workspace(B, S, D, dev) -> None:
+    """32 x 32 tiles, rows without 16-byte alignment and no workspace to copy them to: the
+    register-staged kernel reads them in place.  P and the output are rounded to bf16 once on
+    either side (2 x 2^-9 in the 2-norm)."""
+    from packbalance_amd import _native as N
+    from packbalance_amd.model import attention as A
+
+    Hq, Hkv = 4, 2
+    doc = W.doc_ids_from_lengths([[S - 30, 30]] * B, S).to(dev)
+
+    def odd(t):  # the same values one element past a 16-byte boundary
+        b, h, s, d = t.shape
+        buf = torch.empty(b * s * h * d + 8, dtype=t.dtype, device=dev)
+        v = buf[1:1 + b * s * h * d].view(b, s, h, d).transpose(1, 2)
+        return v.copy_(t)
+
+    q, k, v, _ = _inputs(B, Hq, Hkv, S, D, dev, seed=8)
+    want, want_lse = _fwd_abi(q, k, v, doc)
+    cfg = A.attn_config(B, Hq, Hkv, S, D)
+    assert cfg["fwd_workspace"] > 0 and cfg["tiles"][A.FWD] == (32, 32)
+    q, k, v, out = odd(q), odd(k), odd(v), odd(torch.full_like(want, float("nan")))
+    assert q.data_ptr() % 16 == 2
+    lse = torch.empty_like(want_lse)
+    p = A._plans(doc, Hq, Hkv, D, None)[A.FWD]
+    N.call("pb_attn_fwd", N.BHSD.of(q), N.BHSD.of(k), N.BHSD.of(v), N.BHSD.of(out),
+           lse.data_ptr(), None, doc.data_ptr(), doc.stride(0), p.counts.data_ptr(),
+           p.lists.data_ptr(), B, Hq, Hkv, S, D, 1.0 / math.sqrt(D), N.PB_BF16, N.stream_ptr(q))
+    assert (out.double() - want.double()).norm() <= 2 ** -8 * want.double().norm()
+    torch.testing.assert_close(lse, want_lse, atol=1e-4, rtol=0)
