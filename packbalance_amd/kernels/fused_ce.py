@@ -235,12 +235,13 @@ def _ce_backward(xb, wb, t, lse, go, lg, lg_dtype, n, v, d8, ignore_index, z, vc
 def own_dx(n: int, d8: int) -> bool:
     """True when ``dx = dL W`` of a chunk runs on this build's split-K GEMM: up to 128 of its
     256 x 128 output tiles (the vocabulary is split to fill the CUs) and at most 8 of them
-    side by side, which share one XCD's reads of dL.  Library product against split-K GEMM
-    and transposed copy of W, in us: d 576, V 49152: n 520 193 / 74, n 2999 370 / 214, n 6001
-    465 / 396; d 768, V 50257: n 2999 443 / 391, n 4096 518 / 487, but n 6001 649 / 685;
-    d 1000, V 32000: n 4096 377 / 283, n 6001 376 / 444.  Wider rows make the copy the larger
-    part: d 2048, V 128256: n 1999 1556 / 1226, n 2999 1324 / 1755; d 4096, V 32000: n 520
-    269 / 320, n 2999 643 / 864."""
+    side by side, which share one XCD's reads of dL.  Library product / split-K GEMM, copy of
+    W and reduction, in us, repeated calls: d 576, V 49152: n 520 187 / 76, n 2999 362 / 226,
+    n 6001 464 / 395; d 768, V 50257: n 2999 444 / 402, n 4096 520 / 491, but n 6001 653 /
+    692; d 1000, V 32000: n 4096 371 / 290, n 6001 388 / 436.  With the operands out of the
+    caches: 379 / 257, 462 / 421, 488 / 442, 553 / 526 (n 2999, 6001, 2999, 4096 above).
+    Wider rows make the copy the larger part: d 2048, V 128256: n 1999 1570 / 1217, but n 2999
+    1317 / 1752; d 4096, V 32000: n 520 271 / 324, n 2999 645 / 862."""
     return d8 <= 1024 and -(-n // 256) * -(-d8 // 128) <= 128
 
 
